@@ -149,6 +149,7 @@ static void free_fields(bfvm_ctx* ctx)
 		dfree(t.coef);
 		dfree(t.red);
 		dfree(t.A);
+		dfree(t.filter_tab);
 		t = axis_tables {};
 	}
 	ctx->n_interior = 0;

@@ -324,11 +324,27 @@ struct partition
 	int vec = 1; // substrates per thread (1 or 4)
 };
 
+// Launch shape of the recursive-filter sweep along one axis (filter_sweep.hip); blocks == 0: not used.
+struct filter_plan
+{
+	int m = 0, blocks = 0, kw = 0; // elements per block (one lane), blocks of a line, blocks per wave
+	bool staged = false;		   // x rows staged through LDS
+	bool streamed = false;		   // loads and stores past the caches
+	int waves = 1;				   // waves of a line group (one workgroup)
+	int64_t tasks = 0;			   // line groups
+	int lines_group = 0;		   // lines of a line group (S a multiple of 4: of 4 substrates)
+	int lds = 0, exchange_at = 0;  // LDS bytes of a workgroup, offset of its exchange area
+	int clog = 0;				   // log2 of the columns of a line group
+	int rows = 0, lines_pass = 0, passes = 0, rows_at = 0; // staged: rows, lines side by side, LDS offset
+};
+
 // Device-side tables of one axis.
 struct axis_tables
 {
 	int n = 0;
 	partition part;
+	filter_plan filter;
+	float* filter_tab = nullptr;
 	// exact (reference-order FP32) Thomas coefficients: b' [n][S], c [S], e [n-1][S]
 	float* exact_b = nullptr;
 	float* exact_c = nullptr;
@@ -574,6 +590,13 @@ void launch_cell_sort(bfvm_ctx* ctx); // sorted reduction: order the agents by v
 void launch_cell_release(bfvm_ctx* ctx, int index);
 void launch_voxel_positions(bfvm_ctx* ctx, int count, const float* d_pos, int* d_out);
 
+filter_plan choose_filter(const bfvm_ctx* ctx, int axis);
+size_t filter_table_floats(const filter_plan& p, int S);
+void launch_filter_coefficients(const bfvm_ctx* ctx, int axis, const filter_plan& p, float* tab, hipStream_t stream);
+void launch_filter_sweep(bfvm_ctx* ctx, int axis);
+
+// (mul, shift) for n / d = (n * mul) >> shift, n < 2^31 (1 <= d < 2^31)
+void fast_divisor(uint32_t d, uint32_t& mul, int& shift);
 int supported_chunk(int request);
 partition choose_partition(const bfvm_ctx* ctx, int axis, int chunk, int lines_request, int max_vec);
 

@@ -1603,7 +1603,10 @@ static void free_partition_tables(axis_tables& t)
 		BFVM_HIP(hipFree(t.red));
 	if (t.A)
 		BFVM_HIP(hipFree(t.A));
-	t.coef = t.red = t.A = nullptr;
+	if (t.filter_tab)
+		BFVM_HIP(hipFree(t.filter_tab));
+	t.coef = t.red = t.A = t.filter_tab = nullptr;
+	t.filter = filter_plan {};
 }
 
 // Most threads of a register-sweep workgroup: 4-substrate sweeps without the 16-bit prefetch fit 1024 threads
@@ -1708,10 +1711,25 @@ void build_partition(bfvm_ctx* ctx, int axis, int chunk, int lines_request)
 	free_partition_tables(t);
 	// the staged sweep runs one line per thread on 16-element blocks
 	const bool staged = ctx->algorithm == BFVM_SWEEP_STAGED;
+	const bool automatic = ctx->algorithm == BFVM_SWEEP_PARTITIONED && chunk == 0 && lines_request == 0;
 	// 16-bit forms take z lines in groups of 8, not 16 (measured on 400^3 x 8 BF16: 1.38 -> 1.11 ms)
 	if (lines_request == 0 && axis == 2 && ctx->storage != BFVM_STORAGE_F32 && !staged)
 		lines_request = 8;
 	t.part = choose_partition(ctx, axis, staged ? batch_chunk : chunk, lines_request, staged ? 1 : 4);
+	if (automatic && t.part.P > 0)
+	{
+		const filter_plan p = choose_filter(ctx, axis);
+		if (p.blocks > 0)
+		{
+			t.filter = p;
+			t.part.P = p.blocks;
+			t.part.base = t.part.n / p.blocks;
+			t.part.rem = p.m > t.part.base ? 1 : 0;
+			t.part.lpg = p.lines_group;
+			BFVM_HIP(hipMalloc(&t.filter_tab, sizeof(float) * filter_table_floats(p, ctx->mesh.S)));
+			return;
+		}
+	}
 	if (t.part.P > 0)
 		alloc_partition_tables(t.part, ctx->mesh.S, t.coef, t.red, t.A);
 }
@@ -1731,6 +1749,11 @@ void launch_partition_tables(const bfvm_ctx* ctx, int axis, const partition& p, 
 void launch_partition_coefficients(bfvm_ctx* ctx, int axis)
 {
 	auto& t = ctx->axes[axis];
+	if (t.filter.blocks > 0)
+	{
+		launch_filter_coefficients(ctx, axis, t.filter, t.filter_tab, ctx->stream);
+		return;
+	}
 	launch_partition_tables(ctx, axis, t.part, t.coef, t.red, t.A, ctx->stream);
 }
 
@@ -1741,7 +1764,7 @@ void launch_partition_coefficients(bfvm_ctx* ctx, int axis)
 static constexpr int64_t sweep_max_blocks = BFVM_SWEEP_MAX_BLOCKS;
 
 // (mul, shift) of fdiv for divisor d (1 <= d < 2^31)
-static void fast_divisor(uint32_t d, uint32_t& mul, int& shift)
+void fast_divisor(uint32_t d, uint32_t& mul, int& shift)
 {
 	int l = 0;
 	while ((1ull << l) < d)
@@ -1963,6 +1986,11 @@ static void launch_sweep_storage(bfvm_ctx* ctx, int axis)
 			launch_staged_axis<1, K>(ctx, g, t);
 		else
 			launch_staged_axis<2, K>(ctx, g, t);
+		return;
+	}
+	if (t.filter.blocks > 0)
+	{
+		launch_filter_sweep(ctx, axis);
 		return;
 	}
 	if (axis == 0)

@@ -1,0 +1,968 @@
+// The x/y/z sweeps as two-sided recursive filters on gfx950.
+//
+// The system of a line (diffusion.hip) is Toeplitz up to its end rows: with a = dt*D/dx^2 and B = 1 +
+// decay*dt/dims + 2a, the interior rows are -a x_{i-1} + B x_i - a x_{i+1} = d_i, and the end rows, whose diagonal
+// is B - a, are the interior row with a ghost x_{-1} = x_0 (x_n = x_{n-1}): zero flux, i.e. the line mirrored about
+// its ends.  On the mirrored infinite line the matrix factors exactly into two first-order recursions with one
+// constant, mu = 2a / (B + sqrt(B^2 - 4a^2)) (the smaller root of a mu^2 - B mu + a = 0, 0 <= mu < 1):
+//   u_j = d_j + mu u_{j-1},   x_j = s (u_j + mu x'_{j+1}),   s = (1 - mu)^2 / (1 + decay*dt/dims)
+// (x' without the factor s).  The same solution as the Thomas algorithm's (host/diffusion_solver.cpp:72-142,
+// 297-480), with constants instead of a table entry per element: 5 operations per element and no table reads.
+// Every term is positive for positive densities, so rounding errors do not amplify: against an FP64 solve of
+// uniform densities, n = 400, the FP32 relative L2 error is 0.4-1.3e-7 for a = 0.025..250, where the reference's
+// FP32 recurrence has 0.5e-7 at a = 0.025, 1.2e-7 at 2.5 and 3.7e-5 at 250 (its coefficients are rounded row by
+// row, here s is chosen from the rounded mu so that a constant field keeps its exact gain).
+//
+// A line is split into blocks of m elements held in the registers of one lane each.  Per block: f = sum mu^{m-1-j}
+// d_j and e = sum mu^j d_j (the block's contribution to everything right and left of it), one two-sided scan of
+// (f, e) over the line's blocks (factor W = mu^m per block; lane shuffles within a wave, one LDS exchange where a
+// line takes several waves), the mirror images at both ends in closed form, then the two recursions started with
+// the exact values of the neighbouring blocks.  Small workgroups (the waves of one line group, 1 to 8) with at most
+// one barrier: the groups of a CU drift apart and keep loads, arithmetic and stores in flight at the same time.
+//   scan:  U_k = sum_{k'<k} W^{k-1-k'} f_{k'},  T_k = sum_{k'>=k} W^{k'-k} e_{k'}
+//   line:  E = T_0, F = f_last + mu^{mlast} U_last (sums of d_j weighted by the distance to the first / last element)
+//   ends:  u_{-1} = (E + mu^n F) / (1 - mu^{2n}),  z_n = (F + mu^n E) / (1 - mu^{2n})
+//   block: u_{start-1} = U_k + mu^{m k} u_{-1},  Z = T_{k+1} + mu^{n - min(n, m(k+1))} z_n,
+//          x'_{end+1} = (mu u_end + Z) / (1 - mu^2)
+#include <algorithm>
+#include <cmath>
+
+#include "bfvm_internal.hpp"
+
+namespace bfvm {
+
+// Coefficient table of one axis, rows of S floats (powers of the rounded mu, computed in FP64).  A wave holds `kw`
+// blocks of a line; blocks rows each of mu^{m k} / (1 - mu^{2n}) and mu^{n - min(n, m(k+1))} / (1 - mu^{2n}) and kw
+// rows of mu^{m i} follow the single rows.  A workgroup keeps the table in LDS: held in registers, the 12 vectors a
+// lane needs cost it a wave per SIMD.
+enum filter_row
+{
+	fr_mu,
+	fr_s,	   // output factor
+	fr_inv1,   // 1 / (1 - mu^2)
+	fr_mun,	   // mu^n
+	fr_w,	   // W = mu^m
+	fr_mulast, // mu^mlast
+	fr_wk,	   // W^kw: one wave's blocks
+	fr_flast,  // mu^mlast W^i, i = the last block's index within its wave
+	fr_min,	   // this axis's Dirichlet faces: value and condition (1 or 0) at the line's first and last element
+	fr_min_on,
+	fr_max,
+	fr_max_on,
+	fr_ends
+};
+
+__global__ void filter_coefficients_kernel(float* __restrict__ tab, const float* __restrict__ D,
+										   const float* __restrict__ decay, const float* __restrict__ fval,
+										   const uint8_t* __restrict__ fcond, float dt, int shape, int dims, int n,
+										   int S, int m, int blocks, int kw)
+{
+	const int s = blockIdx.x * blockDim.x + threadIdx.x;
+	if (s >= S)
+		return;
+	const double a = (double)dt * (double)D[s] / ((double)shape * (double)shape);
+	const double lam = 1.0 + (double)decay[s] * (double)dt / dims; // B - 2a
+	const float muf = (float)(2.0 * a / (lam + 2.0 * a + sqrt(lam * (lam + 4.0 * a))));
+	const double mu = muf;
+	auto row = [&](int r, double v) { tab[(size_t)r * S + s] = (float)v; };
+	const int mlast = n - (blocks - 1) * m;
+	const double iden = 1.0 / (1.0 - pow(mu, 2.0 * n));
+	row(fr_mu, mu);
+	row(fr_s, (1.0 - mu) * (1.0 - mu) / lam);
+	row(fr_inv1, 1.0 / (1.0 - mu * mu));
+	row(fr_mun, pow(mu, (double)n));
+	row(fr_w, pow(mu, (double)m));
+	row(fr_mulast, pow(mu, (double)mlast));
+	row(fr_wk, pow(mu, (double)m * kw));
+	row(fr_flast, pow(mu, (double)mlast + (double)m * ((blocks - 1) % kw)));
+	// fval, fcond: [2][S] of this axis
+	row(fr_min, fval[s]);
+	row(fr_min_on, fcond[s] ? 1.0 : 0.0);
+	row(fr_max, fval[S + s]);
+	row(fr_max_on, fcond[S + s] ? 1.0 : 0.0);
+	for (int k = 0; k < blocks; k++)
+	{
+		row(fr_ends + k, pow(mu, (double)m * k) * iden);
+		row(fr_ends + blocks + k, pow(mu, (double)(n - min(n, m * (k + 1)))) * iden);
+	}
+	for (int i = 0; i < kw; i++)
+		row(fr_ends + 2 * blocks + i, pow(mu, (double)m * i));
+}
+
+// One axis of one instance, as launched.
+struct filter_args
+{
+	void* data;
+	const float* scale;		  // [S] storage scale (16-bit forms)
+	const unsigned* rounding; // step counter keying the stochastic rounding (16-bit forms)
+	const float* fval;		  // Dirichlet faces (null: none)
+	const uint8_t* fcond;
+	const float* tab;
+	int grid[3];
+	int S, dims, axis;
+	int m, blocks, mlast, kw; // block length, blocks of a line, elements of the last block, blocks per wave
+	int64_t tasks;			  // line groups, one per workgroup pass
+	int64_t stride;			  // elements between neighbours of a line
+	// a task is 1 << clog columns of 4 consecutive elements; columns run over ranges of row_elems elements, outer_stride
+	// apart (x: the S elements of a voxel, one range per row; y: the XS elements of a plane's rows, one range per z; z:
+	// the whole plane, one range)
+	int clog;
+	uint32_t columns, row_columns;
+	int64_t row_elems, outer_stride;
+	uint32_t row_mul, s_mul, x_mul; // fdiv pairs of row_columns, S and X (x axis: Y)
+	int row_shift, s_shift, x_shift;
+	// staged x rows: a task is `rows` rows of XS elements in the workgroup's LDS, lines_pass lines of a row at a time
+	int rows, lines_pass, passes, row_lines;
+	int64_t total_rows;
+	int table_floats;			// floats of the table; in LDS, the storage scales [S] follow (16-bit forms)
+	int exchange_at, rows_at; // LDS offsets in bytes of the exchange area and the staged rows
+};
+
+// value of lane `src` (any lane of the wave that runs this code)
+template <int V>
+__device__ __forceinline__ typename vec_of<V>::type lane_vec(typename vec_of<V>::type v, int src)
+{
+	typename vec_of<V>::type r;
+#pragma unroll
+	for (int c = 0; c < V; c++)
+		set_comp(r, c, __int_as_float(__builtin_amdgcn_ds_bpermute(src << 2, __float_as_int(comp(v, c)))));
+	return r;
+}
+
+// Values the compiler must take as new: without, everything that depends only on the thread and the mesh (an address
+// for each of the M elements, several times over) is computed once before the task loop and held in registers.
+__device__ __forceinline__ int fresh_lane_value(int x)
+{
+	asm volatile("" : "+v"(x));
+	return x;
+}
+template <typename T>
+__device__ __forceinline__ T fresh_uniform(T x)
+{
+	asm volatile("" : "+s"(x));
+	return x;
+}
+
+// Where a lane's block stands: block k = 0..last of its line, index i = 0..kw-1 among the blocks of its wave (`dist`
+// lanes apart), wave 0..waves-1 of the line; `slot` numbers the lines of the workgroup and `slots` counts them.
+struct filter_place
+{
+	int k, last, i, kw, wave, waves, lane, dist, slot, slots;
+	bool active;
+};
+
+// Elements of a block that every lane has: all of them (FULL), else at least half (choose_filter sees to it).  The
+// others are there where j < mk, by selects: branches around single loads or operations made the compiler wait for
+// each load where it was issued.
+template <int M, bool FULL>
+constexpr int sure() { return FULL ? M : M / 2; }
+
+// The filter on one block v[0..mk), mk = M except in the last block of a line (not FULL), the rest of its v zero on
+// entry.  store(j, x) runs in descending j < mk, in active lanes.  `sh`: [2][waves][slots] vectors and
+// [slots] more, exchanged once where a line takes several waves (then every thread of the workgroup comes here).
+template <int M, bool FULL, int V, typename Row, typename Store>
+__device__ __forceinline__ void filter_line(typename vec_of<V>::type (&v)[M], Row&& row, int mk, int blocks,
+											const filter_place& at, typename vec_of<V>::type* sh, Store&& store)
+{
+	// held to a tolerance, not to the reference's operation order: multiply-adds fuse
+#pragma clang fp contract(fast)
+	using vec = typename vec_of<V>::type;
+	constexpr int N = sure<M, FULL>();
+	auto has = [&](int j) { return j < N || j < mk; };
+	const vec mu = row(fr_mu);
+	vec f = v[0], e = v[M - 1];
+#pragma unroll
+	for (int j = 1; j < M; j++)
+		f = has(j) ? v[j] + mu * f : f;
+#pragma unroll
+	for (int j = M - 2; j >= 0; j--)
+		e = v[j] + mu * e;
+	// scan over the blocks of this wave; selects, not products with zero: lanes of other lines may hold anything
+	vec w = row(fr_w), sx = f, tx = e;
+	const int upto = min(at.kw - 1, at.last - (at.k - at.i)); // index of the line's last block in this wave
+#pragma unroll 1
+	for (int d = 1; d < at.kw && d <= at.last; d <<= 1)
+	{
+		const vec a = lane_vec<V>(sx, at.lane - d * at.dist), b = lane_vec<V>(tx, at.lane + d * at.dist);
+		sx = at.i >= d ? sx + w * a : sx;
+		tx = at.i + d <= upto ? tx + w * b : tx;
+		w = w * w;
+	}
+	vec u = lane_vec<V>(sx, at.lane - at.dist), z = lane_vec<V>(tx, at.lane + at.dist);
+	u = at.i > 0 ? u : vec(0.f);
+	z = at.i < upto ? z : vec(0.f);
+	vec E, F;
+	if (at.waves == 1)
+	{
+		const int lane0 = at.lane - at.i * at.dist;
+		E = lane_vec<V>(tx, lane0);
+		F = lane_vec<V>(f + row(fr_mulast) * u, lane0 + at.last * at.dist);
+	}
+	else
+	{
+		vec* shs = sh + at.wave * at.slots + at.slot;
+		vec* sht = shs + at.waves * at.slots;
+		if (at.active)
+		{
+			if (at.i == at.kw - 1)
+				*shs = sx;
+			if (at.i == 0)
+				*sht = tx;
+			if (at.k == at.last)
+				sh[2 * at.waves * at.slots + at.slot] = f + row(fr_mulast) * u;
+		}
+		__syncthreads();
+		const vec wk = row(fr_wk);
+		vec ul = vec(0.f), tr = vec(0.f), ulast = vec(0.f); // carried into this wave from the left, the right; last wave
+		E = vec(0.f);
+#pragma unroll 1
+		for (int o = 0; o < at.waves - 1; o++)
+		{
+			ulast = sh[o * at.slots + at.slot] + wk * ulast;
+			if (o < at.wave)
+				ul = ulast;
+		}
+#pragma unroll 1
+		for (int o = at.waves - 1; o >= 0; o--)
+		{
+			E = sh[(at.waves + o) * at.slots + at.slot] + wk * E;
+			if (o == at.wave + 1)
+				tr = E;
+		}
+		F = sh[2 * at.waves * at.slots + at.slot] + row(fr_flast) * ulast;
+		u = u + row(fr_ends + 2 * blocks + at.i) * ul;
+		z = z + row(fr_ends + 2 * blocks + at.kw - 1 - at.i) * tr;
+	}
+	const vec mun = row(fr_mun);
+	const int kt = min(at.k, at.last); // inactive lanes read a row that is there
+	u = u + row(fr_ends + kt) * (E + mun * F);
+	z = z + row(fr_ends + blocks + kt) * (F + mun * E);
+#pragma unroll
+	for (int j = 0; j < M; j++)
+	{
+		u = has(j) ? v[j] + mu * u : u;
+		v[j] = u;
+	}
+	vec x = (mu * u + z) * row(fr_inv1);
+	const vec s = row(fr_s);
+	if (at.active)
+	{
+#pragma unroll
+		for (int j = M - 1; j >= 0; j--)
+		{
+			x = has(j) ? v[j] + mu * x : x;
+			if (has(j))
+				store(j, s * x);
+		}
+	}
+}
+
+// The table (and the storage scales) into LDS, in two halves so that the loads fly with the data's: table_load
+// before the data's loads, table_store after them.  Tables of more than table_regs floats per thread continue in
+// the second half.
+constexpr int table_regs = 4;
+template <int K>
+__device__ __forceinline__ void table_load(const filter_args& a, float (&t)[table_regs])
+{
+	const int total = a.table_floats + (K == store_f32 ? 0 : a.S);
+#pragma unroll
+	for (int j = 0; j < table_regs; j++)
+	{
+		const int i = threadIdx.x + j * blockDim.x;
+		if (i < a.table_floats)
+			t[j] = gload(a.tab + i);
+		else if (i < total)
+			t[j] = gload(a.scale + i - a.table_floats);
+	}
+}
+template <int K>
+__device__ __forceinline__ void table_store(const filter_args& a, const float (&t)[table_regs], float* lt)
+{
+	const int total = a.table_floats + (K == store_f32 ? 0 : a.S);
+#pragma unroll
+	for (int j = 0; j < table_regs; j++)
+	{
+		const int i = threadIdx.x + j * blockDim.x;
+		if (i < total)
+			lt[i] = t[j];
+	}
+	for (int i = threadIdx.x + table_regs * blockDim.x; i < total; i += blockDim.x)
+		lt[i] = i < a.table_floats ? gload(a.tab + i) : gload(a.scale + i - a.table_floats);
+}
+
+// Order within a workgroup: one wave's LDS accesses complete in order and need no barrier.
+__device__ __forceinline__ void group_sync()
+{
+	if (blockDim.x > 64)
+		__syncthreads();
+	else
+	{
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+	}
+}
+
+// Workgroups are dispatched to the 8 XCDs in turn; this order gives each XCD one run of neighbouring tasks, so that
+// tasks which share cache lines or DRAM pages run behind one L2.  Measured on in-place passes over 2 GB: contiguous
+// rows 5.3 -> 5.6 TB/s, y columns of 128 bytes 4.8 -> 5.1, z columns 4.4 -> 4.9 TB/s.
+__device__ __forceinline__ int64_t xcd_order(int64_t b, int64_t W)
+{
+	const int64_t W8 = W - W % 8;
+	return b < W8 ? (b % 8) * (W8 / 8) + b / 8 : b;
+}
+
+__device__ __forceinline__ uint32_t fdivu(uint32_t n, uint32_t mul, int shift)
+{
+	return (uint32_t)(((uint64_t)n * mul) >> shift);
+}
+
+using raw16 = uint32_t __attribute__((ext_vector_type(4)));
+using raw16u = uint32_t __attribute__((ext_vector_type(4), aligned(2)));
+
+// 4 stored elements at element alignment (rows need not start on a 16-byte boundary)
+template <int K>
+struct unaligned4
+{
+	using type = typename store_of<K>::elem __attribute__((ext_vector_type(4), aligned(sizeof(typename store_of<K>::elem))));
+};
+
+// ---- one lane per (column of 4 consecutive elements, block) --------------------------------------------------------
+//
+// y, z: a task is C neighbouring columns: C lanes read one contiguous segment, and the 64 / C blocks of a wave the
+// segments m planes or rows apart.  Columns are flattened positions (x*S + s along y, (y*X + x)*S + s along z), so 4
+// need not divide S: each component takes its own substrate's constants.  Where 4 does not divide the range, its last
+// column is moved back to end with the range; it computes all 4 components and stores only those that no other
+// column owns.
+//
+// x, S a multiple of 4: the same with the elements of a voxel for a range.  A lane's loads walk along its row, so a
+// cache line is fetched once and hit by the loads that follow.  Rows staged through LDS with coalesced copies instead
+// took 24 against 13 us on 100^3 x 4, 89 against 75 us on 200^3 x 8, 890 against 850 us on 400^3 x 8, and in FP16 746
+// against 576 us.
+//
+// NT: densities that exceed the 256 MB Infinity Cache are streamed past it on y and z.  400^3 x 8, whole diffusion
+// solve: FP32 2.96 -> 2.65 ms, FP16 1.90 -> 1.85 ms; along x, whose lines are hit several times, it costs twice the
+// time.
+template <int M, bool FULL, int K, bool NT>
+__device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_t task, float* lt,
+													typename vec_of<4>::type* sh, bool first)
+{
+	using vec = typename vec_of<4>::type;
+	using elem = typename store_of<K>::elem;
+	using uv = typename unaligned4<K>::type;
+	filter_place at;
+	const int tid = fresh_lane_value(threadIdx.x);
+	at.lane = tid & 63;
+	at.wave = tid >> 6;
+	at.waves = blockDim.x >> 6;
+	at.dist = at.slots = 1 << a.clog;
+	at.slot = at.lane & (at.slots - 1);
+	at.i = at.lane >> a.clog;
+	at.kw = a.kw;
+	at.k = at.wave * a.kw + at.i;
+	at.last = a.blocks - 1;
+	const uint32_t col = (uint32_t)(task << a.clog) + at.slot;
+	at.active = col < a.columns && at.k <= at.last;
+	const int k = at.active ? at.k : 0;
+	const uint32_t cl = at.active ? col : 0;
+	const uint32_t outer = fdivu(cl, a.row_mul, a.row_shift);
+	const uint32_t q0 = (cl - outer * a.row_columns) * 4;
+	const int back = max(0, (int)(q0 + 4 - (uint32_t)a.row_elems)); // components owned by the column before
+	const uint32_t q = q0 - back;
+	const int64_t off = outer * a.outer_stride + q + (int64_t)(k * M) * a.stride;
+	const int64_t stride = fresh_uniform(a.stride);
+	const int S = fresh_uniform(a.S);
+	const int mk = FULL || k < at.last ? M : a.mlast; // (of lanes that read)
+
+	int s[4];
+	const uint32_t vox = fdivu(q, a.s_mul, a.s_shift); // voxel of the first component within the row range
+	s[0] = (int)(q - vox * (uint32_t)S);
+#pragma unroll
+	for (int c = 1; c < 4; c++)
+		s[c] = s[c - 1] + 1 == S ? 0 : s[c - 1] + 1;
+
+	float t[table_regs];
+	if (first)
+		table_load<K>(a, t);
+	const elem* p = (const elem*)a.data + off;
+	constexpr int N = sure<M, FULL>();
+	uv raw[M];
+	// lanes past the columns or the line read the first column's first block, elements past a block its first one
+#pragma unroll
+	for (int j = 0; j < M; j++)
+	{
+		const uv* src = (const uv*)(j < N || j < mk ? p + j * stride : p);
+		raw[j] = NT ? __builtin_nontemporal_load(src) : gload(src);
+	}
+	if (first)
+	{
+		table_store<K>(a, t, lt);
+		group_sync();
+	}
+	auto row = [&](int r) -> vec {
+		const float* x = lt + r * S;
+		if (S % 4 == 0)
+			return *(const vec*)(x + s[0]);
+		return vec { x[s[0]], x[s[1]], x[s[2]], x[s[3]] };
+	};
+	vec v[M];
+#pragma unroll
+	for (int j = 0; j < M; j++)
+	{
+		v[j] = __builtin_convertvector(raw[j], vec);
+		if (j >= N)
+			v[j] = j < mk ? v[j] : vec(0.f);
+	}
+	// an address the compiler cannot tie to the loads' (kept for the stores, those would hold 2 M registers)
+	elem* o = (elem*)a.data + off;
+	asm volatile("" : "+v"(o));
+	uint32_t h = K == store_f32 ? 0u : sr_seed(off, rounding_key(a.rounding, 1 + a.axis));
+	filter_line<M, FULL, 4>(v, row, mk, a.blocks, at, sh, [&](int j, vec x) {
+		uv y;
+		if constexpr (K == store_f32)
+			y = x;
+		else
+		{
+#pragma unroll
+			for (int c = 0; c < 4; c += 2)
+			{
+				h = xorshift32(h);
+				const auto pr = sr_pair<K>(x[c], x[c + 1], h);
+				y[c] = pr[0];
+				y[c + 1] = pr[1];
+			}
+		}
+		if (back == 0)
+		{
+			if constexpr (NT)
+				__builtin_nontemporal_store(y, (uv*)(o + j * stride));
+			else
+				gstore((uv*)(o + j * stride), y);
+		}
+		else
+		{
+#pragma unroll
+			for (int c = 1; c < 4; c++)
+				if (c >= back)
+					gstore(o + j * stride + c, (elem)y[c]);
+		}
+	});
+
+	// Dirichlet faces, written over the solved values in the order x-, x+, y-, y+, z-, z+
+	// (host/dirichlet_solver.cpp:91-110): a face of this axis at the line's ends, a face of another axis through the
+	// whole line.  Same lane, same addresses: the later store stays.
+	if (a.fcond && at.active)
+	{
+		const float* ls = lt + a.table_floats;
+		auto scale = [&]() { return vec { ls[s[0]], ls[s[1]], ls[s[2]], ls[s[3]] }; };
+		for (int d = 0; d < a.dims; d++)
+		{
+			if (d == a.axis)
+			{
+#pragma unroll
+				for (int mx = 0; mx < 2; mx++)
+					if (at.k == (mx ? at.last : 0))
+					{
+						const vec on = row(mx ? fr_max_on : fr_min_on);
+						vec val = row(mx ? fr_max : fr_min);
+						if constexpr (K != store_f32)
+							val = val * scale();
+#pragma unroll
+						for (int c = 0; c < 4; c++)
+							if (on[c] != 0.f && c >= back)
+								gstore(o + (mx ? mk - 1 : 0) * stride + c, (elem)val[c]);
+					}
+				continue;
+			}
+			for (int c = back; c < 4; c++)
+			{
+				// coordinate d of this component's voxel (its components may lie in different voxels)
+				// x: outer = z*Y + y; y: outer = z, vc = x; z: vc = y*X + x
+				const uint32_t vc = fdivu(q + c, a.s_mul, a.s_shift);
+				const uint32_t hi = fdivu(a.axis == 0 ? outer : vc, a.x_mul, a.x_shift);
+				const uint32_t lo = (a.axis == 0 ? outer : vc) - hi * (uint32_t)a.grid[a.axis == 0 ? 1 : 0];
+				const int cd = (int)(a.axis == 0 ? (d == 1 ? lo : hi) : a.axis == 1 ? (d == 0 ? vc : outer) : (d == 0 ? lo : hi));
+				for (int mx = 0; mx < 2; mx++)
+				{
+					if (cd != (mx ? a.grid[d] - 1 : 0) || !gload(a.fcond + (2 * d + mx) * S + s[c]))
+						continue;
+					float val = gload(a.fval + (2 * d + mx) * S + s[c]);
+					if constexpr (K != store_f32)
+						val *= ls[s[c]];
+					for (int j = 0; j < mk; j++)
+						gstore(o + j * stride + c, (elem)val);
+				}
+			}
+		}
+	}
+}
+
+template <int M, bool FULL, int K, bool NT>
+__global__ __launch_bounds__(512) void filter_columns_kernel(filter_args a)
+{
+	extern __shared__ raw16 filter_lds[];
+	using vec = typename vec_of<4>::type;
+	// two exchange areas in turn: a wave may still read one pass's while another writes the next one's
+	const int area = (2 * (blockDim.x >> 6) + 1) << a.clog;
+	vec* sh = (vec*)((char*)filter_lds + a.exchange_at);
+	int parity = 0;
+	bool first = true;
+	for (int64_t t = xcd_order(blockIdx.x, gridDim.x); t < a.tasks; t += gridDim.x, parity ^= 1, first = false)
+		filter_columns_task<M, FULL, K, NT>(a, t, (float*)filter_lds, sh + parity * area, first);
+}
+
+// ---- x, substrate counts that 4 does not divide: rows staged through LDS, one element per lane and position --------
+//
+// A workgroup (one wave, or several for long rows) copies whole rows (contiguous in memory) to LDS with
+// 16-byte accesses, runs the lines from there and copies the rows back; m is odd, so that the LDS reads of
+// neighbouring blocks fall in different banks.  One wave's LDS accesses complete in order and need no barrier.
+// The 16-byte pieces of a task's rows that a thread moves (passes == 1: the rows fill at most 64 lanes x M positions
+// per wave).  A workgroup loads its next task's rows into registers before it solves the present one.
+template <int M, int K>
+struct row_pieces
+{
+	static constexpr int elem_bytes = K == store_f32 ? 4 : 2;
+	static constexpr int count = (M * elem_bytes + 15) / 16;
+	raw16 piece[count];
+	typename store_of<K>::elem tail; // the rows' last elements, fewer than a piece
+};
+
+template <int K>
+struct row_range
+{
+	static constexpr int VE = K == store_f32 ? 4 : 8; // elements of a piece
+	int64_t row0;
+	int nrows, nel, nvec;
+	typename store_of<K>::elem* g;
+	__device__ __forceinline__ row_range(const filter_args& a, int64_t task)
+	{
+		row0 = task * a.rows;
+		nrows = (int)min((int64_t)a.rows, a.total_rows - row0);
+		nel = nrows * (int)a.row_elems;
+		nvec = nel / VE;
+		g = (typename store_of<K>::elem*)a.data + row0 * a.row_elems;
+	}
+};
+
+template <int M, int K>
+__device__ __forceinline__ void rows_fetch(const filter_args& a, int64_t task, row_pieces<M, K>& x)
+{
+	const row_range<K> r(a, task);
+	const int tid = fresh_lane_value(threadIdx.x), nthr = blockDim.x;
+#pragma unroll
+	for (int j = 0; j < row_pieces<M, K>::count; j++)
+		x.piece[j] = gload((const raw16u*)r.g + min(tid + nthr * j, r.nvec - 1)); // past the end: the last one again
+	x.tail = gload(r.g + min(r.nvec * r.VE + tid, r.nel - 1));
+}
+
+template <int M, int K>
+__device__ __forceinline__ void rows_put(const filter_args& a, int64_t task, const row_pieces<M, K>& x, char* rows)
+{
+	const row_range<K> r(a, task);
+	const int tid = fresh_lane_value(threadIdx.x), nthr = blockDim.x;
+#pragma unroll
+	for (int j = 0; j < row_pieces<M, K>::count; j++)
+		((raw16*)rows)[min(tid + nthr * j, r.nvec - 1)] = x.piece[j];
+	// rows longer than the pieces (several passes)
+	for (int i = tid + nthr * row_pieces<M, K>::count; i < r.nvec; i += nthr)
+		((raw16*)rows)[i] = gload((const raw16u*)r.g + i);
+	if (tid < r.nel - r.nvec * r.VE)
+		((typename store_of<K>::elem*)rows)[r.nvec * r.VE + tid] = x.tail;
+}
+
+// The staged rows of one task: solve, Dirichlet faces, copy back.
+template <int M, bool FULL, int K>
+__device__ __forceinline__ void filter_rows_task(const filter_args& a, int64_t task, char* lds)
+{
+	using elem = typename store_of<K>::elem;
+	const int tid = fresh_lane_value(threadIdx.x), nthr = blockDim.x;
+	const int S = fresh_uniform(a.S), XS = (int)a.row_elems;
+	const row_range<K> rg(a, task);
+	const int64_t row0 = rg.row0;
+	const int nrows = rg.nrows, nvec = rg.nvec;
+	elem* g = rg.g;
+	elem* l = (elem*)(lds + a.rows_at);
+	const float* lt = (const float*)lds;
+	const float* ls = lt + a.table_floats;
+
+	filter_place at;
+	at.lane = tid & 63;
+	at.wave = tid >> 6;
+	at.waves = nthr >> 6;
+	at.dist = at.slots = a.lines_pass;
+	at.slot = at.lane % a.lines_pass;
+	const int b = at.lane / a.lines_pass;
+	at.kw = a.kw;
+	at.i = b % a.kw;
+	at.k = at.wave * a.kw + at.i;
+	at.last = a.blocks - 1;
+	const int r = b / a.kw; // several rows only in one wave, which then holds all blocks of a line
+	const int mk = FULL || at.k < at.last ? M : a.mlast;
+	constexpr int N = sure<M, FULL>();
+	const bool in_rows = r < nrows && at.k <= at.last;
+
+	for (int pass = 0; pass < a.passes; pass++)
+	{
+		const int line = pass * a.lines_pass + at.slot;
+		if (pass > 0 && at.waves > 1)
+			__syncthreads(); // the exchange area of the pass before
+		at.active = in_rows && line < a.row_lines;
+		const int pos = r * XS + at.k * M * S + line;
+		float v[M];
+		const elem* lv = l + (at.active ? pos : 0); // inactive lanes read what is there
+#pragma unroll
+		for (int j = 0; j < M; j++)
+		{
+			v[j] = (float)lv[j < N || j < mk ? j * S : 0];
+			if (j >= N)
+				v[j] = j < mk ? v[j] : 0.f;
+		}
+		uint32_t h = K == store_f32 ? 0u : sr_seed(row0 * XS + pos, rounding_key(a.rounding, 1));
+		const int So = fresh_uniform(S); // the stores' addresses are not the loads' held
+		elem* lo = l + pos;
+		const int sl = min(line, a.row_lines - 1);
+		auto row = [&](int rw) { return lt[rw * S + sl]; };
+		filter_line<M, FULL, 1>(v, row, mk, a.blocks, at, (float*)(lds + a.exchange_at), [&](int j, float x) {
+			elem* o = lo + j * So;
+			if constexpr (K == store_f32)
+				*o = x;
+			else
+			{
+				h = xorshift32(h);
+				*o = sr_pair<K>(x, 0.f, h)[0];
+			}
+		});
+		// Dirichlet x faces at the row's ends
+		if (a.fcond && at.active)
+			for (int mx = 0; mx < 2; mx++)
+				if (at.k == (mx ? at.last : 0) && row(mx ? fr_max_on : fr_min_on) != 0.f)
+				{
+					const float val = row(mx ? fr_max : fr_min);
+					l[pos + (mx ? mk - 1 : 0) * S] = (elem)(K == store_f32 ? val : val * ls[sl]);
+				}
+	}
+	group_sync();
+	// then the rows on y and z faces, in the order y-, y+, z-, z+ (host/dirichlet_solver.cpp:91-110)
+	if (a.fcond)
+	{
+		bool any = false;
+		for (int rr = 0; rr < nrows; rr++)
+		{
+			const uint32_t row = (uint32_t)(row0 + rr), z = fdivu(row, a.row_mul, a.row_shift);
+			const int y = (int)(row - z * (uint32_t)a.grid[1]);
+			for (int f = 2; f < 2 * a.dims; f++)
+			{
+				if ((f < 4 ? y : (int)z) != ((f & 1) ? a.grid[f >> 1] - 1 : 0))
+					continue;
+				any = true;
+				for (int i = tid; i < XS; i += nthr)
+				{
+					const int sc = i % S;
+					if (!gload(a.fcond + f * S + sc))
+						continue;
+					float val = gload(a.fval + f * S + sc);
+					if constexpr (K != store_f32)
+						val *= ls[sc];
+					l[rr * XS + i] = (elem)val;
+				}
+			}
+		}
+		if (any)
+			group_sync();
+	}
+	constexpr int U = row_pieces<M, K>::count;
+	raw16 w[U];
+#pragma unroll
+	for (int j = 0; j < U; j++)
+		w[j] = ((const raw16*)l)[min(tid + nthr * j, nvec - 1)];
+#pragma unroll
+	for (int j = 0; j < U; j++)
+		gstore((raw16u*)g + min(tid + nthr * j, nvec - 1), (raw16u)w[j]);
+	for (int i = tid + nthr * U; i < nvec; i += nthr)
+		gstore((raw16u*)g + i, (raw16u)((const raw16*)l)[i]);
+	if (tid < rg.nel - nvec * rg.VE)
+		gstore(g + nvec * rg.VE + tid, l[nvec * rg.VE + tid]);
+}
+
+template <int M, bool FULL, int K>
+__global__ __launch_bounds__(512) void filter_rows_kernel(filter_args a)
+{
+	extern __shared__ raw16 filter_lds[];
+	char* lds = (char*)filter_lds;
+	row_pieces<M, K> x;
+	float tab[table_regs];
+	int64_t t = xcd_order(blockIdx.x, gridDim.x);
+	table_load<K>(a, tab);
+	rows_fetch<M, K>(a, t, x);
+	table_store<K>(a, tab, (float*)lds);
+	for (; t < a.tasks; t += gridDim.x)
+	{
+		rows_put<M, K>(a, t, x, lds + a.rows_at);
+		group_sync();
+		if (t + gridDim.x < a.tasks)
+			rows_fetch<M, K>(a, t + gridDim.x, x);
+		filter_rows_task<M, FULL, K>(a, t, lds);
+		group_sync(); // the next rows are staged over these
+	}
+}
+
+// ---- host side ------------------------------------------------------------------------------------------------------
+
+
+// block lengths the kernels are built for: odd ones where the rows are staged (LDS banks)
+static constexpr int column_blocks[] = { 2, 3, 4, 5, 7, 9, 11, 13, 14, 16, 18, 20, 22, 25 };
+static constexpr int row_blocks[] = { 3, 5, 7, 9, 11, 13, 15, 17 };
+
+// f(block length, every block full) as compile-time constants, for the lengths listed
+template <int... Ms, typename F>
+static void by_block(int m, bool full, F&& f)
+{
+	auto one = [&](auto c) {
+		if (c == m)
+			full ? f(c, std::true_type()) : f(c, std::false_type());
+	};
+	(one(std::integral_constant<int, Ms>()), ...);
+}
+
+// The filter needs 0 <= mu < 1, i.e. a >= 0 and 1 + decay*dt/dims > 0; mu is kept below 0.999 (a < 1e6), where the
+// FP32 error against an FP64 solve stays at 2e-7.
+static bool filter_coefficients_ok(const bfvm_ctx* ctx, int axis)
+{
+	const double h2 = (double)ctx->mesh.vs[axis] * ctx->mesh.vs[axis];
+	for (int s = 0; s < ctx->mesh.S; s++)
+	{
+		const double a = (double)ctx->mesh.dt * ctx->D[s] / h2;
+		const double lam = 1.0 + (double)ctx->decay[s] * ctx->mesh.dt / ctx->mesh.dims;
+		if (!(a >= 0.0) || !(lam > 0.0) || !std::isfinite(a) || !std::isfinite(lam))
+			return false;
+		if (!(2.0 * a / (lam + 2.0 * a + std::sqrt(lam * (lam + 4.0 * a))) <= 0.999))
+			return false;
+	}
+	return true;
+}
+
+// Workgroups: enough that every SIMD holds two waves, while blocks stay long (fewer exchanges, wider loads).
+static constexpr int64_t filter_fill_waves = 2048;
+static constexpr int filter_max_waves = 8; // waves of a workgroup
+static constexpr int64_t infinity_cache_bytes = (int64_t)256 << 20;
+
+// LDS bytes of the coefficient table and the storage scales, to the next vector
+static int filter_lds_table(const bfvm_ctx* ctx, int blocks, int kw)
+{
+	const int S = ctx->mesh.S;
+	const int64_t floats = (int64_t)(fr_ends + 2 * blocks + kw) * S + (ctx->storage == BFVM_STORAGE_F32 ? 0 : S);
+	return (int)std::min<int64_t>((floats * 4 + 15) / 16 * 16, 1 << 20);
+}
+
+// Expected time of an element, up to a factor: a block's scan costs about 8 elements; lanes without elements (the share
+// `used` has them) hold no loads in flight; blocks of at most 16 elements leave room for 3 waves per SIMD, longer ones
+// for 2; a short last block takes selects; more than 4 waves per workgroup wait for each other.  Measured (ms, y / z,
+// FP32 c3 = 8 columns, 16-bit c4 = 16 columns): 400^3 x 8 FP32 16 elements 0.68 / 0.71, 25 elements 0.73 / 0.76, 9
+// elements 0.87 / 0.88; FP16 25 elements 0.46 / 0.49, 16 elements (7 waves) 0.78 / 0.78; 256^3 x 16 BF16 16 elements
+// 0.26 / 0.30, 22 elements (short last block, 3 waves) 0.34 / 0.37; 200^3 x 8 FP32 25 elements 0.068 / 0.071, 16
+// elements 0.069 / 0.072; 100^3 x 4 FP32 13 elements (8 blocks) 0.012 / 0.011, 25 (4 blocks) 0.013 / 0.012.
+static double filter_cost(int m, int waves, bool full, double used)
+{
+	return (m + 8.0) / m * std::pow(used, -0.4) * (m <= 16 ? 0.75 : 1.0) * (full ? 1.0 : 1.15) * (waves > 4 ? 1.5 : 1.0);
+}
+
+filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
+{
+	const auto& g = ctx->mesh;
+	const int n = g.grid[axis], S = g.S;
+	const int64_t XS = (int64_t)g.grid[0] * S, e = (int64_t)storage_bytes(ctx->storage);
+	filter_plan best, quick;
+	double best_cost = 0, quick_cost = 0;
+	if (n < 2 || !filter_coefficients_ok(ctx, axis))
+		return best;
+	// best: the cheapest lengths; quick: the shortest chain of operations, for meshes that do not fill the card anyway
+	auto consider = [&](const filter_plan& p, double used) {
+		const double cost = filter_cost(p.m, p.waves, n % p.m == 0, used), chain = std::max(p.m, 7) + 8 * p.waves;
+		if (best.blocks == 0 || cost < best_cost)
+		{
+			best = p;
+			best_cost = cost;
+		}
+		if (quick.blocks == 0 || chain < quick_cost)
+		{
+			quick = p;
+			quick_cost = chain;
+		}
+	};
+	// a line's last block holds at least half its length (sure)
+	auto fits = [&](int m) { return n - ((n + m - 1) / m - 1) * m >= m / 2; };
+	if (axis == 0 && S % 4 != 0)
+	{
+		const int L = S;
+		const int64_t rows = (int64_t)g.grid[1] * g.grid[2];
+		if (XS * e < 16 || rows >= (int64_t)1 << 31)
+			return best;
+		for (int m : row_blocks)
+		{
+			if (!fits(m))
+				continue;
+			filter_plan p;
+			p.m = m;
+			p.blocks = (n + m - 1) / m;
+			p.staged = true;
+			if (p.blocks * L <= 64)
+			{
+				p.lines_pass = L;
+				p.kw = p.blocks;
+				p.rows = 64 / (L * p.blocks);
+			}
+			else
+			{
+				// one row: as many of its lines side by side as a wave holds, their blocks over several waves
+				p.lines_pass = std::min({ L, 64, std::max(1, 64 * filter_max_waves / p.blocks) });
+				p.kw = std::min(64 / p.lines_pass, p.blocks);
+				p.waves = (p.blocks + p.kw - 1) / p.kw;
+				p.rows = 1;
+			}
+			if (p.waves > filter_max_waves)
+				continue;
+			p.passes = (L + p.lines_pass - 1) / p.lines_pass;
+			p.exchange_at = filter_lds_table(ctx, p.blocks, p.kw);
+			p.rows_at =
+				p.exchange_at + (p.waves > 1 ? ((2 * p.waves + 1) * p.lines_pass * 4 + 15) / 16 * 16 : 0);
+			const int64_t lds = p.rows_at + (p.rows * XS * e + 15) / 16 * 16;
+			if (lds > 64 * 1024)
+				continue;
+			p.lds = (int)lds;
+			p.tasks = (rows + p.rows - 1) / p.rows;
+			p.lines_group = p.rows * L;
+			consider(p, (double)p.rows * L * n / (64.0 * p.waves * m * p.passes));
+		}
+	}
+	else
+	{
+		const int64_t row_elems = axis == 0 ? S : axis == 1 ? XS : (int64_t)g.grid[1] * XS;
+		const int64_t row_columns = (row_elems + 3) / 4;
+		const int64_t columns = row_columns * (axis == 0 ? (int64_t)g.grid[1] * g.grid[2] : axis == 1 ? g.grid[2] : 1);
+		if (row_elems < 4 || columns >= ((int64_t)1 << 31) / 4)
+			return best;
+		// y, z: 128-byte segments (8 lanes of FP32, 16 of 16-bit storage): a wave whose segments are 64 bytes reaches
+		// 4.2-4.7 TB/s on 2 GB, with 128 bytes 4.8-5.2 TB/s.  x: 4 rows side by side (400^3 x 8 FP16 0.58 ms, one row 0.65,
+		// 256^3 x 16 BF16 0.25, one row 0.33 ms).  Long lines take fewer columns where 8 waves cannot hold them.
+		int widest = e == 4 ? 3 : 4;
+		if (axis == 0)
+			for (widest = 2; widest < 5 && (1 << widest) < S; widest++)
+				;
+		for (int clog = widest; clog >= 0 && best.blocks == 0; clog--)
+			for (int m : column_blocks)
+			{
+				if (!fits(m))
+					continue;
+				filter_plan p;
+				p.m = m;
+				p.blocks = (n + m - 1) / m;
+				p.clog = clog;
+				p.kw = 64 >> clog;
+				p.waves = (p.blocks + p.kw - 1) / p.kw;
+				if (p.waves > filter_max_waves)
+					continue;
+				p.exchange_at = filter_lds_table(ctx, p.blocks, p.kw);
+				p.lds = p.exchange_at + (p.waves > 1 ? 2 * ((2 * p.waves + 1) << clog) * 16 : 0);
+				if (p.lds > 64 * 1024)
+					continue;
+				p.tasks = (columns + (1 << clog) - 1) >> clog;
+				p.lines_group = (1 << clog) * (S % 4 == 0 ? 1 : 4);
+				consider(p, (double)n / (m * p.kw * p.waves));
+			}
+	}
+	filter_plan& p = best.tasks * best.waves < filter_fill_waves ? quick : best;
+	p.streamed = axis != 0 && (int64_t)(ctx->mesh.V * S) * e > infinity_cache_bytes;
+	return p;
+}
+
+size_t filter_table_floats(const filter_plan& p, int S) { return (size_t)(fr_ends + 2 * p.blocks + p.kw) * S; }
+
+void launch_filter_coefficients(const bfvm_ctx* ctx, int axis, const filter_plan& p, float* tab, hipStream_t stream)
+{
+	const int S = ctx->mesh.S;
+	hipLaunchKernelGGL(filter_coefficients_kernel, dim3((S + 63) / 64), dim3(64), 0, stream, tab, ctx->d_D,
+					   ctx->d_decay, ctx->face_val + 2 * axis * S, ctx->face_cond + 2 * axis * S, ctx->mesh.dt,
+					   ctx->mesh.vs[axis], ctx->mesh.dims, ctx->mesh.grid[axis], S, p.m, p.blocks, p.kw);
+	BFVM_HIP(hipGetLastError());
+}
+
+static filter_args make_filter_args(const bfvm_ctx* ctx, int axis, const filter_plan& p, const float* tab)
+{
+	const auto& g = ctx->mesh;
+	filter_args a {};
+	a.data = ctx->dens;
+	a.scale = ctx->dscale;
+	a.rounding = ctx->rounding_step;
+	a.fval = ctx->has_faces ? ctx->face_val : nullptr;
+	a.fcond = ctx->has_faces ? ctx->face_cond : nullptr;
+	a.tab = tab;
+	for (int d = 0; d < 3; d++)
+		a.grid[d] = g.grid[d];
+	a.S = g.S;
+	a.dims = g.dims;
+	a.axis = axis;
+	a.m = p.m;
+	a.blocks = p.blocks;
+	a.kw = p.kw;
+	a.mlast = g.grid[axis] - (p.blocks - 1) * p.m;
+	a.tasks = p.tasks;
+	a.table_floats = (int)filter_table_floats(p, g.S);
+	a.exchange_at = p.exchange_at;
+	const int64_t XS = (int64_t)g.grid[0] * g.S;
+	fast_divisor((uint32_t)g.S, a.s_mul, a.s_shift);
+	fast_divisor((uint32_t)g.grid[axis == 0 ? 1 : 0], a.x_mul, a.x_shift);
+	if (p.staged)
+	{
+		a.row_elems = XS;
+		a.rows = p.rows;
+		a.lines_pass = p.lines_pass;
+		a.passes = p.passes;
+		a.row_lines = g.S;
+		a.total_rows = (int64_t)g.grid[1] * g.grid[2];
+		a.rows_at = p.rows_at;
+		fast_divisor((uint32_t)g.grid[1], a.row_mul, a.row_shift);
+		return a;
+	}
+	const int64_t plane = (int64_t)g.grid[1] * XS;
+	a.clog = p.clog;
+	a.stride = axis == 0 ? g.S : axis == 1 ? XS : plane;
+	a.row_elems = a.stride;
+	a.outer_stride = axis == 0 ? XS : axis == 1 ? plane : 0;
+	a.row_columns = (uint32_t)((a.row_elems + 3) / 4);
+	a.columns = a.row_columns * (uint32_t)(axis == 0 ? (int64_t)g.grid[1] * g.grid[2] : axis == 1 ? g.grid[2] : 1);
+	fast_divisor(a.row_columns, a.row_mul, a.row_shift);
+	return a;
+}
+
+void launch_filter_sweep(bfvm_ctx* ctx, int axis)
+{
+	const axis_tables& t = ctx->axes[axis];
+	const filter_plan& p = t.filter;
+	const filter_args a = make_filter_args(ctx, axis, p, t.filter_tab);
+	int64_t cap = ctx->sweep_workgroups[axis] > 0 ? ctx->sweep_workgroups[axis] : (int64_t)1 << 24;
+	// Staged rows: while the densities stay in the Infinity Cache, 8 waves per CU that prefetch their next rows beat one
+	// pass of short-lived ones (200^3 x 8: 89 against 97 us); from memory one pass is the faster (400^3 x 8: 822 against
+	// 848 us).
+	if (p.staged && (int64_t)(ctx->mesh.V * ctx->mesh.S * storage_bytes(ctx->storage)) <= infinity_cache_bytes)
+		cap = std::min<int64_t>(cap, filter_fill_waves / p.waves);
+	const dim3 blocks((unsigned)std::min(p.tasks, cap)), threads(64 * p.waves);
+	const size_t lds = p.lds;
+	const bool full = a.mlast == a.m;
+	by_storage(ctx->storage, [&](auto kind) {
+		constexpr int K = decltype(kind)::value;
+		if (p.staged)
+			by_block<3, 5, 7, 9, 11, 13, 15, 17>(p.m, full, [&](auto m, auto f) {
+				hipLaunchKernelGGL((filter_rows_kernel<m, f, K>), blocks, threads, lds, ctx->stream, a);
+			});
+		else
+			by_block<2, 3, 4, 5, 7, 9, 11, 13, 14, 16, 18, 20, 22, 25>(p.m, full, [&](auto m, auto f) {
+				if (p.streamed)
+					hipLaunchKernelGGL((filter_columns_kernel<m, f, K, true>), blocks, threads, lds, ctx->stream, a);
+				else
+					hipLaunchKernelGGL((filter_columns_kernel<m, f, K, false>), blocks, threads, lds, ctx->stream, a);
+			});
+	});
+	BFVM_HIP(hipGetLastError());
+}
+
+} // namespace bfvm
