@@ -2,6 +2,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
+#include <numeric>
 #include <stdexcept>
 #include <unordered_map>
 
@@ -1362,15 +1364,16 @@ int bfvm_benchmark(bfvm_ctx* ctx, int32_t what, int32_t iterations, float* avg_m
 
 namespace bfvm {
 
-// The per-instance kernels of a batch step run on the batch's stream with the batch's rounding counter.
+// The per-instance kernels of a batch step run on one of the batch's streams with the batch's rounding counter.
 struct batch_override
 {
 	bfvm_ctx* c;
 	hipStream_t stream;
 	unsigned* rounding;
-	batch_override(bfvm_ctx* ctx, const bfvm_batch* b) : c(ctx), stream(ctx->stream), rounding(ctx->rounding_step)
+	batch_override(bfvm_ctx* ctx, const bfvm_batch* b, hipStream_t on)
+		: c(ctx), stream(ctx->stream), rounding(ctx->rounding_step)
 	{
-		c->stream = b->stream;
+		c->stream = on;
 		c->rounding_step = b->rounding;
 	}
 	~batch_override()
@@ -1390,10 +1393,17 @@ static void free_batch(bfvm_batch* b)
 			(void)hipGraphDestroy(g.graph);
 		g = graph_slot {};
 	}
-	for (int a = 0; a < 3; a++)
-		free_batch_sweep(b, a);
 	free_batch_gradient(b);
 	free_batch_cell(b);
+	for (int i = 0; i < bfvm_batch::branches; i++)
+	{
+		if (b->branch_event[i])
+			(void)hipEventDestroy(b->branch_event[i]);
+		if (i > 0 && b->branch_stream[i])
+			(void)hipStreamDestroy(b->branch_stream[i]);
+		b->branch_event[i] = nullptr;
+		b->branch_stream[i] = nullptr;
+	}
 	if (b->rounding)
 		(void)hipFree(b->rounding);
 	b->rounding = nullptr;
@@ -1432,33 +1442,54 @@ static uint64_t batch_epoch(const bfvm_batch* b)
 	return e;
 }
 
+// one(instance) for every instance, its launches on its branch: a step's launches of one instance follow each other
+// on a branch, so the ends of one instance's kernels are covered by the other branches', and an instance of ordinary
+// size stays in the Infinity Cache from one axis to the next.  The branches are forked from the batch's stream and
+// joined to it, also when a launch is refused.  One launch per axis over all instances (workgroups walking a list of
+// line groups) took, for a step without gradient of 64 instances in 16-bit storage, 3.84 ms; branches 2.96 ms.
+template <typename F>
+static void on_branches(bfvm_batch* b, F&& one)
+{
+	BFVM_HIP(hipEventRecord(b->branch_event[0], b->stream));
+	for (int i = 1; i < bfvm_batch::branches; i++)
+		BFVM_HIP(hipStreamWaitEvent(b->branch_stream[i], b->branch_event[0], 0));
+	std::exception_ptr failed;
+	try
+	{
+		for (size_t i = 0; i < b->ctx.size(); i++)
+		{
+			batch_override o(b->ctx[i], b, b->branch_stream[b->branch_of[i]]);
+			one(b->ctx[i]);
+		}
+	}
+	catch (...)
+	{
+		failed = std::current_exception();
+	}
+	for (int i = 1; i < bfvm_batch::branches; i++)
+	{
+		BFVM_HIP(hipEventRecord(b->branch_event[i], b->branch_stream[i]));
+		BFVM_HIP(hipStreamWaitEvent(b->stream, b->branch_event[i], 0));
+	}
+	if (failed)
+		std::rethrow_exception(failed);
+}
+
 static void enqueue_batch_sweeps(bfvm_batch* b)
 {
 	if (b->storage != BFVM_STORAGE_F32)
 	{
-		batch_override o(b->ctx[0], b);
+		batch_override o(b->ctx[0], b, b->stream);
 		launch_advance_rounding(b->ctx[0]);
 	}
-	for (bfvm_ctx* c : b->ctx)
-	{
-		batch_override o(c, b);
+	on_branches(b, [](bfvm_ctx* c) {
 		enqueue_dirichlet(c);
-	}
-	for (int axis = 0; axis < 3; axis++)
-	{
-		for (int i : b->axes[axis].single)
+		for (int axis = 0; axis < c->mesh.dims; axis++)
 		{
-			batch_override o(b->ctx[i], b);
-			launch_sweep(b->ctx[i], axis);
+			launch_sweep(c, axis);
+			launch_dirichlet_interior(c);
 		}
-		launch_batched_sweep(b, axis);
-		for (bfvm_ctx* c : b->ctx)
-			if (axis < c->mesh.dims)
-			{
-				batch_override o(c, b);
-				launch_dirichlet_interior(c);
-			}
-	}
+	});
 }
 
 static void enqueue_batch_gradient(bfvm_batch* b)
@@ -1466,7 +1497,7 @@ static void enqueue_batch_gradient(bfvm_batch* b)
 	launch_batched_gradient(b);
 	for (int i : b->grad.single)
 	{
-		batch_override o(b->ctx[i], b);
+		batch_override o(b->ctx[i], b, b->stream);
 		launch_gradient(b->ctx[i]);
 	}
 }
@@ -1481,7 +1512,7 @@ static void enqueue_batch_cell(bfvm_batch* b, bool recompute)
 	}
 	for (bfvm_ctx* c : b->ctx)
 	{
-		batch_override o(c, b);
+		batch_override o(c, b, b->stream);
 		launch_cell(c, recompute);
 	}
 }
@@ -1533,8 +1564,30 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 			BFVM_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
 			BFVM_HIP(hipMalloc(&b->rounding, sizeof(unsigned)));
 			BFVM_HIP(hipMemsetAsync(b->rounding, 0, sizeof(unsigned), b->stream));
-			for (int a = 0; a < 3; a++)
-				prepare_batch_sweep(b, a);
+			for (int32_t i = 0; i < count; i++)
+				for (int a = 0; a < b->ctx[i]->mesh.dims; a++)
+					if (b->ctx[i]->mesh.grid[a] > 1)
+						check_batch_axis(b->ctx[i], a, i);
+			b->branch_stream[0] = b->stream;
+			for (int i = 0; i < bfvm_batch::branches; i++)
+			{
+				if (i > 0)
+					BFVM_HIP(hipStreamCreateWithFlags(&b->branch_stream[i], hipStreamNonBlocking));
+				BFVM_HIP(hipEventCreateWithFlags(&b->branch_event[i], hipEventDisableTiming));
+			}
+			// instances in order of size, each to the branch with the least work
+			std::vector<int> order(count);
+			std::iota(order.begin(), order.end(), 0);
+			auto size = [&](int i) { return b->ctx[i]->mesh.V * b->ctx[i]->mesh.S; };
+			std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return size(x) > size(y); });
+			size_t load[bfvm_batch::branches] = {};
+			b->branch_of.assign(count, 0);
+			for (int i : order)
+			{
+				const int at = (int)(std::min_element(load, load + bfvm_batch::branches) - load);
+				b->branch_of[i] = at;
+				load[at] += size(i);
+			}
 			prepare_batch_gradient(b);
 			BFVM_HIP(hipStreamSynchronize(b->stream));
 		}
@@ -1619,11 +1672,6 @@ int bfvm_batch_autotune(bfvm_batch* batch)
 		BFVM_HIP(hipStreamSynchronize(batch->stream));
 		if (apply_cached_batch_tuning(batch))
 		{
-			for (int a = 0; a < 3; a++)
-			{
-				free_batch_sweep(batch, a);
-				prepare_batch_sweep(batch, a);
-			}
 			free_batch_gradient(batch);
 			prepare_batch_gradient(batch);
 			BFVM_HIP(hipStreamSynchronize(batch->stream));
@@ -1657,11 +1705,6 @@ int bfvm_batch_autotune(bfvm_batch* batch)
 		catch (...)
 		{
 			restore();
-			for (int a = 0; a < 3; a++)
-			{
-				free_batch_sweep(batch, a);
-				prepare_batch_sweep(batch, a);
-			}
 			free_batch_gradient(batch);
 			prepare_batch_gradient(batch);
 			throw;
@@ -1669,11 +1712,6 @@ int bfvm_batch_autotune(bfvm_batch* batch)
 		restore();
 		// the plans hold the instances' buffers: rebuild them on the real densities, recompute the gradients the
 		// timings overwrote, and let the secretion plan refresh
-		for (int a = 0; a < 3; a++)
-		{
-			free_batch_sweep(batch, a);
-			prepare_batch_sweep(batch, a);
-		}
 		free_batch_gradient(batch);
 		prepare_batch_gradient(batch);
 		enqueue_batch_gradient(batch);
@@ -1736,7 +1774,10 @@ int bfvm_batch_benchmark(bfvm_batch* batch, int32_t what, int32_t iterations, fl
 			case BFVM_KERNEL_SWEEP_X:
 			case BFVM_KERNEL_SWEEP_Y:
 			case BFVM_KERNEL_SWEEP_Z:
-				launch_batched_sweep(batch, what - BFVM_KERNEL_SWEEP_X);
+				on_branches(batch, [&](bfvm_ctx* c) {
+					if (what - BFVM_KERNEL_SWEEP_X < c->mesh.dims)
+						launch_sweep(c, what - BFVM_KERNEL_SWEEP_X);
+				});
 				break;
 			case BFVM_KERNEL_GRADIENT:
 				launch_batched_gradient(batch);

@@ -172,7 +172,7 @@ bool apply_cached_batch_tuning(bfvm_batch* b)
 // Text file, one entry per line:
 //   sweep <axis> <X> <Y> <Z> <S> <storage> <algorithm> <chunk> <lines> <workgroups>
 //   gradient <X> <Y> <Z> <S> <storage> <algorithm> <workgroups> <stacked> [<order>]
-//   batch <key> <group threads [3][2]> <max blocks [3][2]> <gradient tiles> <gradient blocks> <gradient rows>
+//   batch <key> <12 numbers, kept but not used> <gradient tiles> <gradient blocks> <gradient rows>
 //         <gradient z planes> <gradient split> <gradient stacked>
 void save_tuning(const char* path)
 {
@@ -189,12 +189,8 @@ void save_tuning(const char* path)
 	for (const auto& [k, t] : g_batch_cache)
 	{
 		std::fprintf(f, "batch %s", k.c_str());
-		for (int a = 0; a < 3; a++)
-			for (int w = 0; w < 2; w++)
-				std::fprintf(f, " %d", t.group_threads[a][w]);
-		for (int a = 0; a < 3; a++)
-			for (int w = 0; w < 2; w++)
-				std::fprintf(f, " %d", t.max_blocks[a][w]);
+		for (int v : t.sweep_fields)
+			std::fprintf(f, " %d", v);
 		std::fprintf(f, " %d %d %d %d %d %d\n", t.gradient_tiles, t.gradient_blocks, t.gradient_rows, t.gradient_zchunk,
 					 t.gradient_split, t.gradient_stacked);
 	}
@@ -251,12 +247,8 @@ void load_tuning(const char* path)
 			std::string key;
 			bfvm_batch::tuning_t t;
 			ok = static_cast<bool>(in >> key);
-			for (int a = 0; a < 3 && ok; a++)
-				for (int w = 0; w < 2 && ok; w++)
-					ok = static_cast<bool>(in >> t.group_threads[a][w]);
-			for (int a = 0; a < 3 && ok; a++)
-				for (int w = 0; w < 2 && ok; w++)
-					ok = static_cast<bool>(in >> t.max_blocks[a][w]);
+			for (int i = 0; i < 12 && ok; i++)
+				ok = static_cast<bool>(in >> t.sweep_fields[i]);
 			ok = ok && static_cast<bool>(in >> t.gradient_tiles >> t.gradient_blocks >> t.gradient_rows >>
 										  t.gradient_zchunk >> t.gradient_split >> t.gradient_stacked) &&
 				 (t.gradient_rows == 4 || t.gradient_rows == 8);
@@ -338,55 +330,10 @@ void autotune_context(bfvm_ctx* ctx, bool tune_gradient)
 	ctx->epoch++;
 }
 
-// Batches: per axis and thread layout the target threads of a line group and the workgroup cap of the
-// work-list launch; for the gradient the tiles per work item and the workgroup cap.  Each candidate rebuilds
-// that part of the plan.
+// Batches: the tiles per work item and the workgroup cap of the gradient, each candidate rebuilding the plan.
 void autotune_batch(bfvm_batch* b)
 {
 	const int reps = 3;
-	for (int axis = 0; axis < 3; axis++)
-	{
-		if (!b->axes[axis].any)
-			continue;
-		for (int w = 0; w < 2; w++)
-		{
-			if (b->axes[axis].parts[w].nitems == 0)
-				continue;
-			const int max_threads = w == 0 ? 512 : batch_max_threads;
-			int best_threads = b->tuning.group_threads[axis][w], best_blocks = b->tuning.max_blocks[axis][w];
-			float best_t = 1e30f;
-			for (int threads : { 128, 256, 512, 1024 })
-			{
-				if (threads > max_threads)
-					continue;
-				for (int blocks : { 1024, 2048, 4096, 8192 })
-				{
-					b->tuning.group_threads[axis][w] = threads;
-					b->tuning.max_blocks[axis][w] = blocks;
-					free_batch_sweep(b, axis);
-					try
-					{
-						prepare_batch_sweep(b, axis);
-					}
-					catch (const std::runtime_error&)
-					{
-						continue;
-					}
-					const float t = best_ms(b->stream, reps, [&] { launch_batched_sweep(b, axis); });
-					if (t < best_t)
-					{
-						best_t = t;
-						best_threads = threads;
-						best_blocks = blocks;
-					}
-				}
-			}
-			b->tuning.group_threads[axis][w] = best_threads;
-			b->tuning.max_blocks[axis][w] = best_blocks;
-			free_batch_sweep(b, axis);
-			prepare_batch_sweep(b, axis);
-		}
-	}
 	if (b->grad.nitems[2] > 0)
 	{
 		// tile shape first (rows per thread, z planes per tile), then the work distribution

@@ -410,8 +410,7 @@ struct cell_args
 	const unsigned* rounding;
 };
 
-constexpr int batch_chunk = 16; // register block of the staged and batched sweeps (one line per thread)
-constexpr int batch_max_threads = 1024;
+constexpr int batch_chunk = 16; // register block of the staged sweeps (one line per thread)
 
 struct graph_slot
 {
@@ -494,8 +493,8 @@ struct bfvm_ctx
 	bool stream_used = false;
 };
 
-// Many microenvironments advanced together (bfvm_batch_*): one launch per sweep axis and one for the
-// gradient over all instances, driven by device work lists; per-instance kernels for the rest.
+// Many microenvironments advanced together (bfvm_batch_*): the instances' sweeps on parallel branches of one graph,
+// one launch for the gradient over all instances, driven by device work lists.
 struct bfvm_batch
 {
 	int device = 0;
@@ -504,22 +503,13 @@ struct bfvm_batch
 	std::vector<uint64_t> generation; // each instance's initialization when the batch was made
 	int storage = BFVM_STORAGE_F32;
 	unsigned* rounding = nullptr; // step counter of the stochastic rounding, shared by all instances
-	struct sweep_plan
-	{
-		// instances grouped by the vector width of their threads (4, 1), one launch per group
-		struct part
-		{
-			void* inst = nullptr; // device part_args per instance
-			bfvm::batch_item* items = nullptr;
-			int nitems = 0;
-			size_t lds = 0;
-			int threads = 0;
-			int blocks = 0;
-		} parts[2];
-		std::vector<float*> tables; // coefficient tables owned by the batch
-		std::vector<int> single;	// instances whose mesh has length 1 on this axis (per-instance launch)
-		bool any = false;
-	} axes[3];
+	// The instances' sweeps run as chains (x, y, z of one instance after the other), spread over branches that run side
+	// by side: a chain's densities stay in the caches between its sweeps, and a small instance's latency hides behind
+	// the other branches.
+	static constexpr int branches = 4;
+	hipStream_t branch_stream[branches] = {}; // [0] is `stream`
+	hipEvent_t branch_event[branches] = {};   // [0]: the fork
+	std::vector<int> branch_of;				 // per instance
 	struct gradient_plan
 	{
 		void* inst = nullptr; // device gradient_args per instance
@@ -542,13 +532,11 @@ struct bfvm_batch
 		bool batched = false;
 		uint64_t epoch = ~0ull;
 	} cell;
-	// launch shapes of the work-list kernels (bfvm_batch_autotune picks them): per axis and thread layout
-	// (4-element vectors, one element) the threads a line group aims for and the workgroup cap; for the
-	// gradient the y rows per thread, the z planes per tile, the tiles per work item and the workgroup cap
+	// launch shapes of the work-list gradient (bfvm_batch_autotune picks them): the y rows per thread, the z planes per
+	// tile, the tiles per work item and the workgroup cap
 	struct tuning_t
 	{
-		int group_threads[3][2] = { { 256, 256 }, { 256, 256 }, { 256, 256 } };
-		int max_blocks[3][2] = { { 2048, 2048 }, { 2048, 2048 }, { 2048, 2048 } };
+		int sweep_fields[12] = { 256, 256, 256, 256, 256, 256, 2048, 2048, 2048, 2048, 2048, 2048 }; // of tuning files
 		int gradient_tiles = 4;
 		int gradient_blocks = 8192;
 		int gradient_rows = 4;	  // y rows per thread (4 or 8)
@@ -591,6 +579,7 @@ void launch_cell_release(bfvm_ctx* ctx, int index);
 void launch_voxel_positions(bfvm_ctx* ctx, int count, const float* d_pos, int* d_out);
 
 filter_plan choose_filter(const bfvm_ctx* ctx, int axis);
+void check_batch_axis(const bfvm_ctx* ctx, int axis, int instance);
 size_t filter_table_floats(const filter_plan& p, int S);
 void launch_filter_coefficients(const bfvm_ctx* ctx, int axis, const filter_plan& p, float* tab, hipStream_t stream);
 void launch_filter_sweep(bfvm_ctx* ctx, int axis);
@@ -601,9 +590,6 @@ int supported_chunk(int request);
 partition choose_partition(const bfvm_ctx* ctx, int axis, int chunk, int lines_request, int max_vec);
 
 // batched kernels (bfvm_batch): plans are built once at bfvm_batch_create; launches enqueue on b->stream
-void prepare_batch_sweep(bfvm_batch* b, int axis);
-void launch_batched_sweep(bfvm_batch* b, int axis);
-void free_batch_sweep(bfvm_batch* b, int axis);
 void prepare_batch_gradient(bfvm_batch* b);
 void launch_batched_gradient(bfvm_batch* b);
 void free_batch_gradient(bfvm_batch* b);

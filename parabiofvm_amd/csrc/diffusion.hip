@@ -80,9 +80,7 @@ constexpr int max_types = 4;
 // floats of the reduced-system table of a line of P blocks
 __host__ __device__ constexpr int reduced_table_floats(int P, int S) { return 4 * 2 * P * S + S; }
 // LDS of a partitioned sweep workgroup, in floats: the coefficient table [4][ntypes][mb][Sp], the reduced-system
-// table, A and the storage scale [Sp] each, then (from the returned offset, 16-byte aligned) the reduced rows.  Sp is
-// S, or S + V - 1 when substrate vectors wrap (rows extended periodically so V consecutive entries from any
-// substrate are the wrapped substrates).
+// table, A and the storage scale [Sp] each, then (from the returned offset, 16-byte aligned) the reduced rows.
 __host__ __device__ constexpr int part_rows_offset(int ntypes, int mb, int P, int S, int Sp)
 {
 	return (4 * ntypes * mb * Sp + reduced_table_floats(P, S) + 2 * Sp + 3) / 4 * 4;
@@ -522,40 +520,10 @@ __device__ __forceinline__ void thread_slot(int t, int SG, int P, int lpg, int& 
 	}
 }
 
-// Substrate s and voxel coordinates cc of component c of a thread's substrate vector (first substrate s0,
-// line coordinates `coord`).  Without wrapping the V substrates belong to one voxel.  With wrapping (y/z
-// sweeps whose substrate count V does not divide) the vector holds V consecutive flattened plane positions,
-// so component c is substrate (s0 + c) mod S of a voxel (s0 + c) / S further along x (and, along z, possibly
-// in the next y row).
-template <int AXIS, bool WRAP>
-__device__ __forceinline__ void comp_coords(const sweep_geometry& g, const int* coord, int s0, int c, int& s, int* cc)
-{
-	cc[0] = coord[0];
-	cc[1] = coord[1];
-	cc[2] = coord[2];
-	if constexpr (!WRAP)
-		s = s0 + c;
-	else
-	{
-		static_assert(AXIS != 0, "x lines hold whole voxels");
-		const int t = s0 + c;
-		s = t % g.S;
-		const int adv = t / g.S;
-		if constexpr (AXIS == 1)
-			cc[0] += adv;
-		else
-		{
-			const int xx = coord[0] + adv;
-			cc[0] = xx % g.X;
-			cc[1] += xx / g.X;
-		}
-	}
-}
-
 // Dirichlet faces for the elements a thread stores: the common case (an interior line away from its ends)
 // stores the solved value; lines on a face of another axis, and the two ends of the line, resolve every
 // face in the order x-, x+, y-, y+, z-, z+ (host/dirichlet_solver.cpp:91-110).
-template <int AXIS, int V, bool WRAP, int K>
+template <int AXIS, int V, int K>
 __device__ __forceinline__ typename vec_of<V>::type faces_slow(typename vec_of<V>::type x, const sweep_geometry& g,
 															  int s0, const int* coord, int i,
 															  const typename vec_of<V>::type& scale)
@@ -563,14 +531,12 @@ __device__ __forceinline__ typename vec_of<V>::type faces_slow(typename vec_of<V
 	const int grid[3] = { g.X, g.Y, g.Z };
 	for (int c = 0; c < V; c++)
 	{
-		int s = s0 + c, cc[3];
-		if constexpr (WRAP)
-			comp_coords<AXIS, WRAP>(g, coord, s0, c, s, cc);
+		const int s = s0 + c;
 		float val = comp(x, c);
 		bool face = false;
 		for (int d = 0; d < g.dims; d++)
 		{
-			const int cd = d == AXIS ? i : (WRAP ? cc[d] : coord[d]);
+			const int cd = d == AXIS ? i : coord[d];
 			if (cd == 0 && g.fcond[(2 * d) * g.S + s])
 			{
 				val = g.fval[(2 * d) * g.S + s];
@@ -667,8 +633,7 @@ __device__ __forceinline__ void twisted_solve(const float4* tab, float mu, int S
 // synchronises the workgroup before reusing `lds`.  FULL: every block holds M - 1 or M elements
 // (a.base >= M - 1), so only the last element's presence differs between threads and the other per-element
 // guards are known at compile time.
-template <int M, int AXIS, int V, int K, bool PF = (K != store_f32 && AXIS != 0), bool NT = (K == store_f32 && AXIS != 0),
-		  bool FULL = false>
+template <int M, int AXIS, int V, int K, bool PF, bool NT, bool FULL>
 __device__ __forceinline__ void sweep_groups(const part_args& a, float* lds, int64_t g_first, int64_t g_end,
 											 int64_t g_step)
 {
@@ -894,7 +859,7 @@ __device__ __forceinline__ void sweep_groups(const part_args& a, float* lds, int
 					{
 						const bool fj = j == 0 ? (face_lo || (last(j) && face_hi)) : (last(j) ? face_hi : line_face);
 						if (fj)
-							x = faces_slow<AXIS, V, false, K>(x, g, s0, coord, start + j, sc);
+							x = faces_slow<AXIS, V, K>(x, g, s0, coord, start + j, sc);
 					}
 					// NT: FP32 y/z outputs of a large instance are streamed past the caches (measured: y 0.964 ->
 					// 0.947 ms, z 1.037 -> 1.023 ms on 400^3 x 8; along x, whose rows stay in cache, and for the
@@ -903,251 +868,6 @@ __device__ __forceinline__ void sweep_groups(const part_args& a, float* lds, int
 						__builtin_nontemporal_store(x, (vec*)((float*)g.data + off0 + j * stride));
 					else
 						dstore_sr_stream<K, V>(g.data, off0 + j * stride, x, h);
-				}
-			}
-		}
-		__syncthreads();
-	}
-}
-
-// sweep_groups for y/z lines whose threads hold V consecutive flattened plane positions that may wrap over
-// the substrates (V need not divide S): per-substrate tables in LDS extended periodically to S + V - 1 entries
-// and read component by component, per-component substrate and voxel coordinates for the faces.
-template <int M, int AXIS, int V, int K, bool FULL = false>
-__device__ __forceinline__ void sweep_groups_wrapped(const part_args& a, float* lds, int64_t g_first,
-													 int64_t g_end, int64_t g_step)
-{
-	// this path is held to a tolerance, not to the reference's operation order: multiply-adds may fuse
-#pragma clang fp contract(fast)
-	using vec = typename vec_of<V>::type;
-	const sweep_geometry& g = a.g;
-	int S = g.S; // redefined opaquely in every group iteration, below
-	const int P = a.P;
-	const int lpg = a.lines_per_group;
-	const int Sp = S + V - 1; // LDS row length of the per-substrate tables
-	const int ncoef = 4 * a.ntypes * a.mb * Sp;
-	const int nred = reduced_table_floats(P, S);
-	float* lcoef = lds;
-	float* lred = lds + ncoef;
-	// per-substrate A and storage scale, so the group loop reads no global memory besides the densities
-	float* lA = lred + nred;
-	float* lscale = lA + Sp;
-	vec* rv = (vec*)(lds + part_rows_offset(a.ntypes, a.mb, P, S, Sp)); // [2P][lpg]
-
-	for (int i = threadIdx.x; i < ncoef; i += blockDim.x)
-	{
-		const int row = i / Sp;
-		lcoef[i] = a.coef[row * S + (i - row * Sp) % S];
-	}
-	for (int i = threadIdx.x; i < nred; i += blockDim.x)
-		lred[i] = a.red[i];
-	for (int i = threadIdx.x; i < Sp; i += blockDim.x)
-	{
-		const int si = i % S;
-		lA[i] = a.A[si];
-		lscale[i] = K == store_f32 ? 1.f : g.scale[si];
-	}
-	// V table entries from substrate s0 on, component by component (wrapping leaves the start unaligned)
-	auto cld = [](const float* p) -> vec {
-		vec r;
-#pragma unroll
-		for (int c = 0; c < V; c++)
-			set_comp(r, c, p[c]);
-		return r;
-	};
-
-	int line_local, k;
-	thread_slot<AXIS>(threadIdx.x, 1, P, lpg, line_local, k);
-	int64_t stride = line_stride<AXIS>(g); // redefined opaquely in every group iteration, below
-	const int grid[3] = { g.X, g.Y, g.Z };
-	const size_t fstride = (size_t)a.ntypes * a.mb * Sp;
-	const uint32_t key = K == store_f32 ? 0u : rounding_key(g.rounding, 1 + AXIS);
-
-	int start = 0, mk = 0, type = 0;
-	if (k >= 0)
-	{
-		start = k * a.base + min(k, a.rem);
-		mk = a.base + (k < a.rem ? 1 : 0);
-		type = (P == 1) ? 0 : (k == 0 ? 0 : (k == P - 1 ? 3 : (k < a.rem ? 1 : 2)));
-	}
-	auto has = [&](int j) { return (FULL && j < M - 1) || j < mk; };
-	auto last = [&](int j) { return (!FULL || j >= M - 2) && j == mk - 1; };
-	__syncthreads();
-
-	// 16-bit forms load the next group's block while this one is solved (as in sweep_groups)
-	constexpr bool prefetch = K != store_f32;
-	typename svec_of<K, V>::type pre[prefetch ? M : 1];
-	auto fetch = [&](int64_t grp) {
-		const int64_t ln = grp * lpg + line_local;
-		if (k >= 0 && ln < a.lines)
-		{
-			int64_t b = 0;
-			int sx = 0;
-			int cd[3];
-			vline_coords<AXIS, V>(a, ln, b, sx, cd);
-			const int64_t o = b + (int64_t)start * stride;
-#pragma unroll
-			for (int j = 0; j < M; j++)
-				if (has(j))
-					pre[j] = draw<K, V>(g.data, o + j * stride);
-		}
-	};
-	if constexpr (prefetch)
-		if (g_first < g_end)
-			fetch(g_first);
-
-	for (int64_t group = g_first; group < g_end; group += g_step)
-	{
-		// The unrolled element loops address memory at j * stride and the LDS tables at j * S for every j; held
-		// across the group loop those 16 + 16 uniform offsets overflow the scalar registers and spill into
-		// vector-register lanes (hundreds of SGPR spills per kernel).  Marking stride and S as redefined here
-		// makes them recomputed per group instead: measured on 640^3 x 16 BF16 (autotuned) sweeps 8.7 / 9.3 /
-		// 10.0 -> 7.5 / 8.7 / 8.5 ms, and 10-12 fewer VGPRs in every 4-substrate kernel.
-		asm volatile("" : "+s"(stride), "+s"(S));
-		const int64_t line = group * lpg + line_local;
-		const bool active = k >= 0 && line < a.lines;
-		int64_t base = 0;
-		int s0 = 0;
-		int coord[3] = { 0, 0, 0 };
-		if (active)
-			vline_coords<AXIS, V>(a, line, base, s0, coord);
-		const int64_t off0 = base + (int64_t)start * stride; // element offset of the block's first value
-		const float* cr = lcoef + 0 * fstride + (size_t)type * a.mb * Sp + s0;
-		const float* cg = lcoef + 1 * fstride + (size_t)type * a.mb * Sp + s0;
-		const float* ca = lcoef + 2 * fstride + (size_t)type * a.mb * Sp + s0;
-		const float* cgp = lcoef + 3 * fstride + (size_t)type * a.mb * Sp + s0;
-
-		vec v[M];
-		if constexpr (prefetch)
-		{
-			if (active)
-			{
-#pragma unroll
-				for (int j = 0; j < M; j++)
-					if (has(j))
-						v[j] = dcvt<K, V>(pre[j]);
-			}
-			if (group + g_step < g_end)
-				fetch(group + g_step);
-		}
-		if (active)
-		{
-			if constexpr (!prefetch)
-			{
-#pragma unroll
-				for (int j = 0; j < M; j++)
-					if (has(j))
-						v[j] = dload<K, V>(g.data, off0 + j * stride);
-			}
-			// 16-bit forms solve on the stored values: the scale is a power of two, so solving on scaled values and
-			// scaling the solution give the same bits, and only the Dirichlet values set below need the scale
-			// forward elimination inside the block: v_j = r_j (v_j - A v_{j-1}), written as r_j v_j - (r_j A) v_{j-1}
-			// so that the recurrence carries one multiply-add
-			const vec As = cld(lA + s0);
-#pragma unroll
-			for (int j = 0; j < M; j++)
-			{
-				if (has(j))
-				{
-					const vec r = cld(cr + j * Sp);
-					if (j < 2)
-						v[j] = r * v[j];
-					else
-						v[j] = r * v[j] - (r * As) * v[j - 1];
-				}
-			}
-			// backward elimination towards the block's last unknown
-#pragma unroll
-			for (int j = M - 3; j >= 1; j--)
-				if (has(j + 2))
-					v[j] = v[j] - cld(cg + j * Sp) * v[j + 1];
-			if (has(2))
-				v[0] = cld(ca) * (v[0] - cld(cg) * v[1]);
-			rv[(2 * k) * lpg + line_local] = v[0];
-#pragma unroll
-			for (int j = 1; j < M; j++)
-				if (last(j))
-					rv[(2 * k + 1) * lpg + line_local] = v[j];
-		}
-		__syncthreads();
-		// reduced systems: one pair of adjacent threads per (line, substrate), solving from both ends.  On every
-		// axis the first substrate of line l is (l V) mod S (the lines of a row, column or plane position run
-		// over the substrate groups), and the group's share of it is uniform across the workgroup.
-		const int group_s = (int)((group * lpg * V) % S);
-		for (int pr = threadIdx.x >> 1; threadIdx.x < (blockDim.x & ~1u) && pr < lpg * V; pr += blockDim.x >> 1)
-		{
-			const int ll = pr / V, c = pr - ll * V;
-			if (group * lpg + ll < a.lines)
-			{
-				const int sc = (group_s + ll * V + c) % S;
-				twisted_solve((const float4*)lred + sc, lred[8 * P * S + sc], S, (float*)rv + ll * V + c, lpg * V, P,
-							  threadIdx.x & 1);
-			}
-		}
-		__syncthreads();
-		if (active)
-		{
-			const vec u0 = rv[(2 * k) * lpg + line_local];
-			const vec u1 = rv[(2 * k + 1) * lpg + line_local];
-			// faces touching this line: another axis's face through the whole line, or this axis's faces at
-			// the line ends
-			bool line_face = false, end_min = false, end_max = false;
-			// only lines on a face of another axis and the end blocks of a line can meet a face: the
-			// conditions are read for those alone
-			bool near_face = start == 0 || start + mk == a.n;
-			for (int c = 0; c < V; c++)
-			{
-				int sc, cc[3];
-				comp_coords<AXIS, true>(g, coord, s0, c, sc, cc);
-				for (int d = 0; d < g.dims; d++)
-					if (d != AXIS)
-						near_face |= cc[d] == 0 || cc[d] == grid[d] - 1;
-			}
-			if (g.fcond && near_face)
-			{
-				for (int c = 0; c < V; c++)
-				{
-					int sc, cc[3];
-					comp_coords<AXIS, true>(g, coord, s0, c, sc, cc);
-					for (int d = 0; d < g.dims; d++)
-					{
-						const bool cmin = g.fcond[(2 * d) * S + sc] != 0;
-						const bool cmax = g.fcond[(2 * d + 1) * S + sc] != 0;
-						const int cd = cc[d];
-						if (d == AXIS)
-						{
-							end_min |= cmin;
-							end_max |= cmax;
-						}
-						else
-							line_face |= (cmin && cd == 0) || (cmax && cd == grid[d] - 1);
-					}
-				}
-			}
-			const vec sc = cld(lscale + s0);
-			uint32_t h = K == store_f32 ? 0u : sr_seed(off0, key);
-			const bool face_lo = line_face || (start == 0 && end_min);
-			const bool face_hi = line_face || (start + mk == a.n && end_max);
-			const bool wave_face = __ballot(face_lo || face_hi) != 0;
-#pragma unroll
-			for (int j = 0; j < M; j++)
-			{
-				if (has(j))
-				{
-					vec x;
-					if (j == 0)
-						x = u0;
-					else if (last(j))
-						x = u1;
-					else
-						x = v[j] - cld(ca + j * Sp) * u0 - cld(cgp + j * Sp) * u1;
-					if (wave_face)
-					{
-						const bool fj = j == 0 ? (face_lo || (last(j) && face_hi)) : (last(j) ? face_hi : line_face);
-						if (fj)
-							x = faces_slow<AXIS, V, true, K>(x, g, s0, coord, start + j, sc);
-					}
-					dstore_sr_stream<K, V>(g.data, off0 + j * stride, x, h);
 				}
 			}
 		}
@@ -1186,35 +906,6 @@ void sweep_partitioned_kernel(part_args a)
 		sweep_groups<M, AXIS, V, K, PF, NT, true>(a, lds, first, a.groups, W);
 	else
 		sweep_groups<M, AXIS, V, K, PF, NT, false>(a, lds, first, a.groups, W);
-}
-
-// Many microenvironments in one launch: workgroups walk a work list of (instance, group range) items.  The
-// instances of one launch have V substrates (x) or flattened plane positions (y, z) per thread, with 16-element
-// register blocks; on y and z the V positions may cross voxels (substrate vectors wrap).
-template <int AXIS, int K, int V>
-__global__ __launch_bounds__(V == 1 ? batch_max_threads : 512) void sweep_batched_kernel(
-	const part_args* __restrict__ inst, const batch_item* __restrict__ items, int nitems)
-{
-	extern __shared__ float lds[];
-	for (int it = blockIdx.x; it < nitems; it += gridDim.x)
-	{
-		const batch_item w = items[it];
-		const part_args a = inst[w.instance];
-		if constexpr (V > 1 && AXIS != 0)
-		{
-			if (a.base >= batch_chunk - 1)
-				sweep_groups_wrapped<batch_chunk, AXIS, V, K, true>(a, lds, w.begin, w.end, 1);
-			else
-				sweep_groups_wrapped<batch_chunk, AXIS, V, K, false>(a, lds, w.begin, w.end, 1);
-		}
-		else
-		{
-			if (a.base >= batch_chunk - 1)
-				sweep_groups<batch_chunk, AXIS, V, K, (K != store_f32), false, true>(a, lds, w.begin, w.end, 1);
-			else
-				sweep_groups<batch_chunk, AXIS, V, K, (K != store_f32), false, false>(a, lds, w.begin, w.end, 1);
-		}
-	}
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -2001,6 +1692,29 @@ static void launch_sweep_storage(bfvm_ctx* ctx, int axis)
 		launch_partitioned_axis<2, K>(ctx, g, t);
 }
 
+// The meshes a batch accepts: every axis fits 16-element blocks of one workgroup (512 threads with 4 elements per
+// thread, 1024 with one) and 64 KB of LDS.
+void check_batch_axis(const bfvm_ctx* ctx, int axis, int instance)
+{
+	const std::string who = "batched sweep: instance " + std::to_string(instance);
+	const int S = ctx->mesh.S;
+	const int64_t XS = (int64_t)ctx->mesh.grid[0] * S;
+	const int64_t unit = axis == 0 ? S : (axis == 1 ? XS : (int64_t)ctx->mesh.grid[1] * XS);
+	const int V = unit % 4 == 0 ? 4 : 1;
+	const int max_threads = V == 1 ? 1024 : 512;
+	partition p = choose_partition(ctx, axis, batch_chunk, 1, 1);
+	if (p.chunk != batch_chunk)
+		throw std::runtime_error(who + " does not fit 16-element register blocks (axis too long)");
+	p.vec = V;
+	const int SG = axis == 0 ? S / V : 1;
+	const int request = axis == 0 ? std::max(1, 256 / (SG * p.P)) : std::max(8, 256 / p.P / 8 * 8);
+	group_shape(axis, SG, p.P, request, max_threads, p.lpg, p.threads);
+	if (p.threads > max_threads)
+		throw std::runtime_error(who + " does not fit one workgroup (axis too long)");
+	if (partition_lds_bytes(p, S, p.lpg, V > 1 && axis != 0) > 64 * 1024)
+		throw std::runtime_error("batched sweep: coefficient tables exceed 64 KB of LDS");
+}
+
 void launch_sweep(bfvm_ctx* ctx, int axis)
 {
 	switch (ctx->storage)
@@ -2015,143 +1729,6 @@ void launch_sweep(bfvm_ctx* ctx, int axis)
 		launch_sweep_storage<store_f32>(ctx, axis);
 		break;
 	}
-}
-
-} // namespace bfvm
-
-namespace bfvm {
-
-// ------------------------------------------------------------------------------------------------
-// batched sweeps
-// ------------------------------------------------------------------------------------------------
-
-void free_batch_sweep(bfvm_batch* b, int axis)
-{
-	auto& ax = b->axes[axis];
-	for (float* t : ax.tables)
-		if (t)
-			BFVM_HIP(hipFree(t));
-	ax.tables.clear();
-	for (auto& part : ax.parts)
-	{
-		if (part.inst)
-			BFVM_HIP(hipFree(part.inst));
-		if (part.items)
-			BFVM_HIP(hipFree(part.items));
-	}
-	ax = bfvm_batch::sweep_plan {};
-}
-
-// Per instance: the partition with 16-element register blocks; its own coefficient tables; work items of about
-// 64K elements.  Each thread holds V = 4 or 1 consecutive elements of a row: on x, V substrates of a voxel
-// (V divides S); on y and z, V flattened plane positions (V divides the row or plane length, so every vector
-// is aligned), which wrap over the substrates when V does not divide S.  4-element vectors move 16 (FP32) or
-// 8 bytes per lane, against 4 or 2 for one element.  (Two-element vectors made the compiler move the register
-// blocks through scratch memory, so they are not used.)
-static int batch_vector_width(const bfvm_ctx* ctx, int axis)
-{
-	const int S = ctx->mesh.S;
-	const int64_t XS = (int64_t)ctx->mesh.grid[0] * S;
-	const int64_t unit = axis == 0 ? S : (axis == 1 ? XS : (int64_t)ctx->mesh.grid[1] * XS);
-	return unit % 4 == 0 ? 4 : 1;
-}
-
-void prepare_batch_sweep(bfvm_batch* b, int axis)
-{
-	auto& ax = b->axes[axis];
-	std::vector<part_args> args[2];
-	std::vector<batch_item> items[2];
-	for (auto& a : args)
-		a.assign(b->ctx.size(), part_args {});
-	for (size_t i = 0; i < b->ctx.size(); i++)
-	{
-		bfvm_ctx* ctx = b->ctx[i];
-		if (axis >= ctx->mesh.dims)
-			continue;
-		const int n = ctx->mesh.grid[axis];
-		if (n == 1)
-		{
-			ax.single.push_back((int)i);
-			continue;
-		}
-		const int S = ctx->mesh.S;
-		const int V = batch_vector_width(ctx, axis);
-		const int w = V == 4 ? 0 : 1;
-		const int max_threads = V == 1 ? batch_max_threads : 512;
-		partition p = choose_partition(ctx, axis, batch_chunk, 1, 1);
-		if (p.chunk != batch_chunk)
-			throw std::runtime_error("batched sweep: instance " + std::to_string(i) +
-									 " does not fit 16-element register blocks (axis too long)");
-		p.vec = V;
-		const int SG = axis == 0 ? S / V : 1;
-		const int target = b->tuning.group_threads[axis][w];
-		const int request = axis == 0 ? std::max(1, target / (SG * p.P)) : std::max(8, target / p.P / 8 * 8);
-		group_shape(axis, SG, p.P, request, max_threads, p.lpg, p.threads);
-		if (p.threads > max_threads)
-			throw std::runtime_error("batched sweep: instance " + std::to_string(i) +
-									 " does not fit one workgroup (axis too long)");
-		float *coef = nullptr, *red = nullptr, *A = nullptr;
-		alloc_partition_tables(p, S, coef, red, A);
-		ax.tables.push_back(coef);
-		ax.tables.push_back(red);
-		ax.tables.push_back(A);
-		launch_partition_tables(ctx, axis, p, coef, red, A, b->stream);
-		sweep_geometry g = geometry(ctx);
-		g.rounding = b->rounding;
-		args[w][i] = make_part_args(axis, g, p, coef, red, A);
-		auto& part = ax.parts[w];
-		part.lds = std::max(part.lds, partition_lds_bytes(p, S, p.lpg, V > 1 && axis != 0));
-		part.threads = std::max(part.threads, p.threads);
-		const int64_t per_group = (int64_t)p.lpg * n * V;
-		const int64_t per_item = std::max<int64_t>(1, 65536 / per_group);
-		for (int64_t g0 = 0; g0 < args[w][i].groups; g0 += per_item)
-			items[w].push_back(batch_item { (int32_t)i, 0, g0, std::min(args[w][i].groups, g0 + per_item) });
-		ax.any = true;
-	}
-	for (int w = 0; w < 2; w++)
-	{
-		auto& part = ax.parts[w];
-		if (items[w].empty())
-			continue;
-		if (part.lds > 64 * 1024)
-			throw std::runtime_error("batched sweep: coefficient tables exceed 64 KB of LDS");
-		BFVM_HIP(hipMalloc(&part.inst, sizeof(part_args) * args[w].size()));
-		BFVM_HIP(hipMemcpy(part.inst, args[w].data(), sizeof(part_args) * args[w].size(), hipMemcpyHostToDevice));
-		BFVM_HIP(hipMalloc(&part.items, sizeof(batch_item) * items[w].size()));
-		BFVM_HIP(hipMemcpy(part.items, items[w].data(), sizeof(batch_item) * items[w].size(), hipMemcpyHostToDevice));
-		part.nitems = (int)items[w].size();
-		part.blocks = std::min(part.nitems, b->tuning.max_blocks[axis][w]);
-	}
-}
-
-template <int AXIS, int K>
-static void launch_batched_t(bfvm_batch* b)
-{
-	const auto& ax = b->axes[AXIS];
-	const auto& p4 = ax.parts[0];
-	const auto& p1 = ax.parts[1];
-	if (p4.nitems)
-		hipLaunchKernelGGL((sweep_batched_kernel<AXIS, K, 4>), dim3(p4.blocks), dim3(p4.threads), p4.lds, b->stream,
-						   (const part_args*)p4.inst, p4.items, p4.nitems);
-	if (p1.nitems)
-		hipLaunchKernelGGL((sweep_batched_kernel<AXIS, K, 1>), dim3(p1.blocks), dim3(p1.threads), p1.lds, b->stream,
-						   (const part_args*)p1.inst, p1.items, p1.nitems);
-	BFVM_HIP(hipGetLastError());
-}
-
-void launch_batched_sweep(bfvm_batch* b, int axis)
-{
-	if (!b->axes[axis].any)
-		return;
-	by_storage(b->storage, [&](auto kind) {
-		constexpr int K = decltype(kind)::value;
-		if (axis == 0)
-			launch_batched_t<0, K>(b);
-		else if (axis == 1)
-			launch_batched_t<1, K>(b);
-		else
-			launch_batched_t<2, K>(b);
-	});
 }
 
 } // namespace bfvm

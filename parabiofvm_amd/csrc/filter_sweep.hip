@@ -136,11 +136,16 @@ __device__ __forceinline__ int fresh_lane_value(int x)
 	asm volatile("" : "+v"(x));
 	return x;
 }
-template <typename T>
-__device__ __forceinline__ T fresh_uniform(T x)
+__device__ __forceinline__ int fresh_uniform(int x)
 {
+	x = __builtin_amdgcn_readfirstlane(x);
 	asm volatile("" : "+s"(x));
 	return x;
+}
+__device__ __forceinline__ int64_t fresh_uniform(int64_t x)
+{
+	const uint32_t lo = (uint32_t)fresh_uniform((int)(uint32_t)x), hi = (uint32_t)fresh_uniform((int)(x >> 32));
+	return (int64_t)((uint64_t)hi << 32 | lo);
 }
 
 // Where a lane's block stands: block k = 0..last of its line, index i = 0..kw-1 among the blocks of its wave (`dist`
@@ -327,6 +332,29 @@ struct unaligned4
 	using type = typename store_of<K>::elem __attribute__((ext_vector_type(4), aligned(sizeof(typename store_of<K>::elem))));
 };
 
+// The last n = 1, 2 or 3 (uniform) of 4 components, in one store
+template <int K>
+__device__ __forceinline__ void store_last(typename store_of<K>::elem* p, typename unaligned4<K>::type y, int n)
+{
+	using elem = typename store_of<K>::elem;
+	using e2 = elem __attribute__((ext_vector_type(2), aligned(sizeof(elem))));
+	using e3 = elem __attribute__((ext_vector_type(3), aligned(sizeof(elem))));
+	if (n == 1)
+		gstore(p + 3, (elem)y[3]);
+	else if (n == 2)
+		gstore((e2*)(p + 2), e2 { y[2], y[3] });
+	else
+	{
+		if constexpr (K == store_f32)
+			*(__attribute__((address_space(1))) e3*)(p + 1) = e3 { y[1], y[2], y[3] };
+		else
+		{
+			gstore(p + 1, (elem)y[1]);
+			gstore((e2*)(p + 2), e2 { y[2], y[3] });
+		}
+	}
+}
+
 // ---- one lane per (column of 4 consecutive elements, block) --------------------------------------------------------
 //
 // y, z: a task is C neighbouring columns: C lanes read one contiguous segment, and the 64 / C blocks of a wave the
@@ -417,6 +445,7 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 	elem* o = (elem*)a.data + off;
 	asm volatile("" : "+v"(o));
 	uint32_t h = K == store_f32 ? 0u : sr_seed(off, rounding_key(a.rounding, 1 + a.axis));
+	const int part = fresh_uniform((int)(a.row_elems & 3)); // components that a moved-back column owns
 	filter_line<M, FULL, 4>(v, row, mk, a.blocks, at, sh, [&](int j, vec x) {
 		uv y;
 		if constexpr (K == store_f32)
@@ -440,12 +469,7 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 				gstore((uv*)(o + j * stride), y);
 		}
 		else
-		{
-#pragma unroll
-			for (int c = 1; c < 4; c++)
-				if (c >= back)
-					gstore(o + j * stride + c, (elem)y[c]);
-		}
+			store_last<K>(o + j * stride, y, part);
 	});
 
 	// Dirichlet faces, written over the solved values in the order x-, x+, y-, y+, z-, z+
@@ -474,8 +498,11 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 					}
 				continue;
 			}
-			for (int c = back; c < 4; c++)
+#pragma unroll
+			for (int c = 0; c < 4; c++)
 			{
+				if (c < back)
+					continue;
 				// coordinate d of this component's voxel (its components may lie in different voxels)
 				// x: outer = z*Y + y; y: outer = z, vc = x; z: vc = y*X + x
 				const uint32_t vc = fdivu(q + c, a.s_mul, a.s_shift);
@@ -791,7 +818,11 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 	};
 	// a line's last block holds at least half its length (sure)
 	auto fits = [&](int m) { return n - ((n + m - 1) / m - 1) * m >= m / 2; };
-	if (axis == 0 && S % 4 != 0)
+	// x rows of a substrate count that 4 does not divide: through LDS below 6 substrates, where most of a direct
+	// column of 4 overlaps its neighbour (staged / direct, us: 160^3 x 5 FP32 37 / 59, FP16 44 / 65; 131x97x143 x 5
+	// FP32 21 / 30), direct from 6 on (160^3 x 6 FP32 67 / 59, FP16 80 / 65; x 11 111 / 82, 137 / 97; x 15 121 / 96,
+	// 153 / 110; x 9 and x 10 in FP32 alone run 5 % faster staged)
+	if (axis == 0 && S % 4 != 0 && S < 6)
 	{
 		const int L = S;
 		const int64_t rows = (int64_t)g.grid[1] * g.grid[2];
