@@ -368,10 +368,13 @@ __device__ __forceinline__ void store_last(typename store_of<K>::elem* p, typena
 // took 24 against 13 us on 100^3 x 4, 89 against 75 us on 200^3 x 8, 890 against 850 us on 400^3 x 8, and in FP16 746
 // against 576 us.
 //
+// BACK: a range that 4 does not divide, with its own kernels, as the stores of parts of a column cost the others
+// registers (FP16, 16 elements: 153 -> 196, 400^3 x 8 x sweep 0.56 -> 0.78 ms).
+//
 // NT: densities that exceed the 256 MB Infinity Cache are streamed past it on y and z.  400^3 x 8, whole diffusion
 // solve: FP32 2.96 -> 2.65 ms, FP16 1.90 -> 1.85 ms; along x, whose lines are hit several times, it costs twice the
 // time.
-template <int M, bool FULL, int K, bool NT>
+template <int M, bool FULL, int K, bool NT, bool BACK>
 __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_t task, float* lt,
 													typename vec_of<4>::type* sh, bool first)
 {
@@ -395,7 +398,8 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 	const uint32_t cl = at.active ? col : 0;
 	const uint32_t outer = fdivu(cl, a.row_mul, a.row_shift);
 	const uint32_t q0 = (cl - outer * a.row_columns) * 4;
-	const int back = max(0, (int)(q0 + 4 - (uint32_t)a.row_elems)); // components owned by the column before
+	// components owned by the column before
+	const int back = BACK ? max(0, (int)(q0 + 4 - (uint32_t)a.row_elems)) : 0;
 	const uint32_t q = q0 - back;
 	const int64_t off = outer * a.outer_stride + q + (int64_t)(k * M) * a.stride;
 	const int64_t stride = fresh_uniform(a.stride);
@@ -415,12 +419,17 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 	const elem* p = (const elem*)a.data + off;
 	constexpr int N = sure<M, FULL>();
 	uv raw[M];
-	// lanes past the columns or the line read the first column's first block, elements past a block its first one
+	// Lanes past the columns or the line read the first column's first block, elements past a block its first one.
+	// Addresses step from element to element behind the compiler's back, here and at the stores: it would hold M
+	// multiples of the stride in scalar registers, and spill them, or the loads' M addresses for the stores.
+	const elem* pj = p;
 #pragma unroll
 	for (int j = 0; j < M; j++)
 	{
-		const uv* src = (const uv*)(j < N || j < mk ? p + j * stride : p);
+		const uv* src = (const uv*)(j < N || j < mk ? pj : p);
 		raw[j] = NT ? __builtin_nontemporal_load(src) : gload(src);
+		pj += stride;
+		asm volatile("" : "+v"(pj));
 	}
 	if (first)
 	{
@@ -441,8 +450,7 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 		if (j >= N)
 			v[j] = j < mk ? v[j] : vec(0.f);
 	}
-	// an address the compiler cannot tie to the loads' (kept for the stores, those would hold 2 M registers)
-	elem* o = (elem*)a.data + off;
+	elem* o = (elem*)a.data + off + (mk - 1) * stride;
 	asm volatile("" : "+v"(o));
 	uint32_t h = K == store_f32 ? 0u : sr_seed(off, rounding_key(a.rounding, 1 + a.axis));
 	const int part = fresh_uniform((int)(a.row_elems & 3)); // components that a moved-back column owns
@@ -461,15 +469,17 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 				y[c + 1] = pr[1];
 			}
 		}
-		if (back == 0)
+		if (!BACK || back == 0)
 		{
 			if constexpr (NT)
-				__builtin_nontemporal_store(y, (uv*)(o + j * stride));
+				__builtin_nontemporal_store(y, (uv*)o);
 			else
-				gstore((uv*)(o + j * stride), y);
+				gstore((uv*)o, y);
 		}
 		else
-			store_last<K>(o + j * stride, y, part);
+			store_last<K>(o, y, part);
+		o -= stride;
+		asm volatile("" : "+v"(o));
 	});
 
 	// Dirichlet faces, written over the solved values in the order x-, x+, y-, y+, z-, z+
@@ -477,6 +487,7 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 	// whole line.  Same lane, same addresses: the later store stays.
 	if (a.fcond && at.active)
 	{
+		o += stride; // the block's first element
 		const float* ls = lt + a.table_floats;
 		auto scale = [&]() { return vec { ls[s[0]], ls[s[1]], ls[s[2]], ls[s[3]] }; };
 		for (int d = 0; d < a.dims; d++)
@@ -509,13 +520,14 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 				const uint32_t hi = fdivu(a.axis == 0 ? outer : vc, a.x_mul, a.x_shift);
 				const uint32_t lo = (a.axis == 0 ? outer : vc) - hi * (uint32_t)a.grid[a.axis == 0 ? 1 : 0];
 				const int cd = (int)(a.axis == 0 ? (d == 1 ? lo : hi) : a.axis == 1 ? (d == 0 ? vc : outer) : (d == 0 ? lo : hi));
+				const int sc = (int)(q + c - vc * (uint32_t)S);
 				for (int mx = 0; mx < 2; mx++)
 				{
-					if (cd != (mx ? a.grid[d] - 1 : 0) || !gload(a.fcond + (2 * d + mx) * S + s[c]))
+					if (cd != (mx ? a.grid[d] - 1 : 0) || !gload(a.fcond + (2 * d + mx) * S + sc))
 						continue;
-					float val = gload(a.fval + (2 * d + mx) * S + s[c]);
+					float val = gload(a.fval + (2 * d + mx) * S + sc);
 					if constexpr (K != store_f32)
-						val *= ls[s[c]];
+						val *= ls[sc];
 					for (int j = 0; j < mk; j++)
 						gstore(o + j * stride + c, (elem)val);
 				}
@@ -524,7 +536,7 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 	}
 }
 
-template <int M, bool FULL, int K, bool NT>
+template <int M, bool FULL, int K, bool NT, bool BACK>
 __global__ __launch_bounds__(512) void filter_columns_kernel(filter_args a)
 {
 	extern __shared__ raw16 filter_lds[];
@@ -535,7 +547,7 @@ __global__ __launch_bounds__(512) void filter_columns_kernel(filter_args a)
 	int parity = 0;
 	bool first = true;
 	for (int64_t t = xcd_order(blockIdx.x, gridDim.x); t < a.tasks; t += gridDim.x, parity ^= 1, first = false)
-		filter_columns_task<M, FULL, K, NT>(a, t, (float*)filter_lds, sh + parity * area, first);
+		filter_columns_task<M, FULL, K, NT, BACK>(a, t, (float*)filter_lds, sh + parity * area, first);
 }
 
 // ---- x, substrate counts that 4 does not divide: rows staged through LDS, one element per lane and position --------
@@ -978,7 +990,7 @@ void launch_filter_sweep(bfvm_ctx* ctx, int axis)
 		cap = std::min<int64_t>(cap, filter_fill_waves / p.waves);
 	const dim3 blocks((unsigned)std::min(p.tasks, cap)), threads(64 * p.waves);
 	const size_t lds = p.lds;
-	const bool full = a.mlast == a.m;
+	const bool full = a.mlast == a.m, back = a.row_elems % 4 != 0;
 	by_storage(ctx->storage, [&](auto kind) {
 		constexpr int K = decltype(kind)::value;
 		if (p.staged)
@@ -986,11 +998,12 @@ void launch_filter_sweep(bfvm_ctx* ctx, int axis)
 				hipLaunchKernelGGL((filter_rows_kernel<m, f, K>), blocks, threads, lds, ctx->stream, a);
 			});
 		else
-			by_block<2, 3, 4, 5, 7, 9, 11, 13, 14, 16, 18, 20, 22, 25>(p.m, full, [&](auto m, auto f) {
-				if (p.streamed)
-					hipLaunchKernelGGL((filter_columns_kernel<m, f, K, true>), blocks, threads, lds, ctx->stream, a);
-				else
-					hipLaunchKernelGGL((filter_columns_kernel<m, f, K, false>), blocks, threads, lds, ctx->stream, a);
+			by_block<2, 3, 4, 5, 7, 9, 11, 13, 14, 16, 18, 20, 22, 25>(p.m, full && !back, [&](auto m, auto f) {
+				auto kernel = p.streamed ? filter_columns_kernel<m, f, K, true, false> : filter_columns_kernel<m, f, K, false, false>;
+				if constexpr (!f)
+					if (back)
+						kernel = p.streamed ? filter_columns_kernel<m, f, K, true, true> : filter_columns_kernel<m, f, K, false, true>;
+				hipLaunchKernelGGL(kernel, blocks, threads, lds, ctx->stream, a);
 			});
 	});
 	BFVM_HIP(hipGetLastError());
