@@ -1393,7 +1393,6 @@ static void free_batch(bfvm_batch* b)
 			(void)hipGraphDestroy(g.graph);
 		g = graph_slot {};
 	}
-	free_batch_gradient(b);
 	free_batch_cell(b);
 	for (int i = 0; i < bfvm_batch::branches; i++)
 	{
@@ -1475,31 +1474,28 @@ static void on_branches(bfvm_batch* b, F&& one)
 		std::rethrow_exception(failed);
 }
 
-static void enqueue_batch_sweeps(bfvm_batch* b)
+static void enqueue_batch_sweeps(bfvm_batch* b, bool with_gradient = false)
 {
 	if (b->storage != BFVM_STORAGE_F32)
 	{
 		batch_override o(b->ctx[0], b, b->stream);
 		launch_advance_rounding(b->ctx[0]);
 	}
-	on_branches(b, [](bfvm_ctx* c) {
+	on_branches(b, [&](bfvm_ctx* c) {
 		enqueue_dirichlet(c);
 		for (int axis = 0; axis < c->mesh.dims; axis++)
 		{
 			launch_sweep(c, axis);
 			launch_dirichlet_interior(c);
 		}
+		if (with_gradient)
+			launch_gradient(c);
 	});
 }
 
 static void enqueue_batch_gradient(bfvm_batch* b)
 {
-	launch_batched_gradient(b);
-	for (int i : b->grad.single)
-	{
-		batch_override o(b->ctx[i], b, b->stream);
-		launch_gradient(b->ctx[i]);
-	}
+	on_branches(b, [](bfvm_ctx* c) { launch_gradient(c); });
 }
 
 // the secretion of every instance: batched launches when the plan allows, else instance by instance
@@ -1520,9 +1516,7 @@ static void enqueue_batch_cell(bfvm_batch* b, bool recompute)
 static void enqueue_batch_step(bfvm_batch* b, bool recompute, bool with_gradient)
 {
 	enqueue_batch_cell(b, recompute);
-	enqueue_batch_sweeps(b);
-	if (with_gradient)
-		enqueue_batch_gradient(b);
+	enqueue_batch_sweeps(b, with_gradient);
 }
 
 } // namespace bfvm
@@ -1588,7 +1582,6 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 				b->branch_of[i] = at;
 				load[at] += size(i);
 			}
-			prepare_batch_gradient(b);
 			BFVM_HIP(hipStreamSynchronize(b->stream));
 		}
 		catch (...)
@@ -1670,54 +1663,14 @@ int bfvm_batch_autotune(bfvm_batch* batch)
 		BFVM_HIP(hipSetDevice(batch->device));
 		join_instance_streams(batch);
 		BFVM_HIP(hipStreamSynchronize(batch->stream));
-		if (apply_cached_batch_tuning(batch))
+		// the instances' launches are shaped by rules and by each context's own tuning: there is nothing to time
+		if (!apply_cached_batch_tuning(batch))
 		{
-			free_batch_gradient(batch);
-			prepare_batch_gradient(batch);
-			BFVM_HIP(hipStreamSynchronize(batch->stream));
-			batch->epoch++;
-			return BFVM_OK;
+			remember_batch_tuning(batch);
+			enqueue_batch_gradient(batch);
 		}
-		// the candidates run on copies of the instances' densities
-		std::vector<void*> real(batch->ctx.size(), nullptr), scratch(batch->ctx.size(), nullptr);
-		auto restore = [&]() {
-			for (size_t i = 0; i < batch->ctx.size(); i++)
-				if (real[i])
-					batch->ctx[i]->dens = real[i];
-			(void)hipStreamSynchronize(batch->stream);
-			for (void* p : scratch)
-				if (p)
-					(void)hipFree(p);
-		};
-		try
-		{
-			for (size_t i = 0; i < batch->ctx.size(); i++)
-			{
-				bfvm_ctx* c = batch->ctx[i];
-				const size_t bytes = c->mesh.V * c->mesh.S * storage_bytes(c->storage);
-				BFVM_HIP(hipMalloc(&scratch[i], bytes));
-				BFVM_HIP(hipMemcpyAsync(scratch[i], c->dens, bytes, hipMemcpyDeviceToDevice, batch->stream));
-				real[i] = c->dens;
-				c->dens = scratch[i];
-			}
-			autotune_batch(batch);
-		}
-		catch (...)
-		{
-			restore();
-			free_batch_gradient(batch);
-			prepare_batch_gradient(batch);
-			throw;
-		}
-		restore();
-		// the plans hold the instances' buffers: rebuild them on the real densities, recompute the gradients the
-		// timings overwrote, and let the secretion plan refresh
-		free_batch_gradient(batch);
-		prepare_batch_gradient(batch);
-		enqueue_batch_gradient(batch);
 		BFVM_HIP(hipStreamSynchronize(batch->stream));
 		batch->epoch++;
-		batch->cell.epoch = ~0ull;
 		return BFVM_OK;
 	});
 }
@@ -1780,7 +1733,7 @@ int bfvm_batch_benchmark(bfvm_batch* batch, int32_t what, int32_t iterations, fl
 				});
 				break;
 			case BFVM_KERNEL_GRADIENT:
-				launch_batched_gradient(batch);
+				enqueue_batch_gradient(batch);
 				break;
 			case BFVM_PHASE_SECRETION:
 			case BFVM_PHASE_SECRETION_RECOMPUTE:

@@ -2,9 +2,8 @@
 // CUDA/diffusion_solver.cpp:11, 256-thread blocks in CUDA/diffusion_solver.cu:947-987); here the shapes of
 // every sweep axis (register chunk, lines per workgroup, workgroup count) and of the gradient (workgroups it
 // aims for) are picked by timing candidates on the context's own mesh, and cached per (axis, mesh shape,
-// substrate count, storage) for the process, so that contexts of the same shape tune once.  Batches tune their
-// work-list launches (group size and workgroup count per axis and thread layout, gradient tiles per work item
-// and workgroup count) the same way, cached per list of instance shapes.  The cache can be written to and read
+// substrate count, storage) for the process, so that contexts of the same shape tune once.  A batch's
+// instances keep their own shapes.  The cache can be written to and read
 // from a text file, so that a later process starts tuned.
 #include <cstdio>
 #include <map>
@@ -172,8 +171,7 @@ bool apply_cached_batch_tuning(bfvm_batch* b)
 // Text file, one entry per line:
 //   sweep <axis> <X> <Y> <Z> <S> <storage> <algorithm> <chunk> <lines> <workgroups>
 //   gradient <X> <Y> <Z> <S> <storage> <algorithm> <workgroups> <stacked> [<order>]
-//   batch <key> <12 numbers, kept but not used> <gradient tiles> <gradient blocks> <gradient rows>
-//         <gradient z planes> <gradient split> <gradient stacked>
+//   batch <key> <18 numbers, kept but not used>
 void save_tuning(const char* path)
 {
 	std::lock_guard<std::mutex> lock(g_cache_mutex);
@@ -189,10 +187,9 @@ void save_tuning(const char* path)
 	for (const auto& [k, t] : g_batch_cache)
 	{
 		std::fprintf(f, "batch %s", k.c_str());
-		for (int v : t.sweep_fields)
+		for (int v : t.fields)
 			std::fprintf(f, " %d", v);
-		std::fprintf(f, " %d %d %d %d %d %d\n", t.gradient_tiles, t.gradient_blocks, t.gradient_rows, t.gradient_zchunk,
-					 t.gradient_split, t.gradient_stacked);
+		std::fprintf(f, "\n");
 	}
 	const bool bad = std::ferror(f) != 0;
 	std::fclose(f);
@@ -247,11 +244,9 @@ void load_tuning(const char* path)
 			std::string key;
 			bfvm_batch::tuning_t t;
 			ok = static_cast<bool>(in >> key);
-			for (int i = 0; i < 12 && ok; i++)
-				ok = static_cast<bool>(in >> t.sweep_fields[i]);
-			ok = ok && static_cast<bool>(in >> t.gradient_tiles >> t.gradient_blocks >> t.gradient_rows >>
-										  t.gradient_zchunk >> t.gradient_split >> t.gradient_stacked) &&
-				 (t.gradient_rows == 4 || t.gradient_rows == 8);
+			for (int i = 0; i < 18 && ok; i++)
+				ok = static_cast<bool>(in >> t.fields[i]);
+			ok = ok && (t.fields[14] == 4 || t.fields[14] == 8);
 			if (ok)
 				g_batch_cache[key] = t;
 		}
@@ -305,20 +300,22 @@ void autotune_context(bfvm_ctx* ctx, bool tune_gradient)
 		if (!cached)
 		{
 			float best_t = 1e30f;
+			auto consider = [&](const gradient_shape& shape) {
+				ctx->gradient_groups = shape.groups;
+				ctx->gradient_stacked = shape.stacked;
+				ctx->gradient_order = shape.order;
+				const float t = best_ms(ctx->stream, reps, [&] { launch_gradient(ctx); });
+				if (t < best_t * 0.99f)
+				{
+					best_t = t;
+					best = shape;
+				}
+			};
+			consider(gradient_shape {}); // the automatic shape
 			for (int order : { 0, 1 })
 				for (bool stacked : { false, true })
-					for (int g : { 2048, 4096, 8192, 16384, 32768, 65536 })
-					{
-						ctx->gradient_groups = g;
-						ctx->gradient_stacked = stacked;
-						ctx->gradient_order = order;
-						const float t = best_ms(ctx->stream, reps, [&] { launch_gradient(ctx); });
-						if (t < best_t)
-						{
-							best_t = t;
-							best = gradient_shape { g, stacked, order };
-						}
-					}
+					for (int g : { 4096, 8192, 16384, 32768, 65536 })
+						consider(gradient_shape { g, stacked, order });
 			std::lock_guard<std::mutex> lock(g_cache_mutex);
 			g_gradient_cache[key] = best;
 		}
@@ -330,65 +327,8 @@ void autotune_context(bfvm_ctx* ctx, bool tune_gradient)
 	ctx->epoch++;
 }
 
-// Batches: the tiles per work item and the workgroup cap of the gradient, each candidate rebuilding the plan.
-void autotune_batch(bfvm_batch* b)
+void remember_batch_tuning(bfvm_batch* b)
 {
-	const int reps = 3;
-	if (b->grad.nitems[2] > 0)
-	{
-		// tile shape first (rows per thread, z planes per tile), then the work distribution
-		int best_rows = b->tuning.gradient_rows, best_zc = b->tuning.gradient_zchunk;
-		int best_split = b->tuning.gradient_split, best_stacked = b->tuning.gradient_stacked;
-		float best_shape = 1e30f;
-		for (int stacked = 0; stacked < 2; stacked++)
-			for (int split = 0; split < (b->storage == BFVM_STORAGE_F32 ? 2 : 1); split++)
-				for (int rows : { 4, 8 })
-					for (int zc : { 16, 32, 64 })
-					{
-						b->tuning.gradient_stacked = stacked;
-						b->tuning.gradient_split = split;
-						b->tuning.gradient_rows = rows;
-						b->tuning.gradient_zchunk = zc;
-						free_batch_gradient(b);
-						prepare_batch_gradient(b);
-						const float t = best_ms(b->stream, reps, [&] { launch_batched_gradient(b); });
-						if (t < best_shape)
-						{
-							best_shape = t;
-							best_rows = rows;
-							best_zc = zc;
-							best_split = split;
-							best_stacked = stacked;
-						}
-					}
-		b->tuning.gradient_stacked = best_stacked;
-		b->tuning.gradient_split = best_split;
-		b->tuning.gradient_rows = best_rows;
-		b->tuning.gradient_zchunk = best_zc;
-		int best_tiles = b->tuning.gradient_tiles, best_blocks = b->tuning.gradient_blocks;
-		float best_t = 1e30f;
-		for (int tiles : { 1, 2, 4, 8 })
-			for (int blocks : { 2048, 4096, 8192, 16384, 32768, 65536 })
-			{
-				b->tuning.gradient_tiles = tiles;
-				b->tuning.gradient_blocks = blocks;
-				free_batch_gradient(b);
-				prepare_batch_gradient(b);
-				const float t = best_ms(b->stream, reps, [&] { launch_batched_gradient(b); });
-				if (t < best_t)
-				{
-					best_t = t;
-					best_tiles = tiles;
-					best_blocks = blocks;
-				}
-			}
-		b->tuning.gradient_tiles = best_tiles;
-		b->tuning.gradient_blocks = best_blocks;
-		free_batch_gradient(b);
-		prepare_batch_gradient(b);
-	}
-	BFVM_HIP(hipStreamSynchronize(b->stream));
-	b->epoch++;
 	std::lock_guard<std::mutex> lock(g_cache_mutex);
 	g_batch_cache[batch_key(b)] = b->tuning;
 }

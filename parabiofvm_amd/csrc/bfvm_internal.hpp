@@ -388,7 +388,7 @@ struct mesh_info
 };
 
 // Work-list item of the batched (many microenvironment) kernels: a range of workgroup-sized units
-// (sweep line groups or gradient tiles) of one instance.
+// (agents' blocks) of one instance.
 struct batch_item
 {
 	int32_t instance;
@@ -474,8 +474,8 @@ struct bfvm_ctx
 	int chunk_request[3] = { 0, 0, 0 };
 	int lines_request[3] = { 0, 0, 0 };
 	int gradient_groups = 0; // workgroups the 3-D gradient aims for (0 = automatic)
-	bool gradient_stacked = false; // 3-D gradient tiles with the workgroup's waves stacked along y
-	int gradient_order = 0; // 3-D gradient workgroup order: 0 = z chunks of a row band per XCD, 1 = plane order
+	bool gradient_stacked = false; // 3-D gradient with 8 rows per thread instead of 4
+	int gradient_order = 0; // 3-D gradient workgroup order: 0 = consecutive tiles per XCD, 1 = plane order
 	int sweep_workgroups[3] = { 0, 0, 0 }; // most workgroups of a sweep launch per axis (0 = the built-in cap)
 
 	bfvm::agents_buffers ag;
@@ -493,8 +493,8 @@ struct bfvm_ctx
 	bool stream_used = false;
 };
 
-// Many microenvironments advanced together (bfvm_batch_*): the instances' sweeps on parallel branches of one graph,
-// one launch for the gradient over all instances, driven by device work lists.
+// Many microenvironments advanced together (bfvm_batch_*): the instances' sweeps and gradients on parallel
+// branches of one graph.
 struct bfvm_batch
 {
 	int device = 0;
@@ -503,22 +503,13 @@ struct bfvm_batch
 	std::vector<uint64_t> generation; // each instance's initialization when the batch was made
 	int storage = BFVM_STORAGE_F32;
 	unsigned* rounding = nullptr; // step counter of the stochastic rounding, shared by all instances
-	// The instances' sweeps run as chains (x, y, z of one instance after the other), spread over branches that run side
+	// The instances' sweeps and gradients run as chains (x, y, z, gradient of one instance after the other), spread over branches that run side
 	// by side: a chain's densities stay in the caches between its sweeps, and a small instance's latency hides behind
 	// the other branches.
 	static constexpr int branches = 4;
 	hipStream_t branch_stream[branches] = {}; // [0] is `stream`
 	hipEvent_t branch_event[branches] = {};   // [0]: the fork
 	std::vector<int> branch_of;				 // per instance
-	struct gradient_plan
-	{
-		void* inst = nullptr; // device gradient_args per instance
-		// work items per thread layout: one element, 4 substrates of a voxel, and all of them
-		bfvm::batch_item* items[3] = { nullptr, nullptr, nullptr };
-		int nitems[3] = { 0, 0, 0 };
-		int blocks[3] = { 0, 0, 0 };
-		std::vector<int> single; // instances of fewer than 3 dimensions (per-instance launch)
-	} grad;
 	// batched secretion: per-instance arguments and work items over (agent, substrate) and agent blocks, rebuilt
 	// when an instance's agents change (cell_epoch); per-instance launches when an instance uses the sorted
 	// reduction
@@ -532,17 +523,10 @@ struct bfvm_batch
 		bool batched = false;
 		uint64_t epoch = ~0ull;
 	} cell;
-	// launch shapes of the work-list gradient (bfvm_batch_autotune picks them): the y rows per thread, the z planes per
-	// tile, the tiles per work item and the workgroup cap
+	// the numbers of a batch's entry in a tuning file: kept, not used (the instances' own shapes apply)
 	struct tuning_t
 	{
-		int sweep_fields[12] = { 256, 256, 256, 256, 256, 256, 2048, 2048, 2048, 2048, 2048, 2048 }; // of tuning files
-		int gradient_tiles = 4;
-		int gradient_blocks = 8192;
-		int gradient_rows = 4;	  // y rows per thread (4 or 8)
-		int gradient_zchunk = 16; // z planes per gradient tile
-		int gradient_split = 0;	  // FP32: one gradient launch per thread layout instead of one for both
-		int gradient_stacked = 0; // tiles with the workgroup's waves stacked along y
+		int fields[18] = { 256, 256, 256, 256, 256, 256, 2048, 2048, 2048, 2048, 2048, 2048, 4, 8192, 4, 16, 0, 0 };
 	} tuning;
 	uint64_t epoch = 0;
 	bfvm::graph_slot graphs[4];
@@ -589,11 +573,6 @@ void fast_divisor(uint32_t d, uint32_t& mul, int& shift);
 int supported_chunk(int request);
 partition choose_partition(const bfvm_ctx* ctx, int axis, int chunk, int lines_request, int max_vec);
 
-// batched kernels (bfvm_batch): plans are built once at bfvm_batch_create; launches enqueue on b->stream
-void prepare_batch_gradient(bfvm_batch* b);
-void launch_batched_gradient(bfvm_batch* b);
-void free_batch_gradient(bfvm_batch* b);
-
 // entry point without allocation: the file-scope device scratch of noalloc.hip, looked up per device
 constexpr int noalloc_max_points = 1 << 20;
 void setup_noalloc_scratch(int device); // with `device` current, once per device (bfvm_create)
@@ -601,7 +580,7 @@ void voxel_positions_noalloc(bfvm_ctx* ctx, int count, const float* positions, i
 
 // autotuner: time candidate launch shapes on the context's mesh / the batch and keep the fastest
 void autotune_context(bfvm_ctx* ctx, bool tune_gradient);
-void autotune_batch(bfvm_batch* b);
+void remember_batch_tuning(bfvm_batch* b);
 bool apply_cached_batch_tuning(bfvm_batch* b); // false when this list of instance shapes has no cached tuning
 void save_tuning(const char* path);
 void load_tuning(const char* path);
