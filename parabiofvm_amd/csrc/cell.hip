@@ -17,6 +17,8 @@
 //
 // Agents whose position maps outside the grid (or is not finite) get voxel -1 and are ignored; the
 // reference would index out of bounds (src/mesh.cpp:47-53 does not clamp).
+#include <algorithm>
+
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "bfvm_internal.hpp"
@@ -56,63 +58,41 @@ __global__ __launch_bounds__(256) void cell_voxels_kernel(cell_geom g, int A, co
 		vox[i] = agent_voxel(g, pos, i);
 }
 
-// recompute, part 1 (host/cell_solver.cpp:35-85): intermediates and reduced-slot reset per (agent, s);
-// ballot reset per agent.
-__device__ __forceinline__ void cell_prepare_at(int64_t k, int A, int S, float voxel_volume, float dt,
-														   const int64_t* __restrict__ vox,
-														   const float* __restrict__ vol, const float* __restrict__ sec,
-														   const float* __restrict__ sat, const float* __restrict__ upt,
-														   const float* __restrict__ nex, float* __restrict__ num,
-														   float* __restrict__ den, float* __restrict__ fac,
-														   float* __restrict__ rnum, float* __restrict__ rden,
-														   float* __restrict__ rfac, int* __restrict__ ballots,
-														   int* __restrict__ conflict)
+// Recompute, claim scheme: reset, ballot, prepare, sum.  1M clustered agents x 8 substrates on 200^3, all phases with
+// the apply: 405 -> 276 us.  Winners are known before the terms are formed, so a winner's slot starts with its own
+// terms and only the other agents add with atomics (sum 120 -> 72 us).
+//
+// part 1: ballots of the agents' voxels back to unclaimed, no conflict yet
+__device__ __forceinline__ void cell_reset_at(int64_t i, int A, const int64_t* __restrict__ vox,
+											  int* __restrict__ ballots, int* __restrict__ conflict)
 {
-	if (k == 0)
+	if (i == 0)
 		atomicExch(conflict, 0);
-	if (k >= (int64_t)A * S)
+	if (i >= A)
 		return;
-	const int64_t i = k / S;
-	const int s = (int)(k - i * S);
-	if (s == 0)
-	{
-		const int64_t v = vox[i];
-		if (v >= 0)
-			ballots[v] = -1;
-	}
-	const float cv = vol[i];
-	num[k] = sec[k] * sat[k] * dt * cv / voxel_volume;
-	den[k] = (upt[k] + sec[k]) * dt * cv / voxel_volume;
-	fac[k] = nex[k] * dt / voxel_volume;
-	rnum[k] = 0;
-	rden[k] = 0;
-	rfac[k] = 0;
+	const int64_t v = vox[i];
+	if (v >= 0)
+		ballots[v] = -1;
 }
 
-__global__ __launch_bounds__(256) void cell_prepare_kernel(int A, int S, float voxel_volume, float dt,
-														   const int64_t* __restrict__ vox,
-														   const float* __restrict__ vol, const float* __restrict__ sec,
-														   const float* __restrict__ sat, const float* __restrict__ upt,
-														   const float* __restrict__ nex, float* __restrict__ num,
-														   float* __restrict__ den, float* __restrict__ fac,
-														   float* __restrict__ rnum, float* __restrict__ rden,
-														   float* __restrict__ rfac, int* __restrict__ ballots,
-														   int* __restrict__ conflict)
+__global__ __launch_bounds__(256) void cell_reset_kernel(int A, const int64_t* __restrict__ vox,
+														 int* __restrict__ ballots, int* __restrict__ conflict)
 {
-	cell_prepare_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, S, voxel_volume, dt, vox, vol, sec, sat, upt,
-					nex, num, den, fac, rnum, rden, rfac, ballots, conflict);
+	cell_reset_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, vox, ballots, conflict);
 }
 
-// *flag = 1 when `cond` holds for an active lane of the wave: one atomic per wave (by the lowest such lane)
-// instead of one per lane, as atomics to one address are serialised
+// *flag = 1 when `cond` holds for an active lane of the wave: at most one store per wave, and none once the wave sees
+// the flag set.  Accesses to one address are serialised: with an atomic from every wave, 1M crowded agents took 192 us
+// for their claims, now 102 us.
 __device__ __forceinline__ void flag_any(int* flag, bool cond)
 {
 	const unsigned long long m = __ballot(cond);
-	if (cond && (unsigned)__lane_id() == (unsigned)(__ffsll((long long)m) - 1))
-		atomicOr(flag, 1);
+	if (cond && (unsigned)__lane_id() == (unsigned)(__ffsll((long long)m) - 1) &&
+		__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+		__hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// recompute, part 2 (host/cell_solver.cpp:98-122): claim the voxel; win[i] = the agent whose slot collects i
+// part 2 (host/cell_solver.cpp:98-122): claim the voxel; win[i] = the agent whose slot collects i
 __device__ __forceinline__ void cell_ballot_at(int64_t i, int A, const int64_t* __restrict__ vox,
 														  int* __restrict__ ballots, int* __restrict__ win,
 														  int* __restrict__ conflict)
@@ -125,6 +105,7 @@ __device__ __forceinline__ void cell_ballot_at(int64_t i, int A, const int64_t* 
 		win[i] = -1;
 		return;
 	}
+	// (loading the ballot first and claiming only unclaimed voxels: 102 -> 151 us for 1M crowded agents)
 	const int prev = atomicCAS(&ballots[v], -1, (int)i);
 	win[i] = prev == -1 ? (int)i : prev;
 	flag_any(conflict, prev != -1);
@@ -137,8 +118,59 @@ __global__ __launch_bounds__(256) void cell_ballot_kernel(int A, const int64_t* 
 	cell_ballot_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, vox, ballots, win, conflict);
 }
 
-// recompute, part 3 (host/cell_solver.cpp:108-133): every (agent, s) adds into its winner's slot; the
-// winner adds den + 1.
+// The terms of one agent and substrate (host/cell_solver.cpp:35-85)
+struct cell_terms
+{
+	float num, den, fac;
+};
+__device__ __forceinline__ cell_terms make_terms(int64_t i, int64_t k, float voxel_volume, float dt,
+												 const float* __restrict__ vol, const float* __restrict__ sec,
+												 const float* __restrict__ sat, const float* __restrict__ upt,
+												 const float* __restrict__ nex)
+{
+	const float cv = vol[i];
+	return { sec[k] * sat[k] * dt * cv / voxel_volume, (upt[k] + sec[k]) * dt * cv / voxel_volume,
+			 nex[k] * dt / voxel_volume };
+}
+
+// part 3 (host/cell_solver.cpp:35-85): the terms per (agent, s), and the reduced slot: a winner's own terms, with
+// den + 1, else 0
+__device__ __forceinline__ void cell_prepare_at(int64_t k, int A, int S, float voxel_volume, float dt,
+														   const int* __restrict__ win,
+														   const float* __restrict__ vol, const float* __restrict__ sec,
+														   const float* __restrict__ sat, const float* __restrict__ upt,
+														   const float* __restrict__ nex, float* __restrict__ num,
+														   float* __restrict__ den, float* __restrict__ fac,
+														   float* __restrict__ rnum, float* __restrict__ rden,
+														   float* __restrict__ rfac)
+{
+	if (k >= (int64_t)A * S)
+		return;
+	const int64_t i = k / S;
+	const cell_terms t = make_terms(i, k, voxel_volume, dt, vol, sec, sat, upt, nex);
+	const bool won = win[i] == (int)i;
+	num[k] = t.num;
+	den[k] = t.den;
+	fac[k] = t.fac;
+	rnum[k] = won ? t.num : 0.f;
+	rden[k] = won ? t.den + 1 : 0.f;
+	rfac[k] = won ? t.fac : 0.f;
+}
+
+__global__ __launch_bounds__(256) void cell_prepare_kernel(int A, int S, float voxel_volume, float dt,
+														   const int* __restrict__ win,
+														   const float* __restrict__ vol, const float* __restrict__ sec,
+														   const float* __restrict__ sat, const float* __restrict__ upt,
+														   const float* __restrict__ nex, float* __restrict__ num,
+														   float* __restrict__ den, float* __restrict__ fac,
+														   float* __restrict__ rnum, float* __restrict__ rden,
+														   float* __restrict__ rfac)
+{
+	cell_prepare_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, S, voxel_volume, dt, win, vol, sec, sat, upt,
+					nex, num, den, fac, rnum, rden, rfac);
+}
+
+// part 4 (host/cell_solver.cpp:108-133): every other (agent, s) adds into its winner's slot
 __device__ __forceinline__ void cell_sum_at(int64_t k, int A, int S, const int* __restrict__ win,
 													   const float* __restrict__ num, const float* __restrict__ den,
 													   const float* __restrict__ fac, float* __restrict__ rnum,
@@ -149,11 +181,11 @@ __device__ __forceinline__ void cell_sum_at(int64_t k, int A, int S, const int* 
 	const int64_t i = k / S;
 	const int s = (int)(k - i * S);
 	const int w = win[i];
-	if (w < 0)
+	if (w < 0 || w == (int)i)
 		return;
 	const int64_t t = (int64_t)w * S + s;
 	atomicAdd(&rnum[t], num[k]);
-	atomicAdd(&rden[t], w == (int)i ? den[k] + 1 : den[k]);
+	atomicAdd(&rden[t], den[k]);
 	atomicAdd(&rfac[t], fac[k]);
 }
 
@@ -205,63 +237,73 @@ __global__ __launch_bounds__(256) void cell_runs_kernel(int A, uint64_t V, const
 		atomicOr(multi, 1);
 }
 
-// recompute with the sorted order, part 1: the terms gathered into voxel order, one thread per (sorted
-// position, s) with one dependent load each, so that the run sums read consecutive memory.  (Summing the runs
-// straight from agent order made every step of a run head's loop wait for an index load and then a gather:
-// 19.8 ms for 1e7 clustered agents x 16 substrates.)
-__global__ __launch_bounds__(256) void cell_sorted_gather_kernel(int A, int S, uint64_t V,
-																 const uint64_t* __restrict__ keys,
-																 const int* __restrict__ idx,
-																 const float* __restrict__ num,
-																 const float* __restrict__ den,
-																 const float* __restrict__ fac,
-																 float* __restrict__ snum, float* __restrict__ sden,
-																 float* __restrict__ sfac)
+// recompute with the sorted order, part 1, one thread per (sorted position, s): the terms, each agent's in its own
+// place, and, where a voxel has several agents, also in voxel order, so that the run sums read consecutive memory.
+// (Summing the runs straight from agent order made every step of a run head's loop wait for an index load and then a
+// gather: 19.8 ms for 1e7 clustered agents x 16 substrates.)  An agent alone in its voxel has its reduced slot here.
+// Terms, their copy into voxel order and the run sums took 127 + 127 + 151 us as three passes over 1M agents x 16
+// substrates, now 231 + 85 us.
+__global__ __launch_bounds__(256) void cell_sorted_prepare_kernel(
+	int A, int S, uint64_t V, float voxel_volume, float dt, const uint64_t* __restrict__ keys,
+	const int* __restrict__ idx, const float* __restrict__ vol, const float* __restrict__ sec,
+	const float* __restrict__ sat, const float* __restrict__ upt, const float* __restrict__ nex,
+	float* __restrict__ num, float* __restrict__ den, float* __restrict__ fac, float* __restrict__ snum,
+	float* __restrict__ sden, float* __restrict__ sfac, float* __restrict__ rnum, float* __restrict__ rden,
+	float* __restrict__ rfac, int* __restrict__ ballots, const int* __restrict__ multi, int* __restrict__ conflict)
 {
 	const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+	// the voxel order is fixed at upload, and so is whether a voxel holds several agents
+	if (t == 0)
+		atomicExch(conflict, *multi ? 1 : 0);
 	if (t >= (int64_t)A * S)
 		return;
 	const int64_t p = t / S;
 	const int s = (int)(t - p * S);
-	if (keys[p] == V)
-		return;
-	const int64_t k = (int64_t)idx[p] * S + s;
-	snum[t] = num[k];
-	sden[t] = den[k];
-	sfac[t] = fac[k];
+	const int i = idx[p];
+	const int64_t k = (int64_t)i * S + s;
+	const cell_terms c = make_terms(i, k, voxel_volume, dt, vol, sec, sat, upt, nex);
+	const uint64_t key = keys[p];
+	const bool head = key != V && !(p > 0 && keys[p - 1] == key), more = p + 1 < A && keys[p + 1] == key;
+	num[k] = c.num;
+	den[k] = c.den;
+	fac[k] = c.fac;
+	if (key != V && (more || !head))
+	{
+		snum[t] = c.num;
+		sden[t] = c.den;
+		sfac[t] = c.fac;
+	}
+	if (!(head && more))
+	{
+		rnum[k] = head ? c.num : 0.f;
+		rden[k] = head ? c.den + 1 : 0.f;
+		rfac[k] = head ? c.fac : 0.f;
+	}
+	if (head && s == 0)
+		ballots[key] = i;
 }
 
-// part 2: one thread per (sorted position, s); run heads sum their run (winner first with den + 1, then the
-// run's agents in ascending index order) and write the winner's slot.
+// part 2: one thread per (sorted position, s); the heads of runs of several agents sum their run (winner first with
+// den + 1, then the run's agents in ascending index order) and write the winner's slot.
 __global__ __launch_bounds__(256) void cell_sorted_sum_kernel(int A, int S, uint64_t V,
 															  const uint64_t* __restrict__ keys,
 															  const int* __restrict__ idx,
 															  const float* __restrict__ snum,
 															  const float* __restrict__ sden,
 															  const float* __restrict__ sfac, float* __restrict__ rnum,
-															  float* __restrict__ rden, float* __restrict__ rfac,
-															  int* __restrict__ ballots, const int* __restrict__ multi,
-															  int* __restrict__ conflict)
+															  float* __restrict__ rden, float* __restrict__ rfac)
 {
 	const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-	// the voxel order is fixed at upload, and so is whether a voxel holds several agents
-	if (t == 0 && *multi)
-		atomicOr(conflict, 1);
 	if (t >= (int64_t)A * S)
 		return;
 	const int64_t p = t / S;
 	const int s = (int)(t - p * S);
 	const uint64_t key = keys[p];
-	if (key == V || (p > 0 && keys[p - 1] == key))
+	if (key == V || (p > 0 && keys[p - 1] == key) || p + 1 >= A || keys[p + 1] != key)
 		return;
-	const int w = idx[p];
-	const int64_t kw = (int64_t)w * S + s;
-	float sn = 0.f, sd = 0.f, sf = 0.f;
-	sn = sn + snum[t];
-	sd = sd + (sden[t] + 1);
-	sf = sf + sfac[t];
-	int64_t q = p + 1;
-	for (; q < A && keys[q] == key; q++)
+	const int64_t kw = (int64_t)idx[p] * S + s;
+	float sn = snum[t], sd = sden[t] + 1, sf = sfac[t];
+	for (int64_t q = p + 1; q < A && keys[q] == key; q++)
 	{
 		const int64_t k = q * S + s;
 		sn = sn + snum[k];
@@ -271,8 +313,6 @@ __global__ __launch_bounds__(256) void cell_sorted_sum_kernel(int A, int S, uint
 	rnum[kw] = sn;
 	rden[kw] = sd;
 	rfac[kw] = sf;
-	if (s == 0)
-		ballots[key] = w;
 }
 
 // Apply, part 1 (host/cell_solver.cpp:137-152, 173-195, 208-234).  One thread per (agent, substrate).
@@ -381,8 +421,9 @@ __global__ __launch_bounds__(256) void cell_densities_kernel(int A, int S, int w
 // elements, as the single-instance kernels do.
 enum cell_phase
 {
-	phase_prepare,
+	phase_reset,
 	phase_ballot,
+	phase_prepare,
 	phase_sum,
 	phase_apply,
 	phase_densities
@@ -399,11 +440,13 @@ __global__ __launch_bounds__(256) void cell_batched_kernel(const cell_args* __re
 		for (int64_t blk = w.begin; blk < w.end; blk++)
 		{
 			const int64_t k = blk * blockDim.x + threadIdx.x;
-			if constexpr (PHASE == phase_prepare)
-				cell_prepare_at(k, c.A, c.S, (float)c.voxel_volume, c.dt, c.vox, c.vol, c.sec, c.sat, c.upt, c.nex, c.num,
-								c.den, c.fac, c.rnum, c.rden, c.rfac, c.ballots, c.conflict);
+			if constexpr (PHASE == phase_reset)
+				cell_reset_at(k, c.A, c.vox, c.ballots, c.conflict);
 			else if constexpr (PHASE == phase_ballot)
 				cell_ballot_at(k, c.A, c.vox, c.ballots, c.win, c.conflict);
+			else if constexpr (PHASE == phase_prepare)
+				cell_prepare_at(k, c.A, c.S, (float)c.voxel_volume, c.dt, c.win, c.vol, c.sec, c.sat, c.upt, c.nex, c.num,
+								c.den, c.fac, c.rnum, c.rden, c.rfac);
 			else if constexpr (PHASE == phase_sum)
 				cell_sum_at(k, c.A, c.S, c.win, c.num, c.den, c.fac, c.rnum, c.rden, c.rfac);
 			else if constexpr (PHASE == phase_apply)
@@ -524,45 +567,49 @@ void launch_cell(bfvm_ctx* ctx, bool recompute)
 	const unsigned agent_blocks = (unsigned)((A + 255) / 256);
 	const int64_t pairs = (int64_t)A * S;
 	const unsigned pair_blocks = (unsigned)((pairs + 255) / 256);
-	if (recompute)
+	if (recompute && a.sorted && A > 0)
+	{
+		hipLaunchKernelGGL(cell_sorted_prepare_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S,
+						   (uint64_t)ctx->mesh.V, (float)voxel_volume(ctx), ctx->mesh.dt, a.keys + a.capacity,
+						   a.idx + a.capacity, a.vol, a.sec, a.sat, a.upt, a.nex, a.num, a.den, a.fac, a.snum, a.sden,
+						   a.sfac, a.rnum, a.rden, a.rfac, ctx->ballots, a.multi, ctx->conflict);
+		BFVM_HIP(hipGetLastError());
+		hipLaunchKernelGGL(cell_sorted_sum_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S,
+						   (uint64_t)ctx->mesh.V, a.keys + a.capacity, a.idx + a.capacity, a.snum, a.sden, a.sfac,
+						   a.rnum, a.rden, a.rfac);
+		BFVM_HIP(hipGetLastError());
+	}
+	else if (recompute)
 	{
 		// at least one block so the conflict flag is cleared even without agents
-		hipLaunchKernelGGL(cell_prepare_kernel, dim3(pair_blocks > 0 ? pair_blocks : 1), dim3(256), 0, ctx->stream, A,
-						   S, (float)voxel_volume(ctx), ctx->mesh.dt, a.vox, a.vol, a.sec, a.sat, a.upt, a.nex, a.num,
-						   a.den, a.fac, a.rnum, a.rden, a.rfac, ctx->ballots, ctx->conflict);
+		hipLaunchKernelGGL(cell_reset_kernel, dim3(std::max(agent_blocks, 1u)), dim3(256), 0, ctx->stream, A, a.vox,
+						   ctx->ballots, ctx->conflict);
 		BFVM_HIP(hipGetLastError());
 		if (A > 0)
 		{
-			if (a.sorted)
-			{
-				hipLaunchKernelGGL(cell_sorted_gather_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S,
-								   (uint64_t)ctx->mesh.V, a.keys + a.capacity, a.idx + a.capacity, a.num, a.den, a.fac,
-								   a.snum, a.sden, a.sfac);
-				BFVM_HIP(hipGetLastError());
-				hipLaunchKernelGGL(cell_sorted_sum_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S,
-								   (uint64_t)ctx->mesh.V, a.keys + a.capacity, a.idx + a.capacity, a.snum, a.sden,
-								   a.sfac, a.rnum, a.rden, a.rfac, ctx->ballots, a.multi, ctx->conflict);
-				BFVM_HIP(hipGetLastError());
-			}
-			else
-			{
-				hipLaunchKernelGGL(cell_ballot_kernel, dim3(agent_blocks), dim3(256), 0, ctx->stream, A, a.vox,
-								   ctx->ballots, a.win, ctx->conflict);
-				BFVM_HIP(hipGetLastError());
-				hipLaunchKernelGGL(cell_sum_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S, a.win,
-								   a.num, a.den, a.fac, a.rnum, a.rden, a.rfac);
-				BFVM_HIP(hipGetLastError());
-			}
+			hipLaunchKernelGGL(cell_ballot_kernel, dim3(agent_blocks), dim3(256), 0, ctx->stream, A, a.vox,
+							   ctx->ballots, a.win, ctx->conflict);
+			BFVM_HIP(hipGetLastError());
+			hipLaunchKernelGGL(cell_prepare_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S,
+							   (float)voxel_volume(ctx), ctx->mesh.dt, a.win, a.vol, a.sec, a.sat, a.upt, a.nex, a.num,
+							   a.den, a.fac, a.rnum, a.rden, a.rfac);
+			BFVM_HIP(hipGetLastError());
+			hipLaunchKernelGGL(cell_sum_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S, a.win, a.num,
+							   a.den, a.fac, a.rnum, a.rden, a.rfac);
+			BFVM_HIP(hipGetLastError());
 		}
 	}
 	if (A == 0)
 		return;
 	by_storage(ctx->storage, [&](auto kind) {
 		constexpr int K = decltype(kind)::value;
-		hipLaunchKernelGGL(cell_apply_kernel<K>, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S,
-						   (int)ctx->compute_internalized, voxel_volume(ctx), a.vox, ctx->dens, ctx->dscale, ctx->dinv,
-						   ctx->rounding_step, a.intern, a.num, a.den, a.fac, a.rnum, a.rden, a.rfac, ctx->conflict);
-		BFVM_HIP(hipGetLastError());
+		if (ctx->compute_internalized)
+		{
+			hipLaunchKernelGGL(cell_apply_kernel<K>, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S, 1,
+							   voxel_volume(ctx), a.vox, ctx->dens, ctx->dscale, ctx->dinv, ctx->rounding_step,
+							   a.intern, a.num, a.den, a.fac, a.rnum, a.rden, a.rfac, ctx->conflict);
+			BFVM_HIP(hipGetLastError());
+		}
 		hipLaunchKernelGGL(cell_densities_kernel<K>, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S,
 						   (int)ctx->compute_internalized, a.vox, ctx->dens, ctx->dscale, ctx->dinv, ctx->rounding_step,
 						   a.rnum, a.rden,
@@ -585,8 +632,8 @@ void free_batch_cell(bfvm_batch* b)
 
 // Per-instance arguments and work items of the batched secretion, rebuilt when `epoch` (the batch's sum of
 // instance epochs, which moves whenever an instance's agents change) differs from the plan's.  Items cover
-// blocks of 256 (agent, substrate) pairs (at least one block per instance, so the recompute clears every
-// conflict flag) and blocks of 256 agents, 8 blocks per item.
+// blocks of 256 (agent, substrate) pairs and blocks of 256 agents (at least one block per instance, so the recompute
+// clears every conflict flag), 8 blocks per item.
 void refresh_batch_cell(bfvm_batch* b, uint64_t epoch)
 {
 	auto& cp = b->cell;
@@ -636,8 +683,8 @@ void refresh_batch_cell(bfvm_batch* b, uint64_t epoch)
 		c.scale = ctx->dscale;
 		c.inv = ctx->dinv;
 		c.rounding = b->rounding;
-		const int64_t pair_blocks = std::max<int64_t>(1, ((int64_t)c.A * c.S + 255) / 256);
-		const int64_t agent_blocks = ((int64_t)c.A + 255) / 256;
+		const int64_t pair_blocks = ((int64_t)c.A * c.S + 255) / 256;
+		const int64_t agent_blocks = std::max<int64_t>(1, ((int64_t)c.A + 255) / 256);
 		for (int64_t b0 = 0; b0 < pair_blocks; b0 += per_item)
 			pairs.push_back(batch_item { (int32_t)i, 0, b0, std::min(pair_blocks, b0 + per_item) });
 		for (int64_t b0 = 0; b0 < agent_blocks; b0 += per_item)
@@ -675,7 +722,7 @@ static void launch_cell_phase(bfvm_batch* b, const batch_item* items, int n)
 	BFVM_HIP(hipGetLastError());
 }
 
-// The secretion of every instance of a refreshed, batched plan: recompute (prepare, ballot, sum) and apply
+// The secretion of every instance of a refreshed, batched plan: recompute (reset, ballot, prepare, sum) and apply
 // (apply, densities), one launch per phase, in the order of launch_cell.
 void launch_batched_cell(bfvm_batch* b, bool recompute)
 {
@@ -684,8 +731,9 @@ void launch_batched_cell(bfvm_batch* b, bool recompute)
 		constexpr int K = decltype(kind)::value;
 		if (recompute)
 		{
-			launch_cell_phase<K, phase_prepare>(b, cp.pair_items, cp.npair);
+			launch_cell_phase<K, phase_reset>(b, cp.agent_items, cp.nagent);
 			launch_cell_phase<K, phase_ballot>(b, cp.agent_items, cp.nagent);
+			launch_cell_phase<K, phase_prepare>(b, cp.pair_items, cp.npair);
 			launch_cell_phase<K, phase_sum>(b, cp.pair_items, cp.npair);
 		}
 		launch_cell_phase<K, phase_apply>(b, cp.pair_items, cp.npair);
