@@ -111,8 +111,9 @@ struct filter_args
 	int64_t row_elems, outer_stride;
 	uint32_t row_mul, s_mul, x_mul; // fdiv pairs of row_columns, S and X (x axis: Y)
 	int row_shift, s_shift, x_shift;
-	// staged x rows: a task is `rows` rows of XS elements in the workgroup's LDS, lines_pass lines of a row at a time
-	int rows, lines_pass, passes, row_lines;
+	// staged x rows: a task is `rows` rows of XS elements in the workgroup's LDS; lines_pass lines at a time in each wave
+	// (kw == blocks) or in all of them
+	int rows, lines_pass, passes;
 	int64_t total_rows;
 	int table_floats;			// floats of the table; in LDS, the storage scales [S] follow (16-bit forms)
 	int exchange_at, rows_at; // LDS offsets in bytes of the exchange area and the staged rows
@@ -626,8 +627,10 @@ __device__ __forceinline__ void filter_rows_task(const filter_args& a, int64_t t
 
 	filter_place at;
 	at.lane = tid & 63;
-	at.wave = tid >> 6;
-	at.waves = nthr >> 6;
+	const bool whole = a.kw == a.blocks; // each wave has whole lines
+	const int wave = tid >> 6, waves = nthr >> 6;
+	at.wave = whole ? 0 : wave;
+	at.waves = whole ? 1 : waves;
 	at.dist = at.slots = a.lines_pass;
 	at.slot = at.lane % a.lines_pass;
 	const int b = at.lane / a.lines_pass;
@@ -635,17 +638,16 @@ __device__ __forceinline__ void filter_rows_task(const filter_args& a, int64_t t
 	at.i = b % a.kw;
 	at.k = at.wave * a.kw + at.i;
 	at.last = a.blocks - 1;
-	const int r = b / a.kw; // several rows only in one wave, which then holds all blocks of a line
 	const int mk = FULL || at.k < at.last ? M : a.mlast;
 	constexpr int N = sure<M, FULL>();
-	const bool in_rows = r < nrows && at.k <= at.last;
 
 	for (int pass = 0; pass < a.passes; pass++)
 	{
-		const int line = pass * a.lines_pass + at.slot;
 		if (pass > 0 && at.waves > 1)
 			__syncthreads(); // the exchange area of the pass before
-		at.active = in_rows && line < a.row_lines;
+		const int first = (whole ? pass * waves + wave : pass) * a.lines_pass + at.slot;
+		const int r = (int)fdivu((uint32_t)first, a.s_mul, a.s_shift), line = first - r * S;
+		at.active = b < a.kw && at.k <= at.last && r < nrows;
 		const int pos = r * XS + at.k * M * S + line;
 		float v[M];
 		const elem* lv = l + (at.active ? pos : 0); // inactive lanes read what is there
@@ -659,8 +661,7 @@ __device__ __forceinline__ void filter_rows_task(const filter_args& a, int64_t t
 		uint32_t h = K == store_f32 ? 0u : sr_seed(row0 * XS + pos, rounding_key(a.rounding, 1));
 		const int So = fresh_uniform(S); // the stores' addresses are not the loads' held
 		elem* lo = l + pos;
-		const int sl = min(line, a.row_lines - 1);
-		auto row = [&](int rw) { return lt[rw * S + sl]; };
+		auto row = [&](int rw) { return lt[rw * S + line]; };
 		filter_line<M, FULL, 1>(v, row, mk, a.blocks, at, (float*)(lds + a.exchange_at), [&](int j, float x) {
 			elem* o = lo + j * So;
 			if constexpr (K == store_f32)
@@ -677,7 +678,7 @@ __device__ __forceinline__ void filter_rows_task(const filter_args& a, int64_t t
 				if (at.k == (mx ? at.last : 0) && row(mx ? fr_max_on : fr_min_on) != 0.f)
 				{
 					const float val = row(mx ? fr_max : fr_min);
-					l[pos + (mx ? mk - 1 : 0) * S] = (elem)(K == store_f32 ? val : val * ls[sl]);
+					l[pos + (mx ? mk - 1 : 0) * S] = (elem)(K == store_f32 ? val : val * ls[line]);
 				}
 	}
 	group_sync();
@@ -750,7 +751,7 @@ __global__ __launch_bounds__(512) void filter_rows_kernel(filter_args a)
 
 // block lengths the kernels are built for: odd ones where the rows are staged (LDS banks)
 static constexpr int column_blocks[] = { 2, 3, 4, 5, 7, 9, 11, 13, 14, 16, 18, 20, 22, 25 };
-static constexpr int row_blocks[] = { 3, 5, 7, 9, 11, 13, 15, 17 };
+static constexpr int row_blocks[] = { 3, 5, 7, 9, 11, 13, 15, 17, 19, 21, 23, 25 };
 
 // f(block length, every block full) as compile-time constants, for the lengths listed
 template <int... Ms, typename F>
@@ -805,6 +806,13 @@ static double filter_cost(int m, int waves, bool full, double used)
 	return (m + 8.0) / m * std::pow(used, -0.4) * (m <= 16 ? 0.75 : 1.0) * (full ? 1.0 : 1.15) * (waves > 4 ? 1.5 : 1.0);
 }
 
+// Staged rows: lanes without a line cost their full share, and larger workgroups wait for each other.
+static double row_waves_factor(int waves) { return waves > 4 ? 0.75 : waves > 2 ? 0.95 : 1.0; }
+static double row_cost(const filter_plan& p, bool full, double used)
+{
+	return (p.m + 8.0) / p.m / used * (full ? 1.0 : 1.05) / row_waves_factor(p.waves);
+}
+
 filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 {
 	const auto& g = ctx->mesh;
@@ -816,7 +824,10 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 		return best;
 	// best: the cheapest lengths; quick: the shortest chain of operations, for meshes that do not fill the card anyway
 	auto consider = [&](const filter_plan& p, double used) {
-		const double cost = filter_cost(p.m, p.waves, n % p.m == 0, used), chain = std::max(p.m, 7) + 8 * p.waves;
+		const int waves = p.kw < p.blocks ? p.waves : 1; // that a line takes
+		const double cost = p.staged && waves == 1 ? row_cost(p, n % p.m == 0, used)
+												   : filter_cost(p.m, waves, n % p.m == 0, used);
+		const double chain = std::max(p.m, 7) + 8 * waves;
 		if (best.blocks == 0 || cost < best_cost)
 		{
 			best = p;
@@ -830,16 +841,14 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 	};
 	// a line's last block holds at least half its length (sure)
 	auto fits = [&](int m) { return n - ((n + m - 1) / m - 1) * m >= m / 2; };
-	// x rows of a substrate count that 4 does not divide: through LDS below 6 substrates, where most of a direct
-	// column of 4 overlaps its neighbour (staged / direct, us: 160^3 x 5 FP32 37 / 59, FP16 44 / 65; 131x97x143 x 5
-	// FP32 21 / 30), direct from 6 on (160^3 x 6 FP32 67 / 59, FP16 80 / 65; x 11 111 / 82, 137 / 97; x 15 121 / 96,
-	// 153 / 110; x 9 and x 10 in FP32 alone run 5 % faster staged)
-	if (axis == 0 && S % 4 != 0 && S < 6)
+	// x rows of a substrate count that 4 does not divide go through LDS where a row fits there; direct columns of 4
+	// overlap, and their last one stores in parts.  Staged / direct, us: 160^3 x 5 FP32 25 / 58, FP16 28 / 62; 160^3 x 7
+	// 35 / 62, 36 / 79; 160^3 x 13 54 / 77, 67 / 73; 134x200x143 x 15 60 / 79, 75 / 90; 400x200x200 x 7 159 / 310, 111 /
+	// 260; 256^3 x 5 122 / 278, 118 / 207; 147x127x200 x 14 57 / 71, but FP16 71 / 63.
+	const int64_t rows = (int64_t)g.grid[1] * g.grid[2];
+	if (axis == 0 && S % 4 != 0 && XS * e >= 16 && rows < (int64_t)1 << 31)
 	{
 		const int L = S;
-		const int64_t rows = (int64_t)g.grid[1] * g.grid[2];
-		if (XS * e < 16 || rows >= (int64_t)1 << 31)
-			return best;
 		for (int m : row_blocks)
 		{
 			if (!fits(m))
@@ -848,11 +857,25 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 			p.m = m;
 			p.blocks = (n + m - 1) / m;
 			p.staged = true;
-			if (p.blocks * L <= 64)
+			if (p.blocks <= 64)
 			{
-				p.lines_pass = L;
+				// whole lines in each wave, of as many rows as fill the waves best
+				p.lines_pass = 64 / p.blocks;
 				p.kw = p.blocks;
-				p.rows = 64 / (L * p.blocks);
+				double best_used = 0;
+				for (int r = 1; r <= 16 && (r == 1 || r * XS * e <= 24 * 1024); r++)
+				{
+					const int groups = (r * L + p.lines_pass - 1) / p.lines_pass, waves = std::min(groups, filter_max_waves);
+					const int passes = (groups + waves - 1) / waves;
+					const double used = (double)r * L / (waves * passes * p.lines_pass) * row_waves_factor(waves);
+					if (used > best_used * 1.02)
+					{
+						best_used = used;
+						p.rows = r;
+						p.waves = waves;
+						p.passes = passes;
+					}
+				}
 			}
 			else
 			{
@@ -861,13 +884,13 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 				p.kw = std::min(64 / p.lines_pass, p.blocks);
 				p.waves = (p.blocks + p.kw - 1) / p.kw;
 				p.rows = 1;
+				p.passes = (L + p.lines_pass - 1) / p.lines_pass;
 			}
 			if (p.waves > filter_max_waves)
 				continue;
-			p.passes = (L + p.lines_pass - 1) / p.lines_pass;
 			p.exchange_at = filter_lds_table(ctx, p.blocks, p.kw);
 			p.rows_at =
-				p.exchange_at + (p.waves > 1 ? ((2 * p.waves + 1) * p.lines_pass * 4 + 15) / 16 * 16 : 0);
+				p.exchange_at + (p.kw < p.blocks ? ((2 * p.waves + 1) * p.lines_pass * 4 + 15) / 16 * 16 : 0);
 			const int64_t lds = p.rows_at + (p.rows * XS * e + 15) / 16 * 16;
 			if (lds > 64 * 1024)
 				continue;
@@ -877,7 +900,7 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 			consider(p, (double)p.rows * L * n / (64.0 * p.waves * m * p.passes));
 		}
 	}
-	else
+	if (best.blocks == 0)
 	{
 		const int64_t row_elems = axis == 0 ? S : axis == 1 ? XS : (int64_t)g.grid[1] * XS;
 		const int64_t row_columns = (row_elems + 3) / 4;
@@ -960,7 +983,6 @@ static filter_args make_filter_args(const bfvm_ctx* ctx, int axis, const filter_
 		a.rows = p.rows;
 		a.lines_pass = p.lines_pass;
 		a.passes = p.passes;
-		a.row_lines = g.S;
 		a.total_rows = (int64_t)g.grid[1] * g.grid[2];
 		a.rows_at = p.rows_at;
 		fast_divisor((uint32_t)g.grid[1], a.row_mul, a.row_shift);
@@ -982,19 +1004,16 @@ void launch_filter_sweep(bfvm_ctx* ctx, int axis)
 	const axis_tables& t = ctx->axes[axis];
 	const filter_plan& p = t.filter;
 	const filter_args a = make_filter_args(ctx, axis, p, t.filter_tab);
-	int64_t cap = ctx->sweep_workgroups[axis] > 0 ? ctx->sweep_workgroups[axis] : (int64_t)1 << 24;
-	// Staged rows: while the densities stay in the Infinity Cache, 8 waves per CU that prefetch their next rows beat one
-	// pass of short-lived ones (200^3 x 8: 89 against 97 us); from memory one pass is the faster (400^3 x 8: 822 against
-	// 848 us).
-	if (p.staged && (int64_t)(ctx->mesh.V * ctx->mesh.S * storage_bytes(ctx->storage)) <= infinity_cache_bytes)
-		cap = std::min<int64_t>(cap, filter_fill_waves / p.waves);
+	// one task per workgroup unless the caller or the autotuner set a cap: fewer workgroups that fetch their next rows
+	// early took 37 against 35 us on 160^3 x 7, 77 against 60 on 134x200x143 x 15 (16 waves per CU)
+	const int64_t cap = ctx->sweep_workgroups[axis] > 0 ? ctx->sweep_workgroups[axis] : (int64_t)1 << 24;
 	const dim3 blocks((unsigned)std::min(p.tasks, cap)), threads(64 * p.waves);
 	const size_t lds = p.lds;
 	const bool full = a.mlast == a.m, back = a.row_elems % 4 != 0;
 	by_storage(ctx->storage, [&](auto kind) {
 		constexpr int K = decltype(kind)::value;
 		if (p.staged)
-			by_block<3, 5, 7, 9, 11, 13, 15, 17>(p.m, full, [&](auto m, auto f) {
+			by_block<3, 5, 7, 9, 11, 13, 15, 17, 19, 21, 23, 25>(p.m, full, [&](auto m, auto f) {
 				hipLaunchKernelGGL((filter_rows_kernel<m, f, K>), blocks, threads, lds, ctx->stream, a);
 			});
 		else
