@@ -1383,6 +1383,7 @@ struct batch_override
 	}
 };
 
+static void free_batch_small(bfvm_batch* b);
 static void free_batch(bfvm_batch* b)
 {
 	for (auto& g : b->graphs)
@@ -1394,6 +1395,7 @@ static void free_batch(bfvm_batch* b)
 		g = graph_slot {};
 	}
 	free_batch_cell(b);
+	free_batch_small(b);
 	for (int i = 0; i < bfvm_batch::branches; i++)
 	{
 		if (b->branch_event[i])
@@ -1441,13 +1443,15 @@ static uint64_t batch_epoch(const bfvm_batch* b)
 	return e;
 }
 
-// one(instance) for every instance, its launches on its branch: a step's launches of one instance follow each other
+// one(instance, small) for every instance, its launches on its branch: a step's launches of one instance follow each other
 // on a branch, so the ends of one instance's kernels are covered by the other branches', and an instance of ordinary
 // size stays in the Infinity Cache from one axis to the next.  The branches are forked from the batch's stream and
 // joined to it, also when a launch is refused.  One launch per axis over all instances (workgroups walking a list of
 // line groups) took, for a step without gradient of 64 instances in 16-bit storage, 3.84 ms; branches 2.96 ms.
-template <typename F>
-static void on_branches(bfvm_batch* b, F&& one)
+// `first` runs on the batch's stream, beside the other branches; one's second argument: whether the instance is among
+// those that share sweep launches.
+template <typename G, typename F>
+static void on_branches(bfvm_batch* b, G&& first, F&& one)
 {
 	BFVM_HIP(hipEventRecord(b->branch_event[0], b->stream));
 	for (int i = 1; i < bfvm_batch::branches; i++)
@@ -1455,10 +1459,11 @@ static void on_branches(bfvm_batch* b, F&& one)
 	std::exception_ptr failed;
 	try
 	{
+		first();
 		for (size_t i = 0; i < b->ctx.size(); i++)
 		{
 			batch_override o(b->ctx[i], b, b->branch_stream[b->branch_of[i]]);
-			one(b->ctx[i]);
+			one(b->ctx[i], b->small.count > 0 && b->small.member[i]);
 		}
 	}
 	catch (...)
@@ -1474,6 +1479,87 @@ static void on_branches(bfvm_batch* b, F&& one)
 		std::rethrow_exception(failed);
 }
 
+// The instances whose sweeps share launches, and those launches' arguments, for the batch's present epoch.
+// Host-synchronous: call outside stream capture.
+static void refresh_batch_small(bfvm_batch* b, uint64_t epoch)
+{
+	auto& sp = b->small;
+	if (sp.epoch == epoch)
+		return;
+	BFVM_HIP(hipStreamSynchronize(b->stream));
+	sp.member.assign(b->ctx.size(), 0);
+	sp.count = 0;
+	for (size_t i = 0; i < b->ctx.size(); i++)
+		sp.count += sp.member[i] = small_filter(b->ctx[i]) ? 1 : 0;
+	if (sp.count < 2)
+	{
+		sp.member.assign(b->ctx.size(), 0);
+		sp.count = 0;
+	}
+	const size_t each = small_filter_args_bytes();
+	for (int axis = 0; axis < 3; axis++)
+	{
+		std::vector<char> args;
+		std::vector<int> first { 0 };
+		sp.lds[axis] = 0;
+		for (size_t i = 0; i < b->ctx.size(); i++)
+		{
+			if (!sp.member[i] || axis >= b->ctx[i]->mesh.dims)
+				continue;
+			batch_override o(b->ctx[i], b, b->stream);
+			int tasks = 0, lds = 0;
+			args.resize(args.size() + each);
+			small_filter_args(b->ctx[i], axis, args.data() + args.size() - each, tasks, lds);
+			first.push_back(first.back() + tasks);
+			sp.lds[axis] = std::max(sp.lds[axis], lds);
+		}
+		sp.with_axis[axis] = (int)first.size() - 1;
+		sp.tasks[axis] = first.back();
+		if (args.empty())
+			continue;
+		if (!sp.inst[axis]) // for as many instances as the batch has
+		{
+			BFVM_HIP(hipMalloc(&sp.inst[axis], each * b->ctx.size()));
+			BFVM_HIP(hipMalloc(&sp.first[axis], sizeof(int) * (b->ctx.size() + 1)));
+		}
+		BFVM_HIP(hipMemcpy(sp.inst[axis], args.data(), args.size(), hipMemcpyHostToDevice));
+		BFVM_HIP(hipMemcpy(sp.first[axis], first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice));
+	}
+	sp.epoch = epoch;
+}
+
+static void free_batch_small(bfvm_batch* b)
+{
+	for (int axis = 0; axis < 3; axis++)
+	{
+		if (b->small.inst[axis])
+			(void)hipFree(b->small.inst[axis]);
+		if (b->small.first[axis])
+			(void)hipFree(b->small.first[axis]);
+	}
+	b->small = bfvm_batch::small_plan {};
+}
+
+// f(instance) on the batch's stream for the instances that share sweep launches
+template <typename F>
+static void on_small(bfvm_batch* b, F&& f)
+{
+	for (size_t i = 0; i < b->ctx.size(); i++)
+		if (b->small.member[i])
+		{
+			batch_override o(b->ctx[i], b, b->stream);
+			f(b->ctx[i]);
+		}
+}
+
+static void launch_small_axis(bfvm_batch* b, int axis)
+{
+	const auto& sp = b->small;
+	if (sp.with_axis[axis] > 0)
+		launch_small_filters(b->storage, b->stream, sp.inst[axis], sp.first[axis], sp.with_axis[axis], sp.tasks[axis],
+							 sp.lds[axis]);
+}
+
 static void enqueue_batch_sweeps(bfvm_batch* b, bool with_gradient = false)
 {
 	if (b->storage != BFVM_STORAGE_F32)
@@ -1481,21 +1567,41 @@ static void enqueue_batch_sweeps(bfvm_batch* b, bool with_gradient = false)
 		batch_override o(b->ctx[0], b, b->stream);
 		launch_advance_rounding(b->ctx[0]);
 	}
-	on_branches(b, [&](bfvm_ctx* c) {
-		enqueue_dirichlet(c);
-		for (int axis = 0; axis < c->mesh.dims; axis++)
-		{
-			launch_sweep(c, axis);
-			launch_dirichlet_interior(c);
-		}
-		if (with_gradient)
-			launch_gradient(c);
-	});
+	on_branches(
+		b,
+		[&] {
+			on_small(b, enqueue_dirichlet);
+			for (int axis = 0; axis < 3; axis++)
+			{
+				launch_small_axis(b, axis);
+				on_small(b, [&](bfvm_ctx* c) {
+					if (axis < c->mesh.dims)
+						launch_dirichlet_interior(c);
+				});
+			}
+		},
+		[&](bfvm_ctx* c, bool small) {
+			if (small)
+				return;
+			enqueue_dirichlet(c);
+			for (int axis = 0; axis < c->mesh.dims; axis++)
+			{
+				launch_sweep(c, axis);
+				launch_dirichlet_interior(c);
+			}
+			if (with_gradient)
+				launch_gradient(c);
+		});
+	if (with_gradient && b->small.count > 0)
+		on_branches(b, [] {}, [](bfvm_ctx* c, bool small) {
+			if (small)
+				launch_gradient(c);
+		});
 }
 
 static void enqueue_batch_gradient(bfvm_batch* b)
 {
-	on_branches(b, [](bfvm_ctx* c) { launch_gradient(c); });
+	on_branches(b, [] {}, [](bfvm_ctx* c, bool) { launch_gradient(c); });
 }
 
 // the secretion of every instance: batched launches when the plan allows, else instance by instance
@@ -1627,6 +1733,7 @@ int bfvm_batch_timestep(bfvm_batch* batch, int32_t recompute, int32_t with_gradi
 		auto& slot = batch->graphs[(recompute ? 2 : 0) + (with_gradient ? 1 : 0)];
 		const uint64_t epoch = batch_epoch(batch);
 		refresh_batch_cell(batch, epoch);
+		refresh_batch_small(batch, epoch);
 		if (!slot.exec || slot.epoch != epoch)
 		{
 			if (slot.exec)
@@ -1721,16 +1828,19 @@ int bfvm_batch_benchmark(bfvm_batch* batch, int32_t what, int32_t iterations, fl
 			for (bfvm_ctx* c : batch->ctx)
 				account_secretion(c, (int64_t)iterations + 1, batch->stream);
 		refresh_batch_cell(batch, batch_epoch(batch));
+		refresh_batch_small(batch, batch_epoch(batch));
 		auto one = [&]() {
 			switch (what)
 			{
 			case BFVM_KERNEL_SWEEP_X:
 			case BFVM_KERNEL_SWEEP_Y:
 			case BFVM_KERNEL_SWEEP_Z:
-				on_branches(batch, [&](bfvm_ctx* c) {
-					if (what - BFVM_KERNEL_SWEEP_X < c->mesh.dims)
-						launch_sweep(c, what - BFVM_KERNEL_SWEEP_X);
-				});
+				on_branches(
+					batch, [&] { launch_small_axis(batch, what - BFVM_KERNEL_SWEEP_X); },
+					[&](bfvm_ctx* c, bool small) {
+						if (!small && what - BFVM_KERNEL_SWEEP_X < c->mesh.dims)
+							launch_sweep(c, what - BFVM_KERNEL_SWEEP_X);
+					});
 				break;
 			case BFVM_KERNEL_GRADIENT:
 				enqueue_batch_gradient(batch);

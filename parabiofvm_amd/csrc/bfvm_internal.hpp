@@ -510,6 +510,17 @@ struct bfvm_batch
 	hipStream_t branch_stream[branches] = {}; // [0] is `stream`
 	hipEvent_t branch_event[branches] = {};   // [0]: the fork
 	std::vector<int> branch_of;				 // per instance
+	// instances whose sweeps share one launch per axis, and per axis their arguments and running task counts on the
+	// device, rebuilt with the batch's epoch
+	struct small_plan
+	{
+		std::vector<char> member; // per instance
+		int count = 0;
+		void* inst[3] = { nullptr, nullptr, nullptr };
+		int* first[3] = { nullptr, nullptr, nullptr };
+		int with_axis[3] = { 0, 0, 0 }, tasks[3] = { 0, 0, 0 }, lds[3] = { 0, 0, 0 };
+		uint64_t epoch = ~0ull;
+	} small;
 	// batched secretion: per-instance arguments and work items over (agent, substrate) and agent blocks, rebuilt
 	// when an instance's agents change (cell_epoch); per-instance launches when an instance uses the sorted
 	// reduction
@@ -567,6 +578,10 @@ void check_batch_axis(const bfvm_ctx* ctx, int axis, int instance);
 size_t filter_table_floats(const filter_plan& p, int S);
 void launch_filter_coefficients(const bfvm_ctx* ctx, int axis, const filter_plan& p, float* tab, hipStream_t stream);
 void launch_filter_sweep(bfvm_ctx* ctx, int axis);
+bool small_filter(const bfvm_ctx* ctx);
+size_t small_filter_args_bytes();
+void small_filter_args(const bfvm_ctx* ctx, int axis, void* out, int& tasks, int& lds);
+void launch_small_filters(int storage, hipStream_t stream, const void* inst, const int* first, int count, int tasks, int lds);
 
 // (mul, shift) for n / d = (n * mul) >> shift, n < 2^31 (1 <= d < 2^31)
 void fast_divisor(uint32_t d, uint32_t& mul, int& shift);

@@ -113,7 +113,7 @@ struct filter_args
 	int row_shift, s_shift, x_shift;
 	// staged x rows: a task is `rows` rows of XS elements in the workgroup's LDS; lines_pass lines at a time in each wave
 	// (kw == blocks) or in all of them
-	int rows, lines_pass, passes;
+	int rows, lines_pass, passes, staged;
 	int64_t total_rows;
 	int table_floats;			// floats of the table; in LDS, the storage scales [S] follow (16-bit forms)
 	int exchange_at, rows_at; // LDS offsets in bytes of the exchange area and the staged rows
@@ -746,6 +746,59 @@ __global__ __launch_bounds__(512) void filter_rows_kernel(filter_args a)
 	}
 }
 
+// ---- many small meshes in one launch --------------------------------------------------------------------------------
+//
+// A mesh that does not fill the card (small_filter) is bound by its launches and their latency; the small instances of a
+// batch share one launch per axis.  A workgroup (one wave) finds its instance among the running task counts and the
+// block length by a branch; the arguments are read from memory.
+template <int K, int... Ms>
+__device__ __forceinline__ void small_columns(const filter_args& a, int64_t task, raw16* lds)
+{
+	auto* sh = (typename vec_of<4>::type*)((char*)lds + a.exchange_at);
+	((a.m == Ms ? filter_columns_task<Ms, false, K, false, true>(a, task, (float*)lds, sh, true) : void()), ...);
+}
+template <int M, int K>
+__device__ __forceinline__ void small_rows_of(const filter_args& a, int64_t task, raw16* lds)
+{
+	row_pieces<M, K> x;
+	float tab[table_regs];
+	table_load<K>(a, tab);
+	rows_fetch<M, K>(a, task, x);
+	table_store<K>(a, tab, (float*)lds);
+	rows_put<M, K>(a, task, x, (char*)lds + a.rows_at);
+	group_sync();
+	filter_rows_task<M, false, K>(a, task, (char*)lds);
+}
+template <int K, int... Ms>
+__device__ __forceinline__ void small_rows(const filter_args& a, int64_t task, raw16* lds)
+{
+	((a.m == Ms ? small_rows_of<Ms, K>(a, task, lds) : void()), ...);
+}
+
+template <int K>
+__global__ __launch_bounds__(64) void filter_small_kernel(const filter_args* __restrict__ inst,
+														  const int* __restrict__ first, int count)
+{
+	extern __shared__ raw16 filter_lds[];
+	const int b = (int)xcd_order(blockIdx.x, gridDim.x);
+	int lo = 0, hi = count - 1; // first[lo] <= b < first[hi + 1]
+	while (lo < hi)
+	{
+		const int mid = (lo + hi + 1) / 2;
+		if (first[mid] <= b)
+			lo = mid;
+		else
+			hi = mid - 1;
+	}
+	const int i = __builtin_amdgcn_readfirstlane(lo);
+	const filter_args& a = inst[i];
+	const int64_t task = b - first[i];
+	if (a.staged)
+		small_rows<K, 3, 5, 7, 9, 11, 13, 15, 17>(a, task, filter_lds);
+	else
+		small_columns<K, 2, 3, 4, 5, 7, 9, 11, 13, 14, 16>(a, task, filter_lds);
+}
+
 // ---- host side ------------------------------------------------------------------------------------------------------
 
 
@@ -977,6 +1030,7 @@ static filter_args make_filter_args(const bfvm_ctx* ctx, int axis, const filter_
 	const int64_t XS = (int64_t)g.grid[0] * g.S;
 	fast_divisor((uint32_t)g.S, a.s_mul, a.s_shift);
 	fast_divisor((uint32_t)g.grid[axis == 0 ? 1 : 0], a.x_mul, a.x_shift);
+	a.staged = p.staged ? 1 : 0;
 	if (p.staged)
 	{
 		a.row_elems = XS;
@@ -1024,6 +1078,40 @@ void launch_filter_sweep(bfvm_ctx* ctx, int axis)
 						kernel = p.streamed ? filter_columns_kernel<m, f, K, true, true> : filter_columns_kernel<m, f, K, false, true>;
 				hipLaunchKernelGGL(kernel, blocks, threads, lds, ctx->stream, a);
 			});
+	});
+	BFVM_HIP(hipGetLastError());
+}
+
+// Whether an instance of a batch takes its sweeps in the launches shared by the small ones: one-wave workgroups, too few
+// to fill the card, blocks short enough for the shared kernel's registers.
+bool small_filter(const bfvm_ctx* ctx)
+{
+	if (ctx->algorithm != BFVM_SWEEP_PARTITIONED)
+		return false;
+	for (int axis = 0; axis < ctx->mesh.dims; axis++)
+	{
+		const filter_plan& p = ctx->axes[axis].filter;
+		if (p.blocks == 0 || p.waves != 1 || p.kw < p.blocks || p.m > 17 || (!p.staged && p.m > 16) ||
+			p.tasks >= filter_fill_waves || ctx->sweep_workgroups[axis] > 0)
+			return false;
+	}
+	return true;
+}
+
+size_t small_filter_args_bytes() { return sizeof(filter_args); }
+void small_filter_args(const bfvm_ctx* ctx, int axis, void* out, int& tasks, int& lds)
+{
+	const filter_plan& p = ctx->axes[axis].filter;
+	*(filter_args*)out = make_filter_args(ctx, axis, p, ctx->axes[axis].filter_tab);
+	tasks = (int)p.tasks;
+	lds = p.lds;
+}
+
+void launch_small_filters(int storage, hipStream_t stream, const void* inst, const int* first, int count, int tasks, int lds)
+{
+	by_storage(storage, [&](auto kind) {
+		hipLaunchKernelGGL(filter_small_kernel<decltype(kind)::value>, dim3((unsigned)tasks), dim3(64), (size_t)lds,
+						   stream, (const filter_args*)inst, first, count);
 	});
 	BFVM_HIP(hipGetLastError());
 }
