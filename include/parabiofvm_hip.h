@@ -82,7 +82,9 @@ typedef struct bfvm_ctx bfvm_ctx;
 #define BFVM_REDUCTION_SORTED 1 /* agents sorted by voxel at upload, one segmented sum per voxel, no atomics */
 
 /* Sweep algorithm (bfvm_set_sweep_algorithm). */
-#define BFVM_SWEEP_PARTITIONED 0 /* register-resident partitioned (modified) Thomas, FP64-derived coefficients */
+#define BFVM_SWEEP_PARTITIONED 0 /* lines in blocks held in registers: two-sided recursive filter (automatic shape), or
+								  * partitioned (modified) Thomas (a chunk or line count was asked for, or the
+								  * coefficients are outside the filter's range); FP64-derived coefficients */
 #define BFVM_SWEEP_EXACT 1		 /* one thread per line, the reference's FP32 coefficients and operation order */
 #define BFVM_SWEEP_STAGED 2		 /* the partitioned algorithm on tiles staged through LDS, one line per thread */
 
@@ -177,32 +179,33 @@ int bfvm_bulk_solve(bfvm_ctx* ctx);
 int bfvm_set_secretion_reduction(bfvm_ctx* ctx, int32_t mode);
 
 /* Selects the sweep algorithm (default BFVM_SWEEP_PARTITIONED) and, for the partitioned one, the
- * maximum chunk length per thread (0 = automatic).  Takes effect at the next solve. */
+ * maximum chunk length per thread (0 = automatic, the recursive filter).  Takes effect at the next solve. */
 int bfvm_set_sweep_algorithm(bfvm_ctx* ctx, int32_t algorithm, int32_t chunk);
 
 /* Per-axis tuning of the partitioned sweep: register chunk (8..64, 0 = automatic) and lines per workgroup
  * (y/z: consecutive columns per workgroup, x: rows per workgroup; 0 = automatic).  On a configuration the
  * register/LDS budget cannot hold, the previous one is kept and an error is returned. */
 int bfvm_set_sweep_tuning(bfvm_ctx* ctx, int32_t axis, int32_t chunk, int32_t lines_per_group);
-/* Most workgroups a partitioned or staged sweep launches (0 = automatic: 8192 partitioned, 4096 staged).
+/* Most workgroups a partitioned or staged sweep launches (0 = automatic: one line group per workgroup for the
+ * recursive filter, 8192 partitioned, 4096 staged).
  * Each workgroup loops over line groups (or tiles) in steps of the launched count, so a small cap makes
  * every workgroup run several passes.  No counterpart in the reference, whose sweeps launch one 256-thread
  * block per 256 lines (CUDA/diffusion_solver.cu:947-987). */
 int bfvm_set_sweep_workgroups(bfvm_ctx* ctx, int32_t workgroups);
 /* Workgroups the 3-D gradient kernel aims for by splitting z into chunks (0 = automatic). */
 int bfvm_set_gradient_tuning(bfvm_ctx* ctx, int32_t workgroups);
-/* Tile layout of the 3-D gradient: 0 = 256 columns by TY rows per workgroup, 1 = the workgroup's four waves
- * stacked along y (64 columns by 4 TY rows, the rows where waves meet passed through LDS).  Same results. */
+/* Rows of y per thread of the 3-D gradient where it is shaped by hand (a workgroup count, this or the order set):
+ * 0 = 4, 1 = 8.  Same results. */
 int bfvm_set_gradient_stacked(bfvm_ctx* ctx, int32_t stacked);
-/* Workgroup order of the 3-D gradient: 0 = each XCD runs consecutive z chunks of one row band, 1 = plane
+/* Workgroup order of the 3-D gradient: 0 = each XCD runs consecutive tiles, 1 = plane
  * order (the workgroups resident together cover one z chunk of every row band).  Same results.  No
  * counterpart in the reference, whose gradient is a host loop (host/gradient_solver.cpp:275-291). */
 int bfvm_set_gradient_order(bfvm_ctx* ctx, int32_t order);
 
 /* Autotuner, in place of the reference's fixed device launch shapes (work_block_size = 30,
  * CUDA/diffusion_solver.cpp:11; 256-thread blocks, CUDA/diffusion_solver.cu:947-987): times candidate shapes
- * of every sweep axis (register chunk, lines or rows per workgroup, workgroup count) and of the 3-D gradient
- * (workgroups, tile layout, workgroup order) on this context's mesh and keeps the fastest, as
+ * of every sweep axis (workgroup count; register chunk and lines or rows per workgroup where the axis does not take the
+ * recursive filter) and of the 3-D gradient (workgroups, rows per thread, workgroup order) on this context's mesh and keeps the fastest, as
  * bfvm_set_sweep_tuning / bfvm_set_sweep_workgroups / bfvm_set_gradient_tuning / bfvm_set_gradient_stacked /
  * bfvm_set_gradient_order would set them.  Results are cached per (axis, mesh
  * shape, substrate count, storage, algorithm) for the process, so a second context of the same shape tunes
@@ -286,12 +289,10 @@ int bfvm_benchmark(bfvm_ctx* ctx, int32_t what, int32_t iterations, float* avg_m
 /*
  * Batches of independent microenvironments.  No counterpart in the reference, which runs one
  * microenvironment per solver (src/solver.h); a batch advances many initialized contexts of any mesh shape
- * and substrate count with work-list launches over all instances: per secretion phase, per sweep axis (one
- * launch per thread layout: 4-element vectors where 4 divides the row, else one element) and for the
- * gradient, each driven by a device work list of (instance, block / line-group / tile range) items, and
- * replays the whole step (secretion of every instance -> Dirichlet -> x/y/z sweeps -> gradient) as one
- * captured HIP graph.  Per-instance results equal what bfvm_timestep gives for that context to the
- * partitioned sweep's tolerance (the same algorithm with 16-element blocks).
+ * and substrate count as one captured HIP graph (secretion of every instance -> Dirichlet -> x/y/z sweeps ->
+ * gradient): the secretion by one work-list launch per phase, the sweeps of small instances in one launch per axis,
+ * every other instance's sweeps and gradient as a chain on one of the graph's branches.  Per-instance results equal
+ * what bfvm_timestep gives for that context to the sweep's tolerance (the same algorithm).
  *
  * All contexts must be initialized on one device with one storage form and the partitioned sweep; they
  * keep their data (store/load through the per-context calls).  A context re-initialized while the batch
@@ -305,13 +306,11 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 int bfvm_batch_destroy(bfvm_batch* batch);
 int bfvm_batch_timestep(bfvm_batch* batch, int32_t recompute, int32_t with_gradient);
 int bfvm_batch_wait(bfvm_batch* batch);
-/* The batch's autotuner: per sweep axis and thread layout (4-element vectors, one element per thread) the
- * threads a line group aims for and the workgroup count of the work-list launch, and for the gradient the
- * tiles per work item and the workgroup count, each timed on copies of the instances' densities.  The
- * instances' densities are unchanged and their gradients are recomputed.  Synchronous. */
+/* The batch's launches are shaped by rules and by each instance's own tuning: nothing is timed.  The gradients are
+ * recomputed where the process's tuning cache has no entry for this list of shapes, and the entry is made. */
 int bfvm_batch_autotune(bfvm_batch* batch);
-/* Average ms per launch over all instances: BFVM_KERNEL_SWEEP_X/Y/Z and BFVM_KERNEL_GRADIENT (the batched
- * launch alone), BFVM_PHASE_SECRETION(_RECOMPUTE), _DIFFUSION, _GRADIENT and _TIMESTEP. */
+/* Average ms per launch over all instances: BFVM_KERNEL_SWEEP_X/Y/Z and BFVM_KERNEL_GRADIENT (without the
+ * launches around them), BFVM_PHASE_SECRETION(_RECOMPUTE), _DIFFUSION, _GRADIENT and _TIMESTEP. */
 int bfvm_batch_benchmark(bfvm_batch* batch, int32_t what, int32_t iterations, float* avg_ms);
 
 #ifdef __cplusplus

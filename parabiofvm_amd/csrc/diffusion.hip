@@ -5,7 +5,8 @@
 //   b_end = 1 + decay*dt/dims + dt*D/dx^2,  b_mid = 1 + decay*dt/dims + 2*dt*D/dx^2,
 // and for a line of one voxel b = 1 + decay*dt/dims (host/diffusion_solver.cpp:76-85).
 //
-// Two sweep algorithms:
+// Two sweep algorithms here (the recursive filter, which an automatic shape takes where it can, is in
+// filter_sweep.hip):
 //  * exact: one thread per line, the reference's sequential recurrence with its FP32 coefficients in its
 //    operation order (host/diffusion_solver.cpp:297-334, 378-480); bit-identical to the host path.
 //  * partitioned: the line is split into P blocks held in registers, one thread per (line, block).  Each

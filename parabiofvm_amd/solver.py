@@ -233,7 +233,7 @@ class DeviceSolver:
         return p.value, m.value, lpg.value
 
     def set_gradient_stacked(self, stacked):
-        """3-D gradient tiles with the workgroup's waves stacked along y (True) or side by side (False)."""
+        """3-D gradient with 8 (True) or 4 (False) rows per thread, where it is shaped by hand."""
         check("bfvm_set_gradient_stacked", self.lib.bfvm_set_gradient_stacked(self.h, int(bool(stacked))))
 
     def set_gradient_order(self, order):
@@ -282,8 +282,8 @@ class DeviceSolver:
 
 
 class Batch:
-    """Many initialized DeviceSolvers advanced together (bfvm_batch_*): one launch per sweep axis and one for
-    the gradient over all instances, the whole step replayed as one captured HIP graph.  Densities are
+    """Many initialized DeviceSolvers advanced together (bfvm_batch_*): small instances' sweeps
+    in shared launches, the others' sweeps and gradients on parallel branches of one captured HIP graph.  Densities are
     stored and loaded through each solver as before; call wait() before loading."""
 
     def __init__(self, solvers):
