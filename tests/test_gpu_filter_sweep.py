@@ -112,3 +112,58 @@ def test_large_coefficients_keep_the_partitioned_sweep(pkg, oracle_mod):
     err = np.abs(g.densities - o.densities).reshape(-1, 2)
     assert err[:, 1].max() <= REL * np.abs(o.densities).max()
     assert np.isfinite(g.densities).all()
+
+
+@pytest.mark.parametrize("S", [2, 5, 7, 13, 31])
+def test_staged_rows(S, pkg, oracle_mod):
+    """x rows staged several to a workgroup: lengths at which the blocks, the lines of a wave and the rows of a task
+    change, with row counts that leave a short last task; the tolerance is the lengths' test's."""
+    for n in (4, 21, 42, 63, 64, 65, 130, 181, 275):
+        if n > 65 and S > 13:  # longer than the partitioned sweep's tables allow, which every mesh must fit
+            continue
+        for rows in ((2, 2), (7, 3), (5, 13)):
+            p = random_problem(3, (n, *rows), S, seed=3 * n + S)
+            o, g = build_pair(pkg, oracle_mod, p, dtype=np.float64)
+            g.store()
+            for _ in range(2):
+                o.diffusion()
+                g.diffusion()
+            g.load()
+            assert_close(g.densities, o.densities, what=f"n {n} rows {rows} S {S}: {g.partition(0)}")
+            g.close()
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+@pytest.mark.parametrize("gradient", [False, True])
+def test_small_instances_share_launches(storage, gradient, pkg, oracle_mod):
+    """Small meshes of a batch, whose sweeps share launches, beside one that does not, against the same meshes stepped
+    one by one: the same arithmetic up to fused multiply-adds in FP32, one unit of 11 bits per rounding in FP16."""
+    shapes = [((9, 7, 5), 3), ((33, 1 + 16, 4), 4), ((64, 40, 21), 13), ((5, 6, 64), 1), ((17, 50, 33), 8), ((96, 90, 64), 16)]
+    problems = [random_problem(3, sh, S, seed=70 + k) for k, (sh, S) in enumerate(shapes)]
+    alone, together = [], []
+    for p in problems:
+        for out in (alone, together):
+            _, g = build_pair(pkg, oracle_mod, p)
+            g.set_storage(storage)
+            g.initialize()
+            g.store()
+            out.append(g)
+    batch = pkg.Batch(together)
+    for _ in range(3):
+        batch.timestep(True, gradient)
+        for g in alone:
+            g.timestep(True, gradient)
+    batch.wait()
+    for k, (g, h) in enumerate(zip(together, alone)):
+        g.load()
+        h.load()
+        if storage == "f32":
+            assert_close(g.densities, h.densities, what=f"instance {k}")
+        else:
+            # 3 steps of 5 roundings each on both sides (3 sweeps, the conversions)
+            err = np.linalg.norm(g.densities - h.densities) / np.linalg.norm(h.densities)
+            assert err <= 2 * 15 * 2.0**-10, (k, err)
+        if gradient and storage == "f32":
+            scale = np.abs(h.gradients).max()
+            assert np.abs(g.gradients - h.gradients).max() <= 4 * REL * max(scale, np.abs(h.densities).max())
+    batch.close()
