@@ -8,10 +8,9 @@
 //   u_j = d_j + mu u_{j-1},   x_j = s (u_j + mu x'_{j+1}),   s = (1 - mu)^2 / (1 + decay*dt/dims)
 // (x' without the factor s).  The same solution as the Thomas algorithm's (host/diffusion_solver.cpp:72-142,
 // 297-480), with constants instead of a table entry per element: 5 operations per element and no table reads.
-// Every term is positive for positive densities, so rounding errors do not amplify: against an FP64 solve of
-// uniform densities, n = 400, the FP32 relative L2 error is 0.4-1.3e-7 for a = 0.025..250, where the reference's
-// FP32 recurrence has 0.5e-7 at a = 0.025, 1.2e-7 at 2.5 and 3.7e-5 at 250 (its coefficients are rounded row by
-// row, here s is chosen from the rounded mu so that a constant field keeps its exact gain).
+// Every term is positive for positive densities, so rounding errors do not amplify, and s is chosen from the rounded mu so
+// that a constant field keeps its exact gain.  What the rounding of mu does cost is the distance over which a local
+// source decays: a relative error of up to 2^-25 / (mu |ln mu|) of it, which grows with a (filter_coefficients_ok).
 //
 // A line is split into blocks of m elements held in the registers of one lane each.  Per block: f = sum mu^{m-1-j}
 // d_j and e = sum mu^j d_j (the block's contribution to everything right and left of it), one two-sided scan of
@@ -817,8 +816,14 @@ static void by_block(int m, bool full, F&& f)
 	(one(std::integral_constant<int, Ms>()), ...);
 }
 
-// The filter needs 0 <= mu < 1, i.e. a >= 0 and 1 + decay*dt/dims > 0; mu is kept below 0.999 (a < 1e6), where the
-// FP32 error against an FP64 solve stays at 2e-7.
+// The filter needs 0 <= mu < 1, i.e. a >= 0 and 1 + decay*dt/dims > 0, and it is used up to mu = 0.73 (a = 10), where its
+// FP32 error against FP64 solves is still no larger than the partitioned sweep's.  Worst of 144 lines of 100, 400 and
+// 1000 voxels each (filter / partitioned), point source, relative L2 and per voxel above 1e-3 of the largest:
+//   a = 1..2.5    1.1e-7 / 1.3e-7  5.4e-7 / 7.0e-7        a = 16..25     1.8e-7 / 2.6e-7  1.3e-6 / 7.8e-7
+//   a = 6..10     1.4e-7 / 2.5e-7  9.2e-7 / 9.7e-7        a = 100..300   4.0e-7 / 3.7e-7  3.3e-6 / 7.1e-7
+//   a = 10..16    1.7e-7 / 2.5e-7  1.1e-6 / 8.8e-7        a = 1e3..1e5   3.2e-6 / 4.6e-7  1.7e-5 / 8.1e-7
+// (uniform random densities hide it: 2.0e-7 / 3.2e-7 at a = 1e3..1e5).
+static constexpr double filter_largest_mu = 0.73;
 static bool filter_coefficients_ok(const bfvm_ctx* ctx, int axis)
 {
 	const double h2 = (double)ctx->mesh.vs[axis] * ctx->mesh.vs[axis];
@@ -828,7 +833,7 @@ static bool filter_coefficients_ok(const bfvm_ctx* ctx, int axis)
 		const double lam = 1.0 + (double)ctx->decay[s] * ctx->mesh.dt / ctx->mesh.dims;
 		if (!(a >= 0.0) || !(lam > 0.0) || !std::isfinite(a) || !std::isfinite(lam))
 			return false;
-		if (!(2.0 * a / (lam + 2.0 * a + std::sqrt(lam * (lam + 4.0 * a))) <= 0.999))
+		if (!(2.0 * a / (lam + 2.0 * a + std::sqrt(lam * (lam + 4.0 * a))) <= filter_largest_mu))
 			return false;
 	}
 	return true;
