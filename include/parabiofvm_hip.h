@@ -208,14 +208,15 @@ int bfvm_set_gradient_order(bfvm_ctx* ctx, int32_t order);
  * recursive filter) and of the 3-D gradient (workgroups, rows per thread, workgroup order) on this context's mesh and keeps the fastest, as
  * bfvm_set_sweep_tuning / bfvm_set_sweep_workgroups / bfvm_set_gradient_tuning / bfvm_set_gradient_stacked /
  * bfvm_set_gradient_order would set them.  Results are cached per (axis, mesh
- * shape, substrate count, storage, algorithm) for the process, so a second context of the same shape tunes
- * at no cost.  The candidates run on a device copy of the densities: the densities are unchanged and the
+ * shape, substrate count, storage, algorithm, recursive filter or not) for the process, so a second context of the
+ * same shape tunes at no cost.  The candidates run on a device copy of the densities: the densities are unchanged and the
  * gradient buffer is recomputed from them.  Call after bfvm_initialize (and after bfvm_set_storage /
  * bfvm_set_sweep_algorithm have taken effect); synchronous. */
 int bfvm_autotune(bfvm_ctx* ctx);
 /* The process's tuning cache (bfvm_autotune and bfvm_batch_autotune results) written to / merged from a text
  * file, so that a later process starts tuned: with every shape of a context or batch in the cache, the
- * autotune calls apply the cached shapes without timing anything. */
+ * autotune calls apply the cached shapes without timing anything.  Entries of older files that shape the partitioned
+ * sweep are applied to axes that still take it, and older gradient and batch entries are kept but not applied. */
 int bfvm_tuning_save(const char* path);
 int bfvm_tuning_load(const char* path);
 

@@ -2,7 +2,8 @@
 // CUDA/diffusion_solver.cpp:11, 256-thread blocks in CUDA/diffusion_solver.cu:947-987); here the shapes of
 // every sweep axis (register chunk, lines per workgroup, workgroup count) and of the gradient (workgroups it
 // aims for) are picked by timing candidates on the context's own mesh, and cached per (axis, mesh shape,
-// substrate count, storage) for the process, so that contexts of the same shape tune once.  A batch's
+// substrate count, storage, whether the axis takes the recursive filter) for the process, so that contexts of the same
+// shape tune once.  A batch's
 // instances keep their own shapes.  The cache can be written to and read
 // from a text file, so that a later process starts tuned.
 #include <cstdio>
@@ -21,10 +22,13 @@ namespace {
 struct sweep_shape
 {
 	int chunk = 0, lines = 0, workgroups = 0;
+	// a shape of the recursive filter (its entries hold a workgroup cap only), or one of the partitioned sweep
+	bool filter() const { return chunk == 0 && lines == 0; }
 };
 
-using shape_key = std::tuple<int, int, int, int, int, int, int>; // axis (or -1: gradient), X, Y, Z, S, storage,
-																   // algorithm
+// axis (or -1: gradient), X, Y, Z, S, storage, algorithm, recursive filter.  Whether an axis takes the filter depends on
+// the coefficients too, and neither sweep's shape serves the other: a chunk asks for the partitioned sweep.
+using shape_key = std::tuple<int, int, int, int, int, int, int, bool>;
 
 std::mutex g_cache_mutex;
 std::map<shape_key, sweep_shape> g_sweep_cache;
@@ -35,12 +39,15 @@ struct gradient_shape
 	int order = 0;
 };
 std::map<shape_key, gradient_shape> g_gradient_cache;
+// "gradient" lines of files from before the branch-free gradient: they shaped its tiles, and would now put its marching
+// form where the automatic one is up to 2.6 times faster; read and written back, not used
+std::map<shape_key, gradient_shape> g_tile_gradients;
 std::map<std::string, bfvm_batch::tuning_t> g_batch_cache; // key: storage and every instance's shape
 
-shape_key key_of(const bfvm_ctx* ctx, int axis)
+shape_key key_of(const bfvm_ctx* ctx, int axis, bool filter)
 {
 	const auto& m = ctx->mesh;
-	return shape_key { axis, m.grid[0], m.grid[1], m.grid[2], m.S, ctx->storage, ctx->algorithm };
+	return shape_key { axis, m.grid[0], m.grid[1], m.grid[2], m.S, ctx->storage, ctx->algorithm, filter };
 }
 
 // Fastest of `reps` launches after one untimed launch, each timed alone with HIP events on `stream`.
@@ -97,8 +104,7 @@ void apply_sweep_shape(bfvm_ctx* ctx, int axis, const sweep_shape& s)
 // 0.79 / 0.85 and 0.55 / 0.49 / 0.52 ms, and on small meshes it is 2-5 times faster.
 sweep_shape search_sweep(bfvm_ctx* ctx, int axis, int reps)
 {
-	apply_sweep_shape(ctx, axis, sweep_shape {});
-	const bool filter = ctx->axes[axis].filter.blocks > 0;
+	const bool filter = ctx->axes[axis].filter.blocks > 0; // of the automatic shape, which the caller applied
 	std::vector<int> chunks = { 16, 32 };
 	if (ctx->storage == BFVM_STORAGE_F32)
 		chunks.push_back(64);
@@ -170,7 +176,10 @@ bool apply_cached_batch_tuning(bfvm_batch* b)
 
 // Text file, one entry per line:
 //   sweep <axis> <X> <Y> <Z> <S> <storage> <algorithm> <chunk> <lines> <workgroups>
-//   gradient <X> <Y> <Z> <S> <storage> <algorithm> <workgroups> <stacked> [<order>]
+//     (chunk and lines 0: a shape of the recursive filter, for axes that take it; else one of the partitioned sweep, for
+//     axes that do not)
+//   gradient_field <X> <Y> <Z> <S> <storage> <algorithm> <workgroups> <stacked> <order>
+//   gradient <X> <Y> <Z> <S> <storage> <algorithm> <workgroups> <stacked> [<order>], kept but not used
 //   batch <key> <18 numbers, kept but not used>
 void save_tuning(const char* path)
 {
@@ -181,9 +190,10 @@ void save_tuning(const char* path)
 	for (const auto& [k, v] : g_sweep_cache)
 		std::fprintf(f, "sweep %d %d %d %d %d %d %d %d %d %d\n", std::get<0>(k), std::get<1>(k), std::get<2>(k),
 					 std::get<3>(k), std::get<4>(k), std::get<5>(k), std::get<6>(k), v.chunk, v.lines, v.workgroups);
-	for (const auto& [k, v] : g_gradient_cache)
-		std::fprintf(f, "gradient %d %d %d %d %d %d %d %d %d\n", std::get<1>(k), std::get<2>(k), std::get<3>(k),
-					 std::get<4>(k), std::get<5>(k), std::get<6>(k), v.groups, v.stacked ? 1 : 0, v.order);
+	for (const auto& [name, cache] : { std::pair { "gradient", &g_tile_gradients }, { "gradient_field", &g_gradient_cache } })
+		for (const auto& [k, v] : *cache)
+			std::fprintf(f, "%s %d %d %d %d %d %d %d %d %d\n", name, std::get<1>(k), std::get<2>(k), std::get<3>(k),
+						 std::get<4>(k), std::get<5>(k), std::get<6>(k), v.groups, v.stacked ? 1 : 0, v.order);
 	for (const auto& [k, t] : g_batch_cache)
 	{
 		std::fprintf(f, "batch %s", k.c_str());
@@ -227,9 +237,9 @@ void load_tuning(const char* path)
 			sweep_shape v;
 			ok = static_cast<bool>(in >> axis >> X >> Y >> Z >> S >> st >> alg >> v.chunk >> v.lines >> v.workgroups);
 			if (ok)
-				g_sweep_cache[shape_key { axis, X, Y, Z, S, st, alg }] = v;
+				g_sweep_cache[shape_key { axis, X, Y, Z, S, st, alg, v.filter() }] = v;
 		}
-		else if (kind == "gradient")
+		else if (kind == "gradient" || kind == "gradient_field")
 		{
 			int X, Y, Z, S, st, alg, groups, stacked, order = 0;
 			ok = static_cast<bool>(in >> X >> Y >> Z >> S >> st >> alg >> groups >> stacked);
@@ -237,7 +247,8 @@ void load_tuning(const char* path)
 				order = 0;
 			ok = ok && (order == 0 || order == 1);
 			if (ok)
-				g_gradient_cache[shape_key { -1, X, Y, Z, S, st, alg }] = gradient_shape { groups, stacked != 0, order };
+				(kind == "gradient" ? g_tile_gradients : g_gradient_cache)[shape_key { -1, X, Y, Z, S, st, alg, false }] =
+					gradient_shape { groups, stacked != 0, order };
 		}
 		else if (kind == "batch")
 		{
@@ -262,7 +273,9 @@ void autotune_context(bfvm_ctx* ctx, bool tune_gradient)
 	{
 		if (ctx->mesh.grid[axis] == 1 || ctx->algorithm != BFVM_SWEEP_PARTITIONED)
 			continue;
-		const shape_key key = key_of(ctx, axis);
+		if (ctx->chunk_request[axis] != 0 || ctx->lines_request[axis] != 0)
+			apply_sweep_shape(ctx, axis, sweep_shape {});
+		const shape_key key = key_of(ctx, axis, ctx->axes[axis].filter.blocks > 0);
 		sweep_shape shape;
 		bool cached = false;
 		{
@@ -285,7 +298,7 @@ void autotune_context(bfvm_ctx* ctx, bool tune_gradient)
 	}
 	if (tune_gradient && ctx->mesh.dims == 3)
 	{
-		const shape_key key = key_of(ctx, -1);
+		const shape_key key = key_of(ctx, -1, false);
 		gradient_shape best;
 		bool cached = false;
 		{
