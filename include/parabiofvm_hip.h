@@ -213,9 +213,9 @@ int bfvm_set_gradient_order(bfvm_ctx* ctx, int32_t order);
  * gradient buffer is recomputed from them.  Call after bfvm_initialize (and after bfvm_set_storage /
  * bfvm_set_sweep_algorithm have taken effect); synchronous. */
 int bfvm_autotune(bfvm_ctx* ctx);
-/* The process's tuning cache (bfvm_autotune and bfvm_batch_autotune results) written to / merged from a text
- * file, so that a later process starts tuned: with every shape of a context or batch in the cache, the
- * autotune calls apply the cached shapes without timing anything.  Entries of older files that shape the partitioned
+/* The process's tuning cache (bfvm_autotune results) written to / merged from a text
+ * file, so that a later process starts tuned: with every shape of a context in the cache, the
+ * autotune call applies the cached shapes without timing anything.  Entries of older files that shape the partitioned
  * sweep are applied to axes that still take it, and older gradient and batch entries are kept but not applied. */
 int bfvm_tuning_save(const char* path);
 int bfvm_tuning_load(const char* path);
@@ -307,8 +307,8 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 int bfvm_batch_destroy(bfvm_batch* batch);
 int bfvm_batch_timestep(bfvm_batch* batch, int32_t recompute, int32_t with_gradient);
 int bfvm_batch_wait(bfvm_batch* batch);
-/* The batch's launches are shaped by rules and by each instance's own tuning: nothing is timed.  The gradients are
- * recomputed where the process's tuning cache has no entry for this list of shapes, and the entry is made. */
+/* The batch's launches are shaped by rules on sizes and by each instance's gradient tuning: nothing is timed.  The
+ * instances' densities are unchanged and their gradients are recomputed.  Synchronous. */
 int bfvm_batch_autotune(bfvm_batch* batch);
 /* Average ms per launch over all instances: BFVM_KERNEL_SWEEP_X/Y/Z and BFVM_KERNEL_GRADIENT (without the
  * launches around them), BFVM_PHASE_SECRETION(_RECOMPUTE), _DIFFUSION, _GRADIENT and _TIMESTEP. */

@@ -1437,7 +1437,7 @@ static void join_instance_streams(bfvm_batch* b)
 
 static uint64_t batch_epoch(const bfvm_batch* b)
 {
-	uint64_t e = b->epoch;
+	uint64_t e = 0;
 	for (const bfvm_ctx* c : b->ctx)
 		e += c->epoch;
 	return e;
@@ -1770,14 +1770,9 @@ int bfvm_batch_autotune(bfvm_batch* batch)
 		BFVM_HIP(hipSetDevice(batch->device));
 		join_instance_streams(batch);
 		BFVM_HIP(hipStreamSynchronize(batch->stream));
-		// the instances' launches are shaped by rules and by each context's own tuning: there is nothing to time
-		if (!apply_cached_batch_tuning(batch))
-		{
-			remember_batch_tuning(batch);
-			enqueue_batch_gradient(batch);
-		}
+		// the instances' launches are shaped by rules and by each context's own gradient tuning: nothing to time
+		enqueue_batch_gradient(batch);
 		BFVM_HIP(hipStreamSynchronize(batch->stream));
-		batch->epoch++;
 		return BFVM_OK;
 	});
 }

@@ -6,6 +6,7 @@
 // shape tune once.  A batch's
 // instances keep their own shapes.  The cache can be written to and read
 // from a text file, so that a later process starts tuned.
+#include <array>
 #include <cstdio>
 #include <map>
 #include <mutex>
@@ -42,7 +43,8 @@ std::map<shape_key, gradient_shape> g_gradient_cache;
 // "gradient" lines of files from before the branch-free gradient: they shaped its tiles, and would now put its marching
 // form where the automatic one is up to 2.6 times faster; read and written back, not used
 std::map<shape_key, gradient_shape> g_tile_gradients;
-std::map<std::string, bfvm_batch::tuning_t> g_batch_cache; // key: storage and every instance's shape
+// "batch" lines, from when batches had launch shapes of their own: read and written back, not used
+std::map<std::string, std::array<int, 18>> g_batch_lines;
 
 shape_key key_of(const bfvm_ctx* ctx, int axis, bool filter)
 {
@@ -152,27 +154,7 @@ sweep_shape search_sweep(bfvm_ctx* ctx, int axis, int reps)
 	return best;
 }
 
-std::string batch_key(const bfvm_batch* b)
-{
-	std::ostringstream k;
-	k << b->storage << ':' << b->ctx.size();
-	for (const bfvm_ctx* c : b->ctx)
-		k << ';' << c->mesh.grid[0] << ',' << c->mesh.grid[1] << ',' << c->mesh.grid[2] << ',' << c->mesh.S << ','
-		  << c->mesh.dims;
-	return k.str();
-}
-
 } // namespace
-
-bool apply_cached_batch_tuning(bfvm_batch* b)
-{
-	std::lock_guard<std::mutex> lock(g_cache_mutex);
-	auto it = g_batch_cache.find(batch_key(b));
-	if (it == g_batch_cache.end())
-		return false;
-	b->tuning = it->second;
-	return true;
-}
 
 // Text file, one entry per line:
 //   sweep <axis> <X> <Y> <Z> <S> <storage> <algorithm> <chunk> <lines> <workgroups>
@@ -180,7 +162,7 @@ bool apply_cached_batch_tuning(bfvm_batch* b)
 //     axes that do not)
 //   gradient_field <X> <Y> <Z> <S> <storage> <algorithm> <workgroups> <stacked> <order>
 //   gradient <X> <Y> <Z> <S> <storage> <algorithm> <workgroups> <stacked> [<order>], kept but not used
-//   batch <key> <18 numbers, kept but not used>
+//   batch <key> <18 numbers>, kept but not used
 void save_tuning(const char* path)
 {
 	std::lock_guard<std::mutex> lock(g_cache_mutex);
@@ -194,10 +176,10 @@ void save_tuning(const char* path)
 		for (const auto& [k, v] : *cache)
 			std::fprintf(f, "%s %d %d %d %d %d %d %d %d %d\n", name, std::get<1>(k), std::get<2>(k), std::get<3>(k),
 						 std::get<4>(k), std::get<5>(k), std::get<6>(k), v.groups, v.stacked ? 1 : 0, v.order);
-	for (const auto& [k, t] : g_batch_cache)
+	for (const auto& [k, fields] : g_batch_lines)
 	{
 		std::fprintf(f, "batch %s", k.c_str());
-		for (int v : t.fields)
+		for (int v : fields)
 			std::fprintf(f, " %d", v);
 		std::fprintf(f, "\n");
 	}
@@ -253,13 +235,13 @@ void load_tuning(const char* path)
 		else if (kind == "batch")
 		{
 			std::string key;
-			bfvm_batch::tuning_t t;
+			std::array<int, 18> fields {};
 			ok = static_cast<bool>(in >> key);
 			for (int i = 0; i < 18 && ok; i++)
-				ok = static_cast<bool>(in >> t.fields[i]);
-			ok = ok && (t.fields[14] == 4 || t.fields[14] == 8);
+				ok = static_cast<bool>(in >> fields[i]);
+			ok = ok && (fields[14] == 4 || fields[14] == 8);
 			if (ok)
-				g_batch_cache[key] = t;
+				g_batch_lines[key] = fields;
 		}
 		if (!ok)
 			throw std::invalid_argument(std::string(path) + ":" + std::to_string(lineno) + ": not a tuning entry");
@@ -338,12 +320,6 @@ void autotune_context(bfvm_ctx* ctx, bool tune_gradient)
 	}
 	BFVM_HIP(hipStreamSynchronize(ctx->stream));
 	ctx->epoch++;
-}
-
-void remember_batch_tuning(bfvm_batch* b)
-{
-	std::lock_guard<std::mutex> lock(g_cache_mutex);
-	g_batch_cache[batch_key(b)] = b->tuning;
 }
 
 } // namespace bfvm

@@ -534,12 +534,6 @@ struct bfvm_batch
 		bool batched = false;
 		uint64_t epoch = ~0ull;
 	} cell;
-	// the numbers of a batch's entry in a tuning file: kept, not used (the instances' own shapes apply)
-	struct tuning_t
-	{
-		int fields[18] = { 256, 256, 256, 256, 256, 256, 2048, 2048, 2048, 2048, 2048, 2048, 4, 8192, 4, 16, 0, 0 };
-	} tuning;
-	uint64_t epoch = 0;
 	bfvm::graph_slot graphs[4];
 };
 
@@ -593,10 +587,8 @@ constexpr int noalloc_max_points = 1 << 20;
 void setup_noalloc_scratch(int device); // with `device` current, once per device (bfvm_create)
 void voxel_positions_noalloc(bfvm_ctx* ctx, int count, const float* positions, int32_t* out3);
 
-// autotuner: time candidate launch shapes on the context's mesh / the batch and keep the fastest
+// autotuner: time candidate launch shapes on the context's mesh and keep the fastest
 void autotune_context(bfvm_ctx* ctx, bool tune_gradient);
-void remember_batch_tuning(bfvm_batch* b);
-bool apply_cached_batch_tuning(bfvm_batch* b); // false when this list of instance shapes has no cached tuning
 void save_tuning(const char* path);
 void load_tuning(const char* path);
 

@@ -313,7 +313,7 @@ class Batch:
         check("bfvm_batch_wait", self.lib.bfvm_batch_wait(self.h))
 
     def autotune(self):
-        """Time candidate work-list launch shapes of the batch's sweeps and gradient and keep the fastest."""
+        """Nothing to time (rules on sizes and the solvers' gradient tuning shape the launches); recomputes the gradients."""
         check("bfvm_batch_autotune", self.lib.bfvm_batch_autotune(self.h))
 
     def benchmark(self, what, iterations):

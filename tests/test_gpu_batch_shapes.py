@@ -1,0 +1,76 @@
+"""Launch shapes within a batch, on an MI355X: an instance's gradient shape is its context's; the batch's autotuner times
+nothing and recomputes the gradients."""
+import numpy as np
+import pytest
+
+from test_gpu_batch import check_gradients_of_stored
+from test_gpu_parity import build_pair, random_problem
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [((20, 12, 9), 4), ((11, 10, 8), 3), ((9, 14, 7), 8), ((13, 6, 10), 5), ((40, 33, 26), 12)]
+
+
+@pytest.fixture(scope="module")
+def pkg():
+    import parabiofvm_amd
+
+    parabiofvm_amd.load()
+    return parabiofvm_amd
+
+
+def solvers_of(pkg, oracle_mod, storage="f32", shapes=SHAPES):
+    out = []
+    for k, (shape, S) in enumerate(shapes):
+        _, g = build_pair(pkg, oracle_mod, random_problem(3, shape, S, seed=500 + k))
+        g.set_storage(storage)
+        g.initialize()
+        g.store()
+        out.append(g)
+    return out
+
+
+def configs_of(solvers, shapes=SHAPES):
+    return [{"grid": shape, "S": S, "voxel_shape": g.voxel_shape} for g, (shape, S) in zip(solvers, shapes)]
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+@pytest.mark.parametrize("stacked", [False, True])
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("groups", [0, 4096])
+def test_gradient_shapes_of_the_contexts(groups, order, stacked, storage, pkg, oracle_mod):
+    """4 and 8 rows per thread, both workgroup orders, chunks of the z planes by a workgroup count: each instance's
+    gradient is that of its densities as stored."""
+    solvers = solvers_of(pkg, oracle_mod, storage)
+    for g in solvers:
+        g.set_gradient_tuning(groups)
+        g.set_gradient_stacked(stacked)
+        g.set_gradient_order(order)
+    batch = pkg.Batch(solvers)
+    batch.timestep(True, True)
+    batch.timestep(False, True)
+    batch.wait()
+    for g in solvers:
+        g.load()
+    check_gradients_of_stored(configs_of(solvers), solvers, f"groups {groups} stacked {stacked} order {order} {storage}")
+    batch.close()
+    for g in solvers:
+        g.close()
+
+
+def test_autotune_recomputes_the_gradients_each_time(pkg, oracle_mod):
+    solvers = solvers_of(pkg, oracle_mod)
+    batch = pkg.Batch(solvers)
+    for step in range(2):
+        batch.timestep(step == 0, False)
+        batch.wait()
+        for g in solvers:
+            g.load()
+        before = [g.densities.copy() for g in solvers]
+        batch.autotune()
+        for g, d in zip(solvers, before):
+            g.gradients[:] = np.nan
+            g.load()
+            np.testing.assert_array_equal(g.densities.view(np.uint32), d.view(np.uint32))
+        check_gradients_of_stored(configs_of(solvers), solvers, f"autotune after step {step}")
+    batch.close()
