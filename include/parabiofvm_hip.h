@@ -295,8 +295,10 @@ int bfvm_benchmark(bfvm_ctx* ctx, int32_t what, int32_t iterations, float* avg_m
  * every other instance's sweeps and gradient as a chain on one of the graph's branches.  Per-instance results equal
  * what bfvm_timestep gives for that context to the sweep's tolerance (the same algorithm).
  *
- * All contexts must be initialized on one device with one storage form and the partitioned sweep; they
- * keep their data (store/load through the per-context calls).  A context re-initialized while the batch
+ * All contexts must be initialized on one device with one storage form, none with the exact sweep; they
+ * keep their data (store/load through the per-context calls).  The batch's sweeps have their own automatic shapes: a
+ * context's sweep algorithm, its sweep tuning and its workgroup cap do not change them, whenever they are set.  A
+ * context's gradient tuning does shape its gradients.  A context re-initialized while the batch
  * exists makes the batch's next step fail with BFVM_ERR_STATE; bfvm_destroy refuses a context that belongs to
  * a batch.  The batch has its own stream, ordered with the contexts' streams both ways: every context call
  * that touches device data first waits for the steps of its batches, and a batch step first waits for work

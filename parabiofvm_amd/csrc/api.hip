@@ -1364,23 +1364,43 @@ int bfvm_benchmark(bfvm_ctx* ctx, int32_t what, int32_t iterations, float* avg_m
 
 namespace bfvm {
 
-// The per-instance kernels of a batch step run on one of the batch's streams with the batch's rounding counter.
+// The per-instance kernels of a batch step run on one of the batch's streams with the batch's rounding counter and
+// sweep tables.
 struct batch_override
 {
-	bfvm_ctx* c;
+	bfvm_batch* b;
+	size_t at;
 	hipStream_t stream;
 	unsigned* rounding;
-	batch_override(bfvm_ctx* ctx, const bfvm_batch* b, hipStream_t on)
-		: c(ctx), stream(ctx->stream), rounding(ctx->rounding_step)
+	int algorithm;
+	int workgroups[3];
+	bfvm_ctx* ctx() const { return b->ctx[at]; }
+	batch_override(bfvm_batch* batch, size_t instance, hipStream_t on)
+		: b(batch), at(instance), stream(ctx()->stream), rounding(ctx()->rounding_step), algorithm(ctx()->algorithm)
 	{
-		c->stream = on;
-		c->rounding_step = b->rounding;
+		ctx()->stream = on;
+		ctx()->rounding_step = b->rounding;
+		ctx()->algorithm = BFVM_SWEEP_PARTITIONED;
+		for (int a = 0; a < 3; a++)
+		{
+			workgroups[a] = ctx()->sweep_workgroups[a];
+			ctx()->sweep_workgroups[a] = 0;
+			std::swap(ctx()->axes[a], b->axes[at][a]);
+		}
 	}
 	~batch_override()
 	{
-		c->stream = stream;
-		c->rounding_step = rounding;
+		ctx()->stream = stream;
+		ctx()->rounding_step = rounding;
+		ctx()->algorithm = algorithm;
+		for (int a = 0; a < 3; a++)
+		{
+			ctx()->sweep_workgroups[a] = workgroups[a];
+			std::swap(ctx()->axes[a], b->axes[at][a]);
+		}
 	}
+	batch_override(const batch_override&) = delete;
+	batch_override& operator=(const batch_override&) = delete;
 };
 
 static void free_batch_small(bfvm_batch* b);
@@ -1396,6 +1416,12 @@ static void free_batch(bfvm_batch* b)
 	}
 	free_batch_cell(b);
 	free_batch_small(b);
+	for (const auto& axes : b->axes)
+		for (const auto& t : axes)
+			for (float* p : { t.filter_tab, t.coef, t.red, t.A })
+				if (p)
+					(void)hipFree(p);
+	b->axes.clear();
 	for (int i = 0; i < bfvm_batch::branches; i++)
 	{
 		if (b->branch_event[i])
@@ -1462,7 +1488,7 @@ static void on_branches(bfvm_batch* b, G&& first, F&& one)
 		first();
 		for (size_t i = 0; i < b->ctx.size(); i++)
 		{
-			batch_override o(b->ctx[i], b, b->branch_stream[b->branch_of[i]]);
+			batch_override o(b, i, b->branch_stream[b->branch_of[i]]);
 			one(b->ctx[i], b->small.count > 0 && b->small.member[i]);
 		}
 	}
@@ -1506,7 +1532,7 @@ static void refresh_batch_small(bfvm_batch* b, uint64_t epoch)
 		{
 			if (!sp.member[i] || axis >= b->ctx[i]->mesh.dims)
 				continue;
-			batch_override o(b->ctx[i], b, b->stream);
+			batch_override o(b, i, b->stream);
 			int tasks = 0, lds = 0;
 			args.resize(args.size() + each);
 			small_filter_args(b->ctx[i], axis, args.data() + args.size() - each, tasks, lds);
@@ -1547,7 +1573,7 @@ static void on_small(bfvm_batch* b, F&& f)
 	for (size_t i = 0; i < b->ctx.size(); i++)
 		if (b->small.member[i])
 		{
-			batch_override o(b->ctx[i], b, b->stream);
+			batch_override o(b, i, b->stream);
 			f(b->ctx[i]);
 		}
 }
@@ -1564,7 +1590,7 @@ static void enqueue_batch_sweeps(bfvm_batch* b, bool with_gradient = false)
 {
 	if (b->storage != BFVM_STORAGE_F32)
 	{
-		batch_override o(b->ctx[0], b, b->stream);
+		batch_override o(b, 0, b->stream);
 		launch_advance_rounding(b->ctx[0]);
 	}
 	on_branches(
@@ -1612,10 +1638,10 @@ static void enqueue_batch_cell(bfvm_batch* b, bool recompute)
 		launch_batched_cell(b, recompute);
 		return;
 	}
-	for (bfvm_ctx* c : b->ctx)
+	for (size_t i = 0; i < b->ctx.size(); i++)
 	{
-		batch_override o(c, b, b->stream);
-		launch_cell(c, recompute);
+		batch_override o(b, i, b->stream);
+		launch_cell(b->ctx[i], recompute);
 	}
 }
 
@@ -1664,10 +1690,16 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 			BFVM_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
 			BFVM_HIP(hipMalloc(&b->rounding, sizeof(unsigned)));
 			BFVM_HIP(hipMemsetAsync(b->rounding, 0, sizeof(unsigned), b->stream));
+			b->axes.resize(count);
 			for (int32_t i = 0; i < count; i++)
 				for (int a = 0; a < b->ctx[i]->mesh.dims; a++)
+				{
 					if (b->ctx[i]->mesh.grid[a] > 1)
 						check_batch_axis(b->ctx[i], a, i);
+					build_batch_axis(b->ctx[i], a, b->axes[i][a]);
+					batch_override o(b, i, b->stream);
+					launch_partition_coefficients(b->ctx[i], a);
+				}
 			b->branch_stream[0] = b->stream;
 			for (int i = 0; i < bfvm_batch::branches; i++)
 			{

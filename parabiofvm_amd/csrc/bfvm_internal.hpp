@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <algorithm>
+#include <array>
 #include <cstdio>
 #include <string>
 #include <type_traits>
@@ -510,6 +511,9 @@ struct bfvm_batch
 	hipStream_t branch_stream[branches] = {}; // [0] is `stream`
 	hipEvent_t branch_event[branches] = {};   // [0]: the fork
 	std::vector<int> branch_of;				 // per instance
+	// per instance and axis the batch's own sweep tables, so that a context's sweep algorithm and tuning, which may change
+	// while the batch exists, leave the batch as it is
+	std::vector<std::array<bfvm::axis_tables, 3>> axes;
 	// instances whose sweeps share one launch per axis, and per axis their arguments and running task counts on the
 	// device, rebuilt with the batch's epoch
 	struct small_plan
@@ -569,6 +573,7 @@ void launch_voxel_positions(bfvm_ctx* ctx, int count, const float* d_pos, int* d
 
 filter_plan choose_filter(const bfvm_ctx* ctx, int axis);
 void check_batch_axis(const bfvm_ctx* ctx, int axis, int instance);
+void build_batch_axis(bfvm_ctx* ctx, int axis, axis_tables& t);
 size_t filter_table_floats(const filter_plan& p, int S);
 void launch_filter_coefficients(const bfvm_ctx* ctx, int axis, const filter_plan& p, float* tab, hipStream_t stream);
 void launch_filter_sweep(bfvm_ctx* ctx, int axis);

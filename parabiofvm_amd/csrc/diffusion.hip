@@ -1397,6 +1397,22 @@ void alloc_partition_tables(const partition& p, int S, float*& coef, float*& red
 	BFVM_HIP(hipMalloc(&A, sizeof(float) * S));
 }
 
+// The recursive filter's plan and its table's memory; false where the axis does not take it
+static bool build_filter(const bfvm_ctx* ctx, int axis, axis_tables& t)
+{
+	const filter_plan p = choose_filter(ctx, axis);
+	if (p.blocks == 0)
+		return false;
+	t.filter = p;
+	t.part.n = ctx->mesh.grid[axis];
+	t.part.P = p.blocks;
+	t.part.base = t.part.n / p.blocks;
+	t.part.rem = p.m > t.part.base ? 1 : 0;
+	t.part.lpg = p.lines_group;
+	BFVM_HIP(hipMalloc(&t.filter_tab, sizeof(float) * filter_table_floats(p, ctx->mesh.S)));
+	return true;
+}
+
 void build_partition(bfvm_ctx* ctx, int axis, int chunk, int lines_request)
 {
 	auto& t = ctx->axes[axis];
@@ -1408,22 +1424,32 @@ void build_partition(bfvm_ctx* ctx, int axis, int chunk, int lines_request)
 	if (lines_request == 0 && axis == 2 && ctx->storage != BFVM_STORAGE_F32 && !staged)
 		lines_request = 8;
 	t.part = choose_partition(ctx, axis, staged ? batch_chunk : chunk, lines_request, staged ? 1 : 4);
-	if (automatic && t.part.P > 0)
-	{
-		const filter_plan p = choose_filter(ctx, axis);
-		if (p.blocks > 0)
-		{
-			t.filter = p;
-			t.part.P = p.blocks;
-			t.part.base = t.part.n / p.blocks;
-			t.part.rem = p.m > t.part.base ? 1 : 0;
-			t.part.lpg = p.lines_group;
-			BFVM_HIP(hipMalloc(&t.filter_tab, sizeof(float) * filter_table_floats(p, ctx->mesh.S)));
-			return;
-		}
-	}
+	if (automatic && t.part.P > 0 && build_filter(ctx, axis, t))
+		return;
 	if (t.part.P > 0)
 		alloc_partition_tables(t.part, ctx->mesh.S, t.coef, t.red, t.A);
+}
+
+// The tables of one axis of an instance for a batch, shaped by rules on sizes and coefficients alone: the recursive
+// filter where the axis takes it, else the partitioned sweep's automatic shape, else the smallest groups of 16-element
+// blocks, which check_batch_axis has seen to fit.
+void build_batch_axis(bfvm_ctx* ctx, int axis, axis_tables& t)
+{
+	t = axis_tables {};
+	t.n = ctx->axes[axis].n;
+	t.exact_b = ctx->axes[axis].exact_b; // the context's: an axis of one voxel divides by it
+	if (ctx->mesh.grid[axis] == 1 || build_filter(ctx, axis, t))
+		return;
+	const int lines = axis == 2 && ctx->storage != BFVM_STORAGE_F32 ? 8 : 0;
+	try
+	{
+		t.part = choose_partition(ctx, axis, 0, lines, 4);
+	}
+	catch (const std::runtime_error&)
+	{
+		t.part = choose_partition(ctx, axis, batch_chunk, 1, 1);
+	}
+	alloc_partition_tables(t.part, ctx->mesh.S, t.coef, t.red, t.A);
 }
 
 void launch_partition_tables(const bfvm_ctx* ctx, int axis, const partition& p, float* coef, float* red, float* A,

@@ -1,5 +1,5 @@
-"""Launch shapes within a batch, on an MI355X: an instance's gradient shape is its context's; the batch's autotuner times
-nothing and recomputes the gradients."""
+"""Launch shapes within a batch, on an MI355X: sweeps are shaped by the batch, whatever the contexts ask for; an
+instance's gradient shape is its context's; the batch's autotuner times nothing and recomputes the gradients."""
 import numpy as np
 import pytest
 
@@ -74,3 +74,47 @@ def test_autotune_recomputes_the_gradients_each_time(pkg, oracle_mod):
             np.testing.assert_array_equal(g.densities.view(np.uint32), d.view(np.uint32))
         check_gradients_of_stored(configs_of(solvers), solvers, f"autotune after step {step}")
     batch.close()
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+@pytest.mark.parametrize("setting", ["staged before", "staged", "exact", "chunk", "tuning", "workgroups"])
+def test_sweeps_do_not_follow_the_contexts(setting, storage, pkg, oracle_mod):
+    """Sweep algorithms, block lengths and workgroup caps that are set on the contexts, before the batch is made or
+    while it exists, leave its results as they are, bit for bit (the densities of meshes without agents are the same
+    from run to run)."""
+    shapes = SHAPES + [((60, 50, 40), 4), ((18, 1, 33), 8)]
+
+    def change(g):
+        if "staged" in setting:
+            g.set_sweep_algorithm(pkg.BFVM_SWEEP_STAGED)
+        elif setting == "exact":
+            g.set_sweep_algorithm(pkg.BFVM_SWEEP_EXACT)
+        elif setting == "chunk":
+            g.set_sweep_algorithm(pkg.BFVM_SWEEP_PARTITIONED, 32)
+        elif setting == "tuning":
+            for axis in range(3):
+                g.set_sweep_tuning(axis, 16, 8)
+        else:
+            g.set_sweep_workgroups(3)
+
+    results = []
+    for changed in (False, True):
+        solvers = solvers_of(pkg, oracle_mod, storage, shapes)
+        if changed and setting != "exact" and setting != "staged":
+            for g in solvers:
+                change(g)
+        batch = pkg.Batch(solvers)
+        batch.timestep(False, False)
+        if changed and setting in ("exact", "staged"):
+            for g in solvers:
+                change(g)
+        batch.timestep(False, False)
+        batch.wait()
+        for g in solvers:
+            g.load()
+        results.append([g.densities.copy() for g in solvers])
+        batch.close()
+        for g in solvers:
+            g.close()
+    for k, (a, b) in enumerate(zip(*results)):
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32), err_msg=f"instance {k} {shapes[k]}")
