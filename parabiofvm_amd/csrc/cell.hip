@@ -4,8 +4,8 @@
 //   D  <- (D + sum num) / (1 + sum den) + sum fac                        (per voxel)
 //   I  -= vv*((-den*D + num)/(1 + den) + fac)                            (per agent, old D)
 //
-// Same-voxel contributions are combined per recompute by a claim ("ballot") per voxel: the first agent
-// to compare-and-swap the voxel's ballot from -1 wins and every agent adds its terms into the winner's
+// Same-voxel contributions are combined per recompute by a claim ("ballot") per voxel: every agent stores its index in
+// its voxel's ballot, the one whose store stays wins, and every agent adds its terms into the winner's
 // reduced slot with float atomics (the winner adds den + 1).  A device flag records whether any voxel had
 // a second agent; it selects, on the device, between the fused per-agent update (no conflict) and the
 // two-phase update (internalized with the old D for every agent, then the winners update D) — the same
@@ -58,12 +58,13 @@ __global__ __launch_bounds__(256) void cell_voxels_kernel(cell_geom g, int A, co
 		vox[i] = agent_voxel(g, pos, i);
 }
 
-// Recompute, claim scheme: reset, ballot, prepare, sum.  1M clustered agents x 8 substrates on 200^3, all phases with
-// the apply: 405 -> 276 us.  Winners are known before the terms are formed, so a winner's slot starts with its own
-// terms and only the other agents add with atomics (sum 120 -> 72 us).
+// Recompute, claim scheme: claim, prepare, sum; small recomputes are bound by the number of launches.  Winners are known
+// before the terms are formed, so a winner's slot starts with its own terms and only the other agents add with atomics.
 //
-// part 1: ballots of the agents' voxels back to unclaimed, no conflict yet
-__device__ __forceinline__ void cell_reset_at(int64_t i, int A, const int64_t* __restrict__ vox,
+// part 1 (host/cell_solver.cpp:98-122): claim the voxels, no conflict yet.  Any agent of a voxel may win, so plain stores
+// do; which one stayed is read after the kernel's end.  They need no earlier launch that resets the ballots, and a
+// compare-and-swap per agent is the slower scatter.
+__device__ __forceinline__ void cell_claim_at(int64_t i, int A, const int64_t* __restrict__ vox,
 											  int* __restrict__ ballots, int* __restrict__ conflict)
 {
 	if (i == 0)
@@ -72,13 +73,13 @@ __device__ __forceinline__ void cell_reset_at(int64_t i, int A, const int64_t* _
 		return;
 	const int64_t v = vox[i];
 	if (v >= 0)
-		ballots[v] = -1;
+		__hip_atomic_store(&ballots[v], (int)i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(256) void cell_reset_kernel(int A, const int64_t* __restrict__ vox,
+__global__ __launch_bounds__(256) void cell_claim_kernel(int A, const int64_t* __restrict__ vox,
 														 int* __restrict__ ballots, int* __restrict__ conflict)
 {
-	cell_reset_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, vox, ballots, conflict);
+	cell_claim_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, vox, ballots, conflict);
 }
 
 // *flag = 1 when `cond` holds for an active lane of the wave: at most one store per wave, and none once the wave sees
@@ -90,32 +91,6 @@ __device__ __forceinline__ void flag_any(int* flag, bool cond)
 	if (cond && (unsigned)__lane_id() == (unsigned)(__ffsll((long long)m) - 1) &&
 		__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
 		__hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// part 2 (host/cell_solver.cpp:98-122): claim the voxel; win[i] = the agent whose slot collects i
-__device__ __forceinline__ void cell_ballot_at(int64_t i, int A, const int64_t* __restrict__ vox,
-														  int* __restrict__ ballots, int* __restrict__ win,
-														  int* __restrict__ conflict)
-{
-	if (i >= A)
-		return;
-	const int64_t v = vox[i];
-	if (v < 0)
-	{
-		win[i] = -1;
-		return;
-	}
-	// (loading the ballot first and claiming only unclaimed voxels: 102 -> 151 us for 1M crowded agents)
-	const int prev = atomicCAS(&ballots[v], -1, (int)i);
-	win[i] = prev == -1 ? (int)i : prev;
-	flag_any(conflict, prev != -1);
-}
-
-__global__ __launch_bounds__(256) void cell_ballot_kernel(int A, const int64_t* __restrict__ vox,
-														  int* __restrict__ ballots, int* __restrict__ win,
-														  int* __restrict__ conflict)
-{
-	cell_ballot_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, vox, ballots, win, conflict);
 }
 
 // The terms of one agent and substrate (host/cell_solver.cpp:35-85)
@@ -133,10 +108,12 @@ __device__ __forceinline__ cell_terms make_terms(int64_t i, int64_t k, float vox
 			 nex[k] * dt / voxel_volume };
 }
 
-// part 3 (host/cell_solver.cpp:35-85): the terms per (agent, s), and the reduced slot: a winner's own terms, with
-// den + 1, else 0
+// part 2 (host/cell_solver.cpp:35-85): the terms per (agent, s), the agent whose slot collects them (win), and the reduced
+// slot: a winner's own terms, with den + 1, else 0
 __device__ __forceinline__ void cell_prepare_at(int64_t k, int A, int S, float voxel_volume, float dt,
-														   const int* __restrict__ win,
+														   const int64_t* __restrict__ vox,
+														   const int* __restrict__ ballots, int* __restrict__ win,
+														   int* __restrict__ conflict,
 														   const float* __restrict__ vol, const float* __restrict__ sec,
 														   const float* __restrict__ sat, const float* __restrict__ upt,
 														   const float* __restrict__ nex, float* __restrict__ num,
@@ -147,18 +124,25 @@ __device__ __forceinline__ void cell_prepare_at(int64_t k, int A, int S, float v
 	if (k >= (int64_t)A * S)
 		return;
 	const int64_t i = k / S;
+	const int64_t v = vox[i];
 	const cell_terms t = make_terms(i, k, voxel_volume, dt, vol, sec, sat, upt, nex);
-	const bool won = win[i] == (int)i;
+	const int w = v < 0 ? -1 : ballots[v];
+	const bool won = w == (int)i;
+	if (k == i * S)
+		win[i] = w;
 	num[k] = t.num;
 	den[k] = t.den;
 	fac[k] = t.fac;
 	rnum[k] = won ? t.num : 0.f;
 	rden[k] = won ? t.den + 1 : 0.f;
 	rfac[k] = won ? t.fac : 0.f;
+	flag_any(conflict, v >= 0 && !won);
 }
 
 __global__ __launch_bounds__(256) void cell_prepare_kernel(int A, int S, float voxel_volume, float dt,
-														   const int* __restrict__ win,
+														   const int64_t* __restrict__ vox,
+														   const int* __restrict__ ballots, int* __restrict__ win,
+														   int* __restrict__ conflict,
 														   const float* __restrict__ vol, const float* __restrict__ sec,
 														   const float* __restrict__ sat, const float* __restrict__ upt,
 														   const float* __restrict__ nex, float* __restrict__ num,
@@ -166,11 +150,11 @@ __global__ __launch_bounds__(256) void cell_prepare_kernel(int A, int S, float v
 														   float* __restrict__ rnum, float* __restrict__ rden,
 														   float* __restrict__ rfac)
 {
-	cell_prepare_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, S, voxel_volume, dt, win, vol, sec, sat, upt,
-					nex, num, den, fac, rnum, rden, rfac);
+	cell_prepare_at((int64_t)blockIdx.x * blockDim.x + threadIdx.x, A, S, voxel_volume, dt, vox, ballots, win, conflict,
+					vol, sec, sat, upt, nex, num, den, fac, rnum, rden, rfac);
 }
 
-// part 4 (host/cell_solver.cpp:108-133): every other (agent, s) adds into its winner's slot
+// part 3 (host/cell_solver.cpp:108-133): every other (agent, s) adds into its winner's slot
 __device__ __forceinline__ void cell_sum_at(int64_t k, int A, int S, const int* __restrict__ win,
 													   const float* __restrict__ num, const float* __restrict__ den,
 													   const float* __restrict__ fac, float* __restrict__ rnum,
@@ -421,8 +405,7 @@ __global__ __launch_bounds__(256) void cell_densities_kernel(int A, int S, int w
 // elements, as the single-instance kernels do.
 enum cell_phase
 {
-	phase_reset,
-	phase_ballot,
+	phase_claim,
 	phase_prepare,
 	phase_sum,
 	phase_apply,
@@ -440,13 +423,11 @@ __global__ __launch_bounds__(256) void cell_batched_kernel(const cell_args* __re
 		for (int64_t blk = w.begin; blk < w.end; blk++)
 		{
 			const int64_t k = blk * blockDim.x + threadIdx.x;
-			if constexpr (PHASE == phase_reset)
-				cell_reset_at(k, c.A, c.vox, c.ballots, c.conflict);
-			else if constexpr (PHASE == phase_ballot)
-				cell_ballot_at(k, c.A, c.vox, c.ballots, c.win, c.conflict);
+			if constexpr (PHASE == phase_claim)
+				cell_claim_at(k, c.A, c.vox, c.ballots, c.conflict);
 			else if constexpr (PHASE == phase_prepare)
-				cell_prepare_at(k, c.A, c.S, (float)c.voxel_volume, c.dt, c.win, c.vol, c.sec, c.sat, c.upt, c.nex, c.num,
-								c.den, c.fac, c.rnum, c.rden, c.rfac);
+				cell_prepare_at(k, c.A, c.S, (float)c.voxel_volume, c.dt, c.vox, c.ballots, c.win, c.conflict, c.vol, c.sec,
+								c.sat, c.upt, c.nex, c.num, c.den, c.fac, c.rnum, c.rden, c.rfac);
 			else if constexpr (PHASE == phase_sum)
 				cell_sum_at(k, c.A, c.S, c.win, c.num, c.den, c.fac, c.rnum, c.rden, c.rfac);
 			else if constexpr (PHASE == phase_apply)
@@ -582,17 +563,14 @@ void launch_cell(bfvm_ctx* ctx, bool recompute)
 	else if (recompute)
 	{
 		// at least one block so the conflict flag is cleared even without agents
-		hipLaunchKernelGGL(cell_reset_kernel, dim3(std::max(agent_blocks, 1u)), dim3(256), 0, ctx->stream, A, a.vox,
+		hipLaunchKernelGGL(cell_claim_kernel, dim3(std::max(agent_blocks, 1u)), dim3(256), 0, ctx->stream, A, a.vox,
 						   ctx->ballots, ctx->conflict);
 		BFVM_HIP(hipGetLastError());
 		if (A > 0)
 		{
-			hipLaunchKernelGGL(cell_ballot_kernel, dim3(agent_blocks), dim3(256), 0, ctx->stream, A, a.vox,
-							   ctx->ballots, a.win, ctx->conflict);
-			BFVM_HIP(hipGetLastError());
 			hipLaunchKernelGGL(cell_prepare_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S,
-							   (float)voxel_volume(ctx), ctx->mesh.dt, a.win, a.vol, a.sec, a.sat, a.upt, a.nex, a.num,
-							   a.den, a.fac, a.rnum, a.rden, a.rfac);
+							   (float)voxel_volume(ctx), ctx->mesh.dt, a.vox, ctx->ballots, a.win, ctx->conflict, a.vol,
+							   a.sec, a.sat, a.upt, a.nex, a.num, a.den, a.fac, a.rnum, a.rden, a.rfac);
 			BFVM_HIP(hipGetLastError());
 			hipLaunchKernelGGL(cell_sum_kernel, dim3(pair_blocks), dim3(256), 0, ctx->stream, A, S, a.win, a.num,
 							   a.den, a.fac, a.rnum, a.rden, a.rfac);
@@ -722,7 +700,7 @@ static void launch_cell_phase(bfvm_batch* b, const batch_item* items, int n)
 	BFVM_HIP(hipGetLastError());
 }
 
-// The secretion of every instance of a refreshed, batched plan: recompute (reset, ballot, prepare, sum) and apply
+// The secretion of every instance of a refreshed, batched plan: recompute (claim, prepare, sum) and apply
 // (apply, densities), one launch per phase, in the order of launch_cell.
 void launch_batched_cell(bfvm_batch* b, bool recompute)
 {
@@ -731,8 +709,7 @@ void launch_batched_cell(bfvm_batch* b, bool recompute)
 		constexpr int K = decltype(kind)::value;
 		if (recompute)
 		{
-			launch_cell_phase<K, phase_reset>(b, cp.agent_items, cp.nagent);
-			launch_cell_phase<K, phase_ballot>(b, cp.agent_items, cp.nagent);
+			launch_cell_phase<K, phase_claim>(b, cp.agent_items, cp.nagent);
 			launch_cell_phase<K, phase_prepare>(b, cp.pair_items, cp.npair);
 			launch_cell_phase<K, phase_sum>(b, cp.pair_items, cp.npair);
 		}
