@@ -1469,15 +1469,10 @@ static uint64_t batch_epoch(const bfvm_batch* b)
 	return e;
 }
 
-// one(instance, small) for every instance, its launches on its branch: a step's launches of one instance follow each other
-// on a branch, so the ends of one instance's kernels are covered by the other branches', and an instance of ordinary
-// size stays in the Infinity Cache from one axis to the next.  The branches are forked from the batch's stream and
-// joined to it, also when a launch is refused.  One launch per axis over all instances (workgroups walking a list of
-// line groups) took, for a step without gradient of 64 instances in 16-bit storage, 3.84 ms; branches 2.96 ms.
-// `first` runs on the batch's stream, beside the other branches; one's second argument: whether the instance is among
-// those that share sweep launches.
-template <typename G, typename F>
-static void on_branches(bfvm_batch* b, G&& first, F&& one)
+// f(instance) for every instance that `with` takes, its launches on its branch.  The branches are forked from the batch's
+// stream and joined to it, also when a launch is refused.  `first` runs on the batch's stream, beside the other branches.
+template <typename G, typename W, typename F>
+static void on_branches(bfvm_batch* b, G&& first, W&& with, F&& f)
 {
 	BFVM_HIP(hipEventRecord(b->branch_event[0], b->stream));
 	for (int i = 1; i < bfvm_batch::branches; i++)
@@ -1487,10 +1482,11 @@ static void on_branches(bfvm_batch* b, G&& first, F&& one)
 	{
 		first();
 		for (size_t i = 0; i < b->ctx.size(); i++)
-		{
-			batch_override o(b, i, b->branch_stream[b->branch_of[i]]);
-			one(b->ctx[i], b->small.count > 0 && b->small.member[i]);
-		}
+			if (with(i))
+			{
+				batch_override o(b, i, b->branch_stream[b->branch_of[i]]);
+				f(b->ctx[i]);
+			}
 	}
 	catch (...)
 	{
@@ -1513,15 +1509,6 @@ static void refresh_batch_small(bfvm_batch* b, uint64_t epoch)
 	if (sp.epoch == epoch)
 		return;
 	BFVM_HIP(hipStreamSynchronize(b->stream));
-	sp.member.assign(b->ctx.size(), 0);
-	sp.count = 0;
-	for (size_t i = 0; i < b->ctx.size(); i++)
-		sp.count += sp.member[i] = small_filter(b->ctx[i]) ? 1 : 0;
-	if (sp.count < 2)
-	{
-		sp.member.assign(b->ctx.size(), 0);
-		sp.count = 0;
-	}
 	const size_t each = small_filter_args_bytes();
 	for (int axis = 0; axis < 3; axis++)
 	{
@@ -1586,6 +1573,12 @@ static void launch_small_axis(bfvm_batch* b, int axis)
 							 sp.lds[axis]);
 }
 
+// The small instances' sweeps, one launch per axis, and gradients on the batch's stream; every other instance's on its
+// branch: its launches follow each other, so the ends of one instance's kernels are covered by the other branches', and an
+// instance of ordinary size stays in the Infinity Cache from one axis to the next.  One launch per axis over all
+// instances (workgroups walking a list of line groups) took, for a step without gradient of 64 instances in 16-bit
+// storage, 3.84 ms; branches 2.96 ms.  (The small ones' gradients spread over the branches: 10 instances of 32..96 voxels
+// an edge 316 us a step, after one another 267; 20 of 32..64 234 and 250.)
 static void enqueue_batch_sweeps(bfvm_batch* b, bool with_gradient = false)
 {
 	if (b->storage != BFVM_STORAGE_F32)
@@ -1593,22 +1586,27 @@ static void enqueue_batch_sweeps(bfvm_batch* b, bool with_gradient = false)
 		batch_override o(b, 0, b->stream);
 		launch_advance_rounding(b->ctx[0]);
 	}
+	auto small = [&] {
+		on_small(b, enqueue_dirichlet);
+		for (int axis = 0; axis < 3; axis++)
+		{
+			launch_small_axis(b, axis);
+			on_small(b, [&](bfvm_ctx* c) {
+				if (axis < c->mesh.dims)
+					launch_dirichlet_interior(c);
+			});
+		}
+		if (with_gradient)
+			on_small(b, launch_gradient);
+	};
+	if (b->small.count == (int)b->ctx.size())
+	{
+		small();
+		return;
+	}
 	on_branches(
-		b,
-		[&] {
-			on_small(b, enqueue_dirichlet);
-			for (int axis = 0; axis < 3; axis++)
-			{
-				launch_small_axis(b, axis);
-				on_small(b, [&](bfvm_ctx* c) {
-					if (axis < c->mesh.dims)
-						launch_dirichlet_interior(c);
-				});
-			}
-		},
-		[&](bfvm_ctx* c, bool small) {
-			if (small)
-				return;
+		b, small, [&](size_t i) { return !b->small.member[i]; },
+		[&](bfvm_ctx* c) {
 			enqueue_dirichlet(c);
 			for (int axis = 0; axis < c->mesh.dims; axis++)
 			{
@@ -1618,16 +1616,12 @@ static void enqueue_batch_sweeps(bfvm_batch* b, bool with_gradient = false)
 			if (with_gradient)
 				launch_gradient(c);
 		});
-	if (with_gradient && b->small.count > 0)
-		on_branches(b, [] {}, [](bfvm_ctx* c, bool small) {
-			if (small)
-				launch_gradient(c);
-		});
 }
 
 static void enqueue_batch_gradient(bfvm_batch* b)
 {
-	on_branches(b, [] {}, [](bfvm_ctx* c, bool) { launch_gradient(c); });
+	on_branches(
+		b, [] {}, [](size_t) { return true; }, launch_gradient);
 }
 
 // the secretion of every instance: batched launches when the plan allows, else instance by instance
@@ -1690,13 +1684,22 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 			BFVM_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
 			BFVM_HIP(hipMalloc(&b->rounding, sizeof(unsigned)));
 			BFVM_HIP(hipMemsetAsync(b->rounding, 0, sizeof(unsigned), b->stream));
+			auto& small = b->small;
+			small.member.assign(count, 0);
+			for (int32_t i = 0; i < count; i++)
+				small.count += small.member[i] = small_filter(b->ctx[i]) ? 1 : 0;
+			if (small.count < 2)
+			{
+				small.member.assign(count, 0);
+				small.count = 0;
+			}
 			b->axes.resize(count);
 			for (int32_t i = 0; i < count; i++)
 				for (int a = 0; a < b->ctx[i]->mesh.dims; a++)
 				{
 					if (b->ctx[i]->mesh.grid[a] > 1)
 						check_batch_axis(b->ctx[i], a, i);
-					build_batch_axis(b->ctx[i], a, b->axes[i][a]);
+					build_batch_axis(b->ctx[i], a, b->axes[i][a], small.member[i] != 0);
 					batch_override o(b, i, b->stream);
 					launch_partition_coefficients(b->ctx[i], a);
 				}
@@ -1707,19 +1710,22 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 					BFVM_HIP(hipStreamCreateWithFlags(&b->branch_stream[i], hipStreamNonBlocking));
 				BFVM_HIP(hipEventCreateWithFlags(&b->branch_event[i], hipEventDisableTiming));
 			}
-			// instances in order of size, each to the branch with the least work
+			// the small instances on the first branch, the others in order of size, each to the branch with the least work
 			std::vector<int> order(count);
 			std::iota(order.begin(), order.end(), 0);
 			auto size = [&](int i) { return b->ctx[i]->mesh.V * b->ctx[i]->mesh.S; };
 			std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return size(x) > size(y); });
 			size_t load[bfvm_batch::branches] = {};
 			b->branch_of.assign(count, 0);
-			for (int i : order)
-			{
-				const int at = (int)(std::min_element(load, load + bfvm_batch::branches) - load);
-				b->branch_of[i] = at;
-				load[at] += size(i);
-			}
+			for (bool small_ones : { true, false })
+				for (int i : order)
+					if ((small.member[i] != 0) == small_ones)
+					{
+						const int at =
+							small_ones ? 0 : (int)(std::min_element(load, load + bfvm_batch::branches) - load);
+						b->branch_of[i] = at;
+						load[at] += size(i);
+					}
 			BFVM_HIP(hipStreamSynchronize(b->stream));
 		}
 		catch (...)
@@ -1864,10 +1870,10 @@ int bfvm_batch_benchmark(bfvm_batch* batch, int32_t what, int32_t iterations, fl
 			case BFVM_KERNEL_SWEEP_Z:
 				on_branches(
 					batch, [&] { launch_small_axis(batch, what - BFVM_KERNEL_SWEEP_X); },
-					[&](bfvm_ctx* c, bool small) {
-						if (!small && what - BFVM_KERNEL_SWEEP_X < c->mesh.dims)
-							launch_sweep(c, what - BFVM_KERNEL_SWEEP_X);
-					});
+					[&](size_t i) {
+						return !batch->small.member[i] && what - BFVM_KERNEL_SWEEP_X < batch->ctx[i]->mesh.dims;
+					},
+					[&](bfvm_ctx* c) { launch_sweep(c, what - BFVM_KERNEL_SWEEP_X); });
 				break;
 			case BFVM_KERNEL_GRADIENT:
 				enqueue_batch_gradient(batch);

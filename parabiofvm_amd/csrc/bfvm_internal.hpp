@@ -514,8 +514,8 @@ struct bfvm_batch
 	// per instance and axis the batch's own sweep tables, so that a context's sweep algorithm and tuning, which may change
 	// while the batch exists, leave the batch as it is
 	std::vector<std::array<bfvm::axis_tables, 3>> axes;
-	// instances whose sweeps share one launch per axis, and per axis their arguments and running task counts on the
-	// device, rebuilt with the batch's epoch
+	// instances whose sweeps share one launch per axis (fixed when the batch is made), and per axis their arguments and
+	// running task counts on the device, rebuilt with the batch's epoch
 	struct small_plan
 	{
 		std::vector<char> member; // per instance
@@ -571,9 +571,9 @@ void launch_cell_sort(bfvm_ctx* ctx); // sorted reduction: order the agents by v
 void launch_cell_release(bfvm_ctx* ctx, int index);
 void launch_voxel_positions(bfvm_ctx* ctx, int count, const float* d_pos, int* d_out);
 
-filter_plan choose_filter(const bfvm_ctx* ctx, int axis);
+filter_plan choose_filter(const bfvm_ctx* ctx, int axis, bool shared = false);
 void check_batch_axis(const bfvm_ctx* ctx, int axis, int instance);
-void build_batch_axis(bfvm_ctx* ctx, int axis, axis_tables& t);
+void build_batch_axis(bfvm_ctx* ctx, int axis, axis_tables& t, bool shared);
 size_t filter_table_floats(const filter_plan& p, int S);
 void launch_filter_coefficients(const bfvm_ctx* ctx, int axis, const filter_plan& p, float* tab, hipStream_t stream);
 void launch_filter_sweep(bfvm_ctx* ctx, int axis);

@@ -1398,9 +1398,9 @@ void alloc_partition_tables(const partition& p, int S, float*& coef, float*& red
 }
 
 // The recursive filter's plan and its table's memory; false where the axis does not take it
-static bool build_filter(const bfvm_ctx* ctx, int axis, axis_tables& t)
+static bool build_filter(const bfvm_ctx* ctx, int axis, axis_tables& t, bool shared = false)
 {
-	const filter_plan p = choose_filter(ctx, axis);
+	const filter_plan p = choose_filter(ctx, axis, shared);
 	if (p.blocks == 0)
 		return false;
 	t.filter = p;
@@ -1431,14 +1431,14 @@ void build_partition(bfvm_ctx* ctx, int axis, int chunk, int lines_request)
 }
 
 // The tables of one axis of an instance for a batch, shaped by rules on sizes and coefficients alone: the recursive
-// filter where the axis takes it, else the partitioned sweep's automatic shape, else the smallest groups of 16-element
+// filter where the axis takes it (`shared`: in launches shared with other instances), else the partitioned sweep's automatic shape, else the smallest groups of 16-element
 // blocks, which check_batch_axis has seen to fit.
-void build_batch_axis(bfvm_ctx* ctx, int axis, axis_tables& t)
+void build_batch_axis(bfvm_ctx* ctx, int axis, axis_tables& t, bool shared)
 {
 	t = axis_tables {};
 	t.n = ctx->axes[axis].n;
 	t.exact_b = ctx->axes[axis].exact_b; // the context's: an axis of one voxel divides by it
-	if (ctx->mesh.grid[axis] == 1 || build_filter(ctx, axis, t))
+	if (ctx->mesh.grid[axis] == 1 || build_filter(ctx, axis, t, shared))
 		return;
 	const int lines = axis == 2 && ctx->storage != BFVM_STORAGE_F32 ? 8 : 0;
 	try

@@ -747,8 +747,8 @@ __global__ __launch_bounds__(512) void filter_rows_kernel(filter_args a)
 
 // ---- many small meshes in one launch --------------------------------------------------------------------------------
 //
-// A mesh that does not fill the card (small_filter) is bound by its launches and their latency; the small instances of a
-// batch share one launch per axis.  A workgroup (one wave) finds its instance among the running task counts and the
+// A small mesh (small_filter) is bound by its launches and their latency; the small instances of a batch share one launch
+// per axis.  A workgroup (one wave) finds its instance among the running task counts and the
 // block length by a branch; the arguments are read from memory.
 template <int K, int... Ms>
 __device__ __forceinline__ void small_columns(const filter_args& a, int64_t task, raw16* lds)
@@ -871,8 +871,14 @@ static double row_cost(const filter_plan& p, bool full, double used)
 	return (p.m + 8.0) / p.m / used * (full ? 1.0 : 1.05) / row_waves_factor(p.waves);
 }
 
-filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
+// `shared`: for a launch shared with other instances (filter_small_kernel): one wave per workgroup that holds whole lines,
+// and the block lengths that kernel is built for.
+filter_plan choose_filter(const bfvm_ctx* ctx, int axis, bool shared)
 {
+	const int most_waves = shared ? 1 : filter_max_waves;
+	// rows of a task in LDS: one wave with 24 KB leaves a CU six waves (shared launches of 20 instances of 32..64 voxels an
+	// edge, FP32 with gradients 254 us, with 8 KB 229)
+	const int64_t most_row_bytes = shared ? 8 * 1024 : 24 * 1024;
 	const auto& g = ctx->mesh;
 	const int n = g.grid[axis], S = g.S;
 	const int64_t XS = (int64_t)g.grid[0] * S, e = (int64_t)storage_bytes(ctx->storage);
@@ -909,7 +915,7 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 		const int L = S;
 		for (int m : row_blocks)
 		{
-			if (!fits(m))
+			if (!fits(m) || (shared && (m > 17 || (n + m - 1) / m > 64)))
 				continue;
 			filter_plan p;
 			p.m = m;
@@ -921,9 +927,9 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 				p.lines_pass = 64 / p.blocks;
 				p.kw = p.blocks;
 				double best_used = 0;
-				for (int r = 1; r <= 16 && (r == 1 || r * XS * e <= 24 * 1024); r++)
+				for (int r = 1; r <= 16 && (r == 1 || r * XS * e <= most_row_bytes); r++)
 				{
-					const int groups = (r * L + p.lines_pass - 1) / p.lines_pass, waves = std::min(groups, filter_max_waves);
+					const int groups = (r * L + p.lines_pass - 1) / p.lines_pass, waves = std::min(groups, most_waves);
 					const int passes = (groups + waves - 1) / waves;
 					const double used = (double)r * L / (waves * passes * p.lines_pass) * row_waves_factor(waves);
 					if (used > best_used * 1.02)
@@ -944,7 +950,7 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 				p.rows = 1;
 				p.passes = (L + p.lines_pass - 1) / p.lines_pass;
 			}
-			if (p.waves > filter_max_waves)
+			if (p.waves > most_waves)
 				continue;
 			p.exchange_at = filter_lds_table(ctx, p.blocks, p.kw);
 			p.rows_at =
@@ -975,7 +981,7 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 		for (int clog = widest; clog >= 0 && best.blocks == 0; clog--)
 			for (int m : column_blocks)
 			{
-				if (!fits(m))
+				if (!fits(m) || (shared && m > 16))
 					continue;
 				filter_plan p;
 				p.m = m;
@@ -983,7 +989,7 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 				p.clog = clog;
 				p.kw = 64 >> clog;
 				p.waves = (p.blocks + p.kw - 1) / p.kw;
-				if (p.waves > filter_max_waves)
+				if (p.waves > most_waves)
 					continue;
 				p.exchange_at = filter_lds_table(ctx, p.blocks, p.kw);
 				p.lds = p.exchange_at + (p.waves > 1 ? 2 * ((2 * p.waves + 1) << clog) * 16 : 0);
@@ -994,7 +1000,9 @@ filter_plan choose_filter(const bfvm_ctx* ctx, int axis)
 				consider(p, (double)n / (m * p.kw * p.waves));
 			}
 	}
-	filter_plan& p = best.tasks * best.waves < filter_fill_waves ? quick : best;
+	// an instance of a shared launch does not have to fill the card by itself: 20 instances of 32..64 voxels an edge, FP16,
+	// 149 us with the short chains, 105 with the cheapest lengths
+	filter_plan& p = !shared && best.tasks * best.waves < filter_fill_waves ? quick : best;
 	p.streamed = axis != 0 && (int64_t)(ctx->mesh.V * S) * e > infinity_cache_bytes;
 	return p;
 }
@@ -1087,19 +1095,19 @@ void launch_filter_sweep(bfvm_ctx* ctx, int axis)
 	BFVM_HIP(hipGetLastError());
 }
 
-// Whether an instance of a batch takes its sweeps in the launches shared by the small ones: one-wave workgroups, too few
-// to fill the card, blocks short enough for the shared kernel's registers.
+// Whether an instance of a batch takes its sweeps in the launches shared by the small ones: every axis has a plan for
+// them, and its densities are at most 8 MB, where a launch of its own is bound by latency and the steps between
+// launches.  us per step at 4 / 8 / 16 / 32 MB, edges from 32: 20 instances up to 64, FP16 130 / 118 / 119 / 120, FP32
+// with gradients 270 / 250 / 264 / 265; 10 up to 96, FP16 161 / 138 / 154 / 158, FP32 314 / 267 / 270 / 289; 12 up to
+// 120, FP16 196 / 202 / 221 / 219, FP32 420 / 370 / 381 / 468; 19 up to 200, FP16 1080 / 1055 / 1084 / 1177.  All in
+// launches of their own: 166 and 268 for the first two, and with one-launch batches before the filter 199 and 346.
 bool small_filter(const bfvm_ctx* ctx)
 {
-	if (ctx->algorithm != BFVM_SWEEP_PARTITIONED)
+	if ((int64_t)(ctx->mesh.V * ctx->mesh.S) * (int64_t)storage_bytes(ctx->storage) > (int64_t)8 << 20)
 		return false;
 	for (int axis = 0; axis < ctx->mesh.dims; axis++)
-	{
-		const filter_plan& p = ctx->axes[axis].filter;
-		if (p.blocks == 0 || p.waves != 1 || p.kw < p.blocks || p.m > 17 || (!p.staged && p.m > 16) ||
-			p.tasks >= filter_fill_waves || ctx->sweep_workgroups[axis] > 0)
+		if (choose_filter(ctx, axis, true).blocks == 0)
 			return false;
-	}
 	return true;
 }
 

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from test_gpu_batch import check_gradients_of_stored
-from test_gpu_parity import build_pair, random_problem
+from test_gpu_parity import assert_close, build_pair, random_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -118,3 +118,36 @@ def test_sweeps_do_not_follow_the_contexts(setting, storage, pkg, oracle_mod):
             g.close()
     for k, (a, b) in enumerate(zip(*results)):
         np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32), err_msg=f"instance {k} {shapes[k]}")
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+@pytest.mark.parametrize("S", [1, 3, 4, 7, 13, 16])
+def test_shared_launches_by_length(S, storage, pkg, oracle_mod):
+    """Small instances whose sweeps share launches, lines of 2 to 257 voxels along each axis with Dirichlet faces: rows in
+    one or several passes of a wave, blocks and segments at the edges of their lengths.  The same meshes stepped one by
+    one differ by the two plans' roundings: FP32 within the parity bar, FP16 one unit of 11 bits per rounding."""
+    shapes = []
+    for n in (2, 3, 5, 17, 33, 49, 64, 65, 97, 130, 200, 257):
+        for axis in range(3):
+            shape = [6, 5, 7]
+            shape[axis] = n
+            shapes.append((tuple(shape), S))
+    alone, together = (solvers_of(pkg, oracle_mod, storage, shapes) for _ in range(2))
+    batch = pkg.Batch(together)
+    for _ in range(2):
+        batch.timestep(False, False)
+        for g in alone:
+            g.timestep(False, False)
+    batch.wait()
+    for (shape, _), g, h in zip(shapes, together, alone):
+        g.load()
+        h.load()
+        if storage == "f32":
+            assert_close(g.densities, h.densities, what=f"{shape} x {S}")
+        else:
+            # 2 steps of 4 roundings each on both sides (3 sweeps, the conversion)
+            err = np.linalg.norm(g.densities - h.densities) / np.linalg.norm(h.densities)
+            assert err <= 2 * 8 * 2.0**-10, (shape, S, err)
+    batch.close()
+    for g in alone + together:
+        g.close()
