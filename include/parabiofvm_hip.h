@@ -290,8 +290,8 @@ int bfvm_benchmark(bfvm_ctx* ctx, int32_t what, int32_t iterations, float* avg_m
 /*
  * Batches of independent microenvironments.  No counterpart in the reference, which runs one
  * microenvironment per solver (src/solver.h); a batch advances many initialized contexts of any mesh shape
- * and substrate count as one captured HIP graph (secretion of every instance -> Dirichlet -> x/y/z sweeps ->
- * gradient): the secretion by one work-list launch per phase, the sweeps of small instances in one launch per axis,
+ * and substrate count as one captured HIP graph, made at the second step after a change (secretion of every instance ->
+ * Dirichlet -> x/y/z sweeps -> gradient): the secretion by one work-list launch per phase, the sweeps of small instances in one launch per axis,
  * every other instance's sweeps and gradient as a chain on one of the graph's branches.  Per-instance results equal
  * what bfvm_timestep gives for that context to the sweep's tolerance (the same algorithm).
  *

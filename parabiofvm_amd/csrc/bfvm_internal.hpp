@@ -418,6 +418,7 @@ struct graph_slot
 	hipGraphExec_t exec = nullptr;
 	hipGraph_t graph = nullptr;
 	uint64_t epoch = 0;
+	uint64_t direct_epoch = ~0ull; // a batch's step of this kind has run without a graph in this epoch
 };
 
 } // namespace bfvm

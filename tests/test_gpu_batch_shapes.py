@@ -151,3 +151,43 @@ def test_shared_launches_by_length(S, storage, pkg, oracle_mod):
     batch.close()
     for g in alone + together:
         g.close()
+
+
+@pytest.mark.parametrize("recompute", [False, True])
+def test_direct_steps_and_replays(recompute, pkg, oracle_mod):
+    """The first step of a kind after a change is launched directly, the second makes the graph, later ones replay it:
+    agents that change before some of the steps, every instance against the oracle after each step."""
+    shapes = [((24, 20, 18), 4), ((33, 28, 21), 3), ((140, 130, 40), 4)]
+    rng = np.random.default_rng(12)
+    pairs = [build_pair(pkg, oracle_mod, random_problem(3, shape, S, seed=600 + k)) for k, (shape, S) in enumerate(shapes)]
+
+    def agents(k, A):
+        S, grid = shapes[k][1], shapes[k][0]
+        uniform = lambda *shape: rng.random(shape, dtype=np.float32)  # noqa: E731
+        size = np.array([n * v for n, v in zip(grid, pairs[k][1].voxel_shape)], dtype=np.float32)
+        a = {"positions": np.array(pairs[k][1].mins, np.float32) + uniform(A, 3) * size * np.float32(0.999),
+             "volumes": uniform(A) * 1000, "secretion_rates": uniform(A, S), "uptake_rates": uniform(A, S),
+             "saturation_densities": uniform(A, S), "net_export_rates": uniform(A, S),
+             "internalized_substrates": np.zeros((A, S), np.float32),
+             "fraction_released_at_death": np.zeros((A, S), np.float32)}
+        for be in pairs[k]:
+            be.set_agents({name: v.copy() for name, v in a.items()})
+        pairs[k][0].initialize()
+        pairs[k][1].store_agents()
+
+    for k, (o, g) in enumerate(pairs):
+        g.store()
+        agents(k, 50)
+    batch = pkg.Batch([g for _, g in pairs])
+    for step in range(7):
+        if step in (0, 1, 4):
+            agents(step % 3, 60 + 20 * step)
+        again = recompute or step in (0, 1, 4)  # new agents need their sums
+        batch.timestep(again, step % 2 == 0 or recompute)
+        for o, _ in pairs:
+            o.timestep(again, step % 2 == 0 or recompute)
+        batch.wait()
+        for k, (o, g) in enumerate(pairs):
+            g.load()
+            assert_close(g.densities, o.densities, what=f"step {step} instance {k}")
+    batch.close()

@@ -59,6 +59,41 @@ b = parabiofvm_amd.Batch(solvers)
 kernels(lambda: (b.timestep(False, False), b.wait()))
 """
 
+GROWING = """
+solvers = [solver(*x) for x in (((41, 37, 60), 7), ((64, 33, 50), 16), ((35, 64, 64), 5), ((70, 90, 80), 12))]
+uniform = lambda *shape: rng.random(shape, dtype=np.float32)  # noqa: E731
+
+
+def agents(g, A):
+    S = g.S
+    g.set_agents({"positions": uniform(A, 3) * np.float32(600), "volumes": uniform(A) * 1000,
+                  "secretion_rates": uniform(A, S), "uptake_rates": uniform(A, S), "saturation_densities": uniform(A, S),
+                  "net_export_rates": uniform(A, S), "internalized_substrates": np.zeros((A, S), np.float32)})
+
+
+for g in solvers:
+    agents(g, 100)
+    g.initialize()
+    g.store()
+    g.store_agents()
+b = parabiofvm_amd.Batch(solvers)
+calls = []
+for step in range(6):
+    if step < 4:
+        agents(solvers[1], 100 + 10 * step)
+        solvers[1].store_agents()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        b.timestep(True, True)
+        b.wait()
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events()]
+    calls.append("%d,%d" % (names.count("hipGraphInstantiate"), names.count("hipGraphLaunch")))
+    if not any("hip" in n for n in names):
+        calls = []
+        break
+print("KERNELS", *calls)
+"""
+
 
 def launched(program, argument):
     r = subprocess.run([sys.executable, "-c", HEAD + program, argument], cwd=ROOT, capture_output=True, text=True, timeout=100)
@@ -81,3 +116,9 @@ def test_small_batch_launches(storage, most):
     """Instances of at most 8 MB share one launch per axis (and the step of the rounding's counter)."""
     kernels = launched(BATCH, storage)
     assert len(kernels) <= most, kernels
+
+
+def test_growing_batch_makes_no_graphs():
+    """Agents that come between steps change the batch's launches: such steps are launched directly, and a graph is made
+    once a step repeats (made, launched)."""
+    assert launched(GROWING, "") == ["0,0"] * 4 + ["1,1", "0,1"]
