@@ -643,6 +643,7 @@ int bfvm_set_sweep_tuning(bfvm_ctx* ctx, int32_t axis, int32_t chunk, int32_t li
 		if (ctx->initialized && axis < ctx->mesh.dims)
 		{
 			BFVM_HIP(hipStreamSynchronize(ctx->stream));
+			ctx->epoch++; // also where the request is refused: the tables are new, and captured steps hold the old ones
 			try
 			{
 				build_partition(ctx, axis, chunk, lines_per_group);

@@ -93,3 +93,24 @@ def test_which_sweep_runs(a, filter_runs, pkg):
     assert any(same) != filter_runs, same
     assert_close(got, exact(x, a), rel=REL, what=f"a {a}")
     g.close()
+
+
+@pytest.mark.parametrize("a", [2.5, 250.0])
+def test_refused_tuning_leaves_the_steps(a, pkg):
+    """A launch shape that does not fit is refused, and steps captured before it run on the tables that replaced theirs."""
+    n = 300
+    x = np.random.default_rng(9).random(n, dtype=np.float32)
+    results = []
+    for refused in (False, True):
+        g = solver(pkg, n, a)
+        g.densities[:] = x
+        g.store()
+        for step in range(4):
+            if refused and step == 2:
+                with pytest.raises(Exception):
+                    g.set_sweep_tuning(0, 16, 1024)
+            g.timestep(False, False)
+        g.load()
+        results.append(g.densities.copy())
+        g.close()
+    np.testing.assert_array_equal(results[0].view(np.uint32), results[1].view(np.uint32))
