@@ -418,8 +418,13 @@ void launch_copy(bfvm_ctx* ctx)
 //  - Larger: 8 rows per thread marching over 3 planes, in plane order.  One march step loads 10 rows for 8, the first
 //    planes of a chunk are the last ones of the chunk before, still cached, and the three outputs are written in narrow
 //    windows; longer chunks spread the windows.  2 rows / 8 rows: 256^3 x 5 FP32 328 / 238, 400^3 x 8 FP32 1735 / 1387
-//    (5.9 TB/s; 8 planes 1480, order 0 1570), FP16 1843 / 1198 (6.0 TB/s), 320^3 x 8 FP16 945 / 611, 256^3 x 16 FP16
+//    (5.9 TB/s; 8 planes 1480, order 0 1570), FP16 1843 / 1198 (6.0 TB/s), 320^3 x 8 FP16 945 / 640, 256^3 x 16 FP16
 //    957 / 689.
+//    The line depends on what the caches hold: as a step leaves the densities, or read over and over, 2 rows are ahead up
+//    to the cache's size (4, 5, 8 substrates at 0.97 of it, FP32 184 238 183 / 226 255 207, FP16 371 357 351 / 441 397
+//    408; at 1.05 FP32 281 277 249 / 205 263 222); on densities that other work has displaced the march is ahead from
+//    0.8 of it (at 0.97 FP32 270 297 265 / 241 261 208, FP16 466 483 468 / 420 411 425; 320^3 x 8 FP16 741 by the
+//    march).  15/16 in FP32, whose loss is the larger on that side, is between the two.
 //  - With workgroup counts or layouts of the caller or the autotuner: 8 rows (stacked) or 4 rows, marching.
 struct gradient_shape
 {
