@@ -1687,9 +1687,17 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 			BFVM_HIP(hipMemsetAsync(b->rounding, 0, sizeof(unsigned), b->stream));
 			auto& small = b->small;
 			small.member.assign(count, 0);
+			auto size = [&](int i) { return b->ctx[i]->mesh.V * b->ctx[i]->mesh.S; };
+			size_t all = 0, small_ones = 0;
 			for (int32_t i = 0; i < count; i++)
+			{
 				small.count += small.member[i] = small_filter(b->ctx[i]) ? 1 : 0;
-			if (small.count < 2)
+				all += size(i);
+				small_ones += small.member[i] ? size(i) : 0;
+			}
+			// a few small ones in a batch of large ones hide behind the other branches (2 of 19, FP16: 1058 us a step, 1117 in
+			// shared launches)
+			if (small.count < 2 || (small.count < bfvm_batch::branches && small_ones < all / 16))
 			{
 				small.member.assign(count, 0);
 				small.count = 0;
@@ -1714,16 +1722,15 @@ int bfvm_batch_create(bfvm_ctx* const* contexts, int32_t count, bfvm_batch** out
 			// the small instances on the first branch, the others in order of size, each to the branch with the least work
 			std::vector<int> order(count);
 			std::iota(order.begin(), order.end(), 0);
-			auto size = [&](int i) { return b->ctx[i]->mesh.V * b->ctx[i]->mesh.S; };
 			std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return size(x) > size(y); });
 			size_t load[bfvm_batch::branches] = {};
 			b->branch_of.assign(count, 0);
-			for (bool small_ones : { true, false })
+			for (bool first : { true, false })
 				for (int i : order)
-					if ((small.member[i] != 0) == small_ones)
+					if ((small.member[i] != 0) == first)
 					{
 						const int at =
-							small_ones ? 0 : (int)(std::min_element(load, load + bfvm_batch::branches) - load);
+							first ? 0 : (int)(std::min_element(load, load + bfvm_batch::branches) - load);
 						b->branch_of[i] = at;
 						load[at] += size(i);
 					}
