@@ -615,13 +615,13 @@ int bfvm_set_sweep_algorithm(bfvm_ctx* ctx, int32_t algorithm, int32_t chunk)
 		ctx->algorithm = algorithm;
 		for (int a = 0; a < 3; a++)
 			ctx->chunk_request[a] = chunk;
+		ctx->epoch++;
 		if (ctx->initialized)
 		{
 			BFVM_HIP(hipStreamSynchronize(ctx->stream));
 			ensure_partitions(ctx);
 			BFVM_HIP(hipStreamSynchronize(ctx->stream));
 		}
-		ctx->epoch++;
 		return BFVM_OK;
 	});
 }

@@ -104,9 +104,8 @@ void apply_sweep_shape(bfvm_ctx* ctx, int axis, const sweep_shape& s)
 // then the workgroup count of the best of those.  The partitioned shapes are not timed against the filter: on 400^3 x
 // 8 their best ran 1.01 / 0.83 / 0.90 ms (x/y/z, FP32) and 0.89 / 0.87 / 0.86 ms (FP16) where the filter takes 0.82 /
 // 0.79 / 0.85 and 0.55 / 0.49 / 0.52 ms, and on small meshes it is 2-5 times faster.
-sweep_shape search_sweep(bfvm_ctx* ctx, int axis, int reps)
+sweep_shape search_sweep(bfvm_ctx* ctx, int axis, bool filter, int reps)
 {
-	const bool filter = ctx->axes[axis].filter.blocks > 0; // of the automatic shape, which the caller applied
 	std::vector<int> chunks = { 16, 32 };
 	if (ctx->storage == BFVM_STORAGE_F32)
 		chunks.push_back(64);
@@ -248,34 +247,64 @@ void load_tuning(const char* path)
 	}
 }
 
+// The automatic shape of an axis applied; false where it does not fit (a shape that the caller asked for may)
+static bool apply_automatic(bfvm_ctx* ctx, int axis)
+{
+	try
+	{
+		apply_sweep_shape(ctx, axis, sweep_shape {});
+		return true;
+	}
+	catch (const std::runtime_error&)
+	{
+		return false;
+	}
+}
+
+static void autotune_axis(bfvm_ctx* ctx, int axis, int reps)
+{
+	const bool automatic =
+		(ctx->chunk_request[axis] == 0 && ctx->lines_request[axis] == 0) || apply_automatic(ctx, axis);
+	const bool filter = automatic && ctx->axes[axis].filter.blocks > 0;
+	const shape_key key = key_of(ctx, axis, filter);
+	sweep_shape shape;
+	bool cached = false;
+	{
+		std::lock_guard<std::mutex> lock(g_cache_mutex);
+		auto it = g_sweep_cache.find(key);
+		if (it != g_sweep_cache.end())
+		{
+			shape = it->second;
+			cached = true;
+		}
+	}
+	if (!cached)
+		shape = search_sweep(ctx, axis, filter, reps);
+	apply_sweep_shape(ctx, axis, shape);
+	if (!cached)
+	{
+		std::lock_guard<std::mutex> lock(g_cache_mutex);
+		g_sweep_cache[key] = shape;
+	}
+}
+
 void autotune_context(bfvm_ctx* ctx, bool tune_gradient)
 {
 	const int reps = 3;
+	ctx->epoch++; // captured steps hold tables that are replaced below, also where tuning fails
 	for (int axis = 0; axis < ctx->mesh.dims; axis++)
 	{
 		if (ctx->mesh.grid[axis] == 1 || ctx->algorithm != BFVM_SWEEP_PARTITIONED)
 			continue;
-		if (ctx->chunk_request[axis] != 0 || ctx->lines_request[axis] != 0)
-			apply_sweep_shape(ctx, axis, sweep_shape {});
-		const shape_key key = key_of(ctx, axis, ctx->axes[axis].filter.blocks > 0);
-		sweep_shape shape;
-		bool cached = false;
+		const sweep_shape asked { ctx->chunk_request[axis], ctx->lines_request[axis], ctx->sweep_workgroups[axis] };
+		try
 		{
-			std::lock_guard<std::mutex> lock(g_cache_mutex);
-			auto it = g_sweep_cache.find(key);
-			if (it != g_sweep_cache.end())
-			{
-				shape = it->second;
-				cached = true;
-			}
+			autotune_axis(ctx, axis, reps);
 		}
-		if (!cached)
-			shape = search_sweep(ctx, axis, reps);
-		apply_sweep_shape(ctx, axis, shape);
-		if (!cached)
+		catch (...)
 		{
-			std::lock_guard<std::mutex> lock(g_cache_mutex);
-			g_sweep_cache[key] = shape;
+			apply_sweep_shape(ctx, axis, asked);
+			throw;
 		}
 	}
 	if (tune_gradient && ctx->mesh.dims == 3)
@@ -319,7 +348,6 @@ void autotune_context(bfvm_ctx* ctx, bool tune_gradient)
 		ctx->gradient_order = best.order;
 	}
 	BFVM_HIP(hipStreamSynchronize(ctx->stream));
-	ctx->epoch++;
 }
 
 } // namespace bfvm

@@ -1416,14 +1416,16 @@ static bool build_filter(const bfvm_ctx* ctx, int axis, axis_tables& t, bool sha
 void build_partition(bfvm_ctx* ctx, int axis, int chunk, int lines_request)
 {
 	auto& t = ctx->axes[axis];
-	free_partition_tables(t);
 	// the staged sweep runs one line per thread on 16-element blocks
 	const bool staged = ctx->algorithm == BFVM_SWEEP_STAGED;
 	const bool automatic = ctx->algorithm == BFVM_SWEEP_PARTITIONED && chunk == 0 && lines_request == 0;
 	// 16-bit forms take z lines in groups of 8, not 16 (measured on 400^3 x 8 BF16: 1.38 -> 1.11 ms)
 	if (lines_request == 0 && axis == 2 && ctx->storage != BFVM_STORAGE_F32 && !staged)
 		lines_request = 8;
-	t.part = choose_partition(ctx, axis, staged ? batch_chunk : chunk, lines_request, staged ? 1 : 4);
+	// a shape that does not fit leaves the axis its tables
+	const partition p = choose_partition(ctx, axis, staged ? batch_chunk : chunk, lines_request, staged ? 1 : 4);
+	free_partition_tables(t);
+	t.part = p;
 	if (automatic && t.part.P > 0 && build_filter(ctx, axis, t))
 		return;
 	if (t.part.P > 0)
@@ -1431,8 +1433,8 @@ void build_partition(bfvm_ctx* ctx, int axis, int chunk, int lines_request)
 }
 
 // The tables of one axis of an instance for a batch, shaped by rules on sizes and coefficients alone: the recursive
-// filter where the axis takes it (`shared`: in launches shared with other instances), else the partitioned sweep's automatic shape, else the smallest groups of 16-element
-// blocks, which check_batch_axis has seen to fit.
+// filter where the axis takes it (`shared`: in launches shared with other instances), else the partitioned sweep's
+// automatic shape, else the smallest groups of 16-element blocks, which check_batch_axis has seen to fit.
 void build_batch_axis(bfvm_ctx* ctx, int axis, axis_tables& t, bool shared)
 {
 	t = axis_tables {};

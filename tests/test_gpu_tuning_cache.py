@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from test_gpu_parity import random_problem
+from test_gpu_parity import assert_close, random_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -66,4 +66,25 @@ def test_entries_of_older_files_leave_the_automatic_kernels(pkg, tmp_path):
     assert f"sweep 0 {entry} 16 2 1024" in lines and f"gradient {entry} 2048 1 0" in lines
     assert any(x.startswith(f"gradient_field {entry} ") for x in lines)
     assert any(x.startswith(f"sweep 0 {entry} 0 0 ") for x in lines)
+    g.close()
+
+
+def test_autotune_where_only_a_requested_shape_fits(pkg, oracle_mod):
+    """Lines of 1200 voxels x 18 substrates fit with 4 lines or fewer to a workgroup, which the automatic shape does not
+    take: a context that asked for such a shape is tuned over the shapes that fit, and steps on."""
+    p = random_problem(3, (4, 1200, 3), 18, seed=6, faces=False, interior=False)
+    args = (p["dims"], p["mins"], p["maxs"], p["vs"], p["S"], p["dt"], p["D"], p["decay"], p["init"])
+    o, g = oracle_mod.Oracle(*args, dtype=np.float64), pkg.DeviceSolver(*args)
+    g.set_sweep_tuning(1, 32, 2)
+    for be in (o, g):
+        be.densities[:] = p["dens"]
+        be.initialize()
+    g.store()
+    g.timestep(False, False)
+    g.autotune()
+    g.timestep(False, False)
+    g.load()
+    for _ in range(2):
+        o.diffusion()
+    assert_close(g.densities, o.densities, what=f"{[g.partition(axis) for axis in range(3)]}")
     g.close()
