@@ -5,24 +5,25 @@
 // is B - a, are the interior row with a ghost x_{-1} = x_0 (x_n = x_{n-1}): zero flux, i.e. the line mirrored about
 // its ends.  On the mirrored infinite line the matrix factors exactly into two first-order recursions with one
 // constant, mu = 2a / (B + sqrt(B^2 - 4a^2)) (the smaller root of a mu^2 - B mu + a = 0, 0 <= mu < 1):
-//   u_j = d_j + mu u_{j-1},   x_j = s (u_j + mu x'_{j+1}),   s = (1 - mu)^2 / (1 + decay*dt/dims)
-// (x' without the factor s).  The same solution as the Thomas algorithm's (host/diffusion_solver.cpp:72-142,
-// 297-480), with constants instead of a table entry per element: 5 operations per element and no table reads.
+//   u_j = s d_j + mu u_{j-1},   x_j = u_j + mu x_{j+1},   s = (1 - mu)^2 / (1 + decay*dt/dims)
+// (s applied to d: nothing on the way exceeds the densities, where it applied to x would have a factor of up to 14).  The
+// same solution as the Thomas algorithm's (host/diffusion_solver.cpp:72-142, 297-480), with constants instead of a table
+// entry per element: 5 operations per element and no table reads.
 // Every term is positive for positive densities, so rounding errors do not amplify, and s is chosen from the rounded mu so
 // that a constant field keeps its exact gain.  What the rounding of mu does cost is the distance over which a local
 // source decays: a relative error of up to 2^-25 / (mu |ln mu|) of it, which grows with a (filter_coefficients_ok).
 //
-// A line is split into blocks of m elements held in the registers of one lane each.  Per block: f = sum mu^{m-1-j}
-// d_j and e = sum mu^j d_j (the block's contribution to everything right and left of it), one two-sided scan of
+// A line is split into blocks of m elements held in the registers of one lane each.  Per block: f = sum mu^{m-1-j} s d_j
+// and e = sum mu^j s d_j (the block's contribution to everything right and left of it), one two-sided scan of
 // (f, e) over the line's blocks (factor W = mu^m per block; lane shuffles within a wave, one LDS exchange where a
 // line takes several waves), the mirror images at both ends in closed form, then the two recursions started with
 // the exact values of the neighbouring blocks.  Small workgroups (the waves of one line group, 1 to 8) with at most
 // one barrier: the groups of a CU drift apart and keep loads, arithmetic and stores in flight at the same time.
 //   scan:  U_k = sum_{k'<k} W^{k-1-k'} f_{k'},  T_k = sum_{k'>=k} W^{k'-k} e_{k'}
-//   line:  E = T_0, F = f_last + mu^{mlast} U_last (sums of d_j weighted by the distance to the first / last element)
+//   line:  E = T_0, F = f_last + mu^{mlast} U_last (sums of s d_j weighted by the distance to the first / last element)
 //   ends:  u_{-1} = (E + mu^n F) / (1 - mu^{2n}),  z_n = (F + mu^n E) / (1 - mu^{2n})
 //   block: u_{start-1} = U_k + mu^{m k} u_{-1},  Z = T_{k+1} + mu^{n - min(n, m(k+1))} z_n,
-//          x'_{end+1} = (mu u_end + Z) / (1 - mu^2)
+//          x_{end+1} = (mu u_end + Z) / (1 - mu^2)
 #include <algorithm>
 #include <cmath>
 
@@ -37,7 +38,7 @@ namespace bfvm {
 enum filter_row
 {
 	fr_mu,
-	fr_s,	   // output factor
+	fr_s,	   // factor of the densities
 	fr_inv1,   // 1 / (1 - mu^2)
 	fr_mun,	   // mu^n
 	fr_w,	   // W = mu^m
@@ -249,7 +250,6 @@ __device__ __forceinline__ void filter_line(typename vec_of<V>::type (&v)[M], Ro
 		v[j] = u;
 	}
 	vec x = (mu * u + z) * row(fr_inv1);
-	const vec s = row(fr_s);
 	if (at.active)
 	{
 #pragma unroll
@@ -257,7 +257,7 @@ __device__ __forceinline__ void filter_line(typename vec_of<V>::type (&v)[M], Ro
 		{
 			x = has(j) ? v[j] + mu * x : x;
 			if (has(j))
-				store(j, s * x);
+				store(j, x);
 		}
 	}
 }
@@ -443,10 +443,11 @@ __device__ __forceinline__ void filter_columns_task(const filter_args& a, int64_
 		return vec { x[s[0]], x[s[1]], x[s[2]], x[s[3]] };
 	};
 	vec v[M];
+	const vec gain = row(fr_s);
 #pragma unroll
 	for (int j = 0; j < M; j++)
 	{
-		v[j] = __builtin_convertvector(raw[j], vec);
+		v[j] = __builtin_convertvector(raw[j], vec) * gain;
 		if (j >= N)
 			v[j] = j < mk ? v[j] : vec(0.f);
 	}
@@ -649,18 +650,19 @@ __device__ __forceinline__ void filter_rows_task(const filter_args& a, int64_t t
 		at.active = b < a.kw && at.k <= at.last && r < nrows;
 		const int pos = r * XS + at.k * M * S + line;
 		float v[M];
+		auto row = [&](int rw) { return lt[rw * S + line]; };
+		const float gain = row(fr_s);
 		const elem* lv = l + (at.active ? pos : 0); // inactive lanes read what is there
 #pragma unroll
 		for (int j = 0; j < M; j++)
 		{
-			v[j] = (float)lv[j < N || j < mk ? j * S : 0];
+			v[j] = (float)lv[j < N || j < mk ? j * S : 0] * gain;
 			if (j >= N)
 				v[j] = j < mk ? v[j] : 0.f;
 		}
 		uint32_t h = K == store_f32 ? 0u : sr_seed(row0 * XS + pos, rounding_key(a.rounding, 1));
 		const int So = fresh_uniform(S); // the stores' addresses are not the loads' held
 		elem* lo = l + pos;
-		auto row = [&](int rw) { return lt[rw * S + line]; };
 		filter_line<M, FULL, 1>(v, row, mk, a.blocks, at, (float*)(lds + a.exchange_at), [&](int j, float x) {
 			elem* o = lo + j * So;
 			if constexpr (K == store_f32)
@@ -819,8 +821,8 @@ static void by_block(int m, bool full, F&& f)
 // The filter needs 0 <= mu < 1, i.e. a >= 0 and 1 + decay*dt/dims > 0, and it is used up to mu = 0.73 (a = 10), where its
 // FP32 error against FP64 solves is still no larger than the partitioned sweep's.  Worst of 144 lines of 100, 400 and
 // 1000 voxels each (filter / partitioned), point source, relative L2 and per voxel above 1e-3 of the largest:
-//   a = 1..2.5    1.1e-7 / 1.3e-7  5.4e-7 / 7.0e-7        a = 16..25     1.8e-7 / 2.6e-7  1.3e-6 / 7.8e-7
-//   a = 6..10     1.4e-7 / 2.5e-7  9.2e-7 / 9.7e-7        a = 100..300   4.0e-7 / 3.7e-7  3.3e-6 / 7.1e-7
+//   a = 1..2.5    1.1e-7 / 1.3e-7  6.7e-7 / 7.0e-7        a = 16..25     1.8e-7 / 2.6e-7  1.3e-6 / 7.8e-7
+//   a = 6..10     1.7e-7 / 2.5e-7  8.6e-7 / 9.7e-7        a = 100..300   4.0e-7 / 3.7e-7  3.3e-6 / 7.1e-7
 //   a = 10..16    1.7e-7 / 2.5e-7  1.1e-6 / 8.8e-7        a = 1e3..1e5   3.2e-6 / 4.6e-7  1.7e-5 / 8.1e-7
 // (uniform random densities hide it: 2.0e-7 / 3.2e-7 at a = 1e3..1e5).
 static constexpr double filter_largest_mu = 0.73;

@@ -114,3 +114,14 @@ def test_refused_tuning_leaves_the_steps(a, pkg):
         results.append(g.densities.copy())
         g.close()
     np.testing.assert_array_equal(results[0].view(np.uint32), results[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("a", [2.5, 9.9])
+def test_values_near_the_largest(a, pkg):
+    """Densities of up to 3e38: a diffused value lies within the range of the densities, and so does everything on the way
+    to it."""
+    n = 400
+    x = (np.random.default_rng(10).random(n) * 2e38 + 1e38).astype(np.float32)
+    g = solver(pkg, n, a)
+    assert_close(diffused(g, x), exact(x, a), rel=REL, what=f"a {a}")
+    g.close()
